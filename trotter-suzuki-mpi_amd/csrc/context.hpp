@@ -80,4 +80,16 @@ namespace tsmi {
 // context precision), asynchronous on c's stream.
 int ctx_exchange(tsmi_ctx *c, void *re, void *im);
 
+// One event of the pair around a step-kernel launch when timing is on (kind 1:
+// several steps per launch; which 0: before, 1: after).
+int ctx_time_mark(tsmi_ctx *c, int kind, int which);
+
+// Tile passes (tsmi_tile.hip), asynchronous on c's stream: whether c's real-time
+// steps run as them; whether c is a doubly periodic lattice whose passes may wrap
+// (several steps per launch); n steps as one or several passes, on the tile
+// closed at its edges or (wrap) on the periodic lattice, the halo refreshed.
+bool tile_runs(const tsmi_ctx *c);
+bool tile_wraps(const tsmi_ctx *c);
+int tile_passes(tsmi_ctx *c, int n, bool wrap);
+
 }  // namespace tsmi

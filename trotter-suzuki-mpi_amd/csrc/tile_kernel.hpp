@@ -1,0 +1,288 @@
+// tile_kernel.hpp -- several real-time steps of a small or medium lattice per
+// launch, the tile held in registers.
+//
+// What bounds a small lattice is not memory but each wave's chain of dependent
+// row updates: step_kernel and step2_kernel stream rows through a pipeline, one
+// row per beat, and a 256^2 lattice gives them a few dozen waves, each alone on
+// its SIMD, whose beats wait for one another (FP64 54 us per two-step launch).
+// Here a workgroup of NW waves holds a tile of 128 columns x (NW R) rows, R rows
+// x 2 columns per lane in registers, and runs k whole steps on it: every pass is
+// R independent row updates per wave, so a wave alone on its SIMD issues back to
+// back, the rows are loaded at once, and one launch serves k steps.  The tile
+// carries an apron of 4k cells on each side (the dependency cone of k steps).
+//
+// Vertical pairs inside a wave's rows are register operations.  A vertical pass
+// pairs rows (y, y+1) where x + y + s is even, so at the border between two
+// waves one of a lane's two columns pairs across it: the waves exchange that
+// column of their first and last rows through LDS (double-buffered, one barrier
+// per vertical pass; the border rows are computed first, so that the other rows'
+// work lies between the write and the barrier).  The last V0 of a step and the
+// first of the next are one pass of twice the angle (coefficients m2, t2 of
+// that angle), which saves one of the four exchanges.
+//
+// Measured against the streaming passes, us per step: 64^2 periodic FP64 17.3 ->
+// 2.8, 256^2 FP64 23.1 -> 4.4, 1024^2 FP32 17.0 -> 6.6, FP64 23.6 -> 10.5.  Now
+// bound by instruction issue (and by the launch, some 4 us of a pass).
+//
+// Two uses, by p.nx: 0: the tile W x H is closed at its edges (closed axes, or
+// one step on the reference tile of a periodic lattice, its halo as it is).
+// Otherwise W and H are the tile of a doubly periodic lattice of nx x ny inner
+// cells, both even (the pair pattern then is periodic too): rows and columns are
+// read from the inner cells they mirror, every cell of the tile is written, and
+// the halo is left as the exchange would leave it.
+#pragma once
+#include "step_kernel.hpp"
+
+namespace tsmi {
+
+constexpr int kTileWavesMax = 8;     // waves per workgroup, at most
+constexpr int kTileCols = 2 * kWave; // columns of a tile
+
+template <typename T>
+struct TileParams {
+    const T *in_re, *in_im;
+    T *out_re, *out_im;
+    const T *ph;                     // phase plane (StepParams::ph)
+    int W, H, pitch;
+    int nx, ny;                      // inner extents of a doubly periodic lattice, or 0
+    int steps;                       // k
+    int n_strips, cols, rows;        // output columns and rows per tile
+    T mH, tH, mV, tV, unH, unV;      // scaled-frame pair factors (StepParams)
+    T m2, t2, un2;                   // the merged V0 V0 pass
+    int mode2;                       // its scaled form
+    T c_nl, c_lhy;
+    double mag, mag_mid;             // |corr| of the last step and of the steps before it
+    T dphi;                          // phase of the merged frame, added to every phase
+};
+
+template <typename T>
+struct TileXch {
+    typedef T __attribute__((ext_vector_type(2))) T2;
+    // [buffer][first / last row of a wave][wave + 1][lane]; the slots of waves -1
+    // and NW hold zeros (no row there)
+    T2 v[2][2][kTileWavesMax + 2][kWave];
+};
+
+// The potential pass of two rows: one wave-uniform test and straight-line code
+// for the four values per lane.
+template <typename T, bool LHY>
+__device__ __forceinline__ void tile_ppass(Row<T, 2> &a, Row<T, 2> &b, const T (&pa)[2], const T (&pb)[2], T c, T cl,
+                                           double mag) {
+    T ang[4], sn[4], cs[4];
+    auto angle = [&](const Row<T, 2> &r, int k, T ph) {
+        const T n2 = r.re[k] * r.re[k] + r.im[k] * r.im[k];
+        return (LHY ? c * n2 + cl * (n2 * sqrt_t(n2)) : c * n2) + ph;
+    };
+    ang[0] = angle(a, 0, pa[0]);
+    ang[1] = angle(a, 1, pa[1]);
+    ang[2] = angle(b, 0, pb[0]);
+    ang[3] = angle(b, 1, pb[1]);
+    sincos_row<T, 4>(ang, sn, cs);
+    const T ca[2] = {cs[0], cs[1]}, sa[2] = {sn[0], sn[1]}, cb[2] = {cs[2], cs[3]}, sb[2] = {sn[2], sn[3]};
+    rotate_row_ph<T, 2>(a, ca, sa, mag);
+    rotate_row_ph<T, 2>(b, cb, sb, mag);
+}
+
+// EH: the strip reaches past the tile's left or right edge (per-lane pair
+// coefficients); EV: so do the wave's rows at the top or bottom (bit r + 1 of ok:
+// rows r and r + 1 of the wave are both inside the tile).
+template <typename T, bool LHY, int MODE, int R, bool EH, bool EV>
+__device__ __forceinline__ void tile_steps(const TileParams<T> &p, Row<T, 2> (&s)[R], const T (&ph)[R][2],
+                                           TileXch<T> &x, int w, int lane, int xl,
+                                           unsigned ok) {
+    static_assert(R % 2 == 0 && R >= 4, "row parities are fixed per register");
+    typedef typename TileXch<T>::T2 T2;
+    constexpr int M = MODE < 0 ? 0 : MODE;
+    const T kH = M == 0 ? p.tH : p.mH;
+    HCoef<T, 2> hc = {};
+    // a periodic lattice has no edge: every column far from one
+    if constexpr (EH)
+        hc = make_hcoef<T, 2>(p.nx ? 2 * lane + 2 : xl, lane, p.nx ? 1 << 30 : p.W, p.mH, p.tH, p.unH);
+    int buf = 0;
+
+    auto hrow = [&](auto ss, Row<T, 2> &r, auto rr) {
+        constexpr int PAR = (decltype(ss)::value + decltype(rr)::value) & 1;
+        if constexpr (EH) hpass<PAR, false>(r, hc);
+        else hpass_fast<PAR, false, M>(r, kH);
+    };
+    // the vertical pass V(S), factors (m, t) in the scaled form FM (-1: both
+    // factors) and un for unpaired cells; `first` has run on the border rows and
+    // `rest` runs on the others between the exchange's write and its barrier
+    auto vpass = [&](auto ss, auto fm, T m, T t, T un, auto &&rest) {
+        constexpr int S = decltype(ss)::value, FM = decltype(fm)::value;
+        constexpr int CX = 1 - S;                    // the column that pairs across the border
+        T2 top, bot;
+        top[0] = s[0].re[CX];
+        top[1] = s[0].im[CX];
+        bot[0] = s[R - 1].re[CX];
+        bot[1] = s[R - 1].im[CX];
+        x.v[buf][0][w + 1][lane] = top;
+        x.v[buf][1][w + 1][lane] = bot;
+        rest();
+        __syncthreads();
+        const T2 up = x.v[buf][1][w][lane], dn = x.v[buf][0][w + 2][lane];
+        buf ^= 1;
+        // cells without a partner only exist at the tile's edges (EV): the test of
+        // their bit is uniform
+        auto pair = [&](int c, int r) {
+            if (EV && __builtin_expect(!(ok >> (r + 1) & 1u), 0)) {
+                s[r].re[c] *= un;
+                s[r].im[c] *= un;
+                s[r + 1].re[c] *= un;
+                s[r + 1].im[c] *= un;
+            } else if constexpr (FM < 0) {
+                rot<false>(m, t, s[r].re[c], s[r].im[c], s[r + 1].re[c], s[r + 1].im[c]);
+            } else {
+                fpair<false, FM>(FM == 0 ? t : m, s[r].re[c], s[r].im[c], s[r + 1].re[c], s[r + 1].im[c]);
+            }
+        };
+#pragma unroll
+        for (int r = 0; r + 1 < R; r += 2) pair(S, r);
+#pragma unroll
+        for (int r = 1; r + 1 < R; r += 2) pair(CX, r);
+        Row<T, 2> &f = s[0], &l = s[R - 1];
+        if (EV && __builtin_expect(!(ok & 1u), 0)) {
+            f.re[CX] *= un;
+            f.im[CX] *= un;
+        } else if constexpr (FM < 0) {
+            rot_q<false>(m, t, up[0], up[1], f.re[CX], f.im[CX]);
+        } else {
+            fpair_q<false, FM>(FM == 0 ? t : m, up[0], up[1], f.re[CX], f.im[CX]);
+        }
+        if (EV && __builtin_expect(!(ok >> R & 1u), 0)) {
+            l.re[CX] *= un;
+            l.im[CX] *= un;
+        } else if constexpr (FM < 0) {
+            rot_p<false>(m, t, l.re[CX], l.im[CX], dn[0], dn[1]);
+        } else {
+            fpair_p<false, FM>(FM == 0 ? t : m, l.re[CX], l.im[CX], dn[0], dn[1]);
+        }
+    };
+    using I0 = std::integral_constant<int, 0>;
+    using I1 = std::integral_constant<int, 1>;
+    using IM = std::integral_constant<int, MODE>;
+    auto h_border = [&](auto ss) {
+        hrow(ss, s[0], I0());
+        hrow(ss, s[R - 1], I1());                    // R - 1 is odd
+    };
+    auto h_rest = [&](auto ss) {
+#pragma unroll
+        for (int r = 1; r + 1 < R; r += 2) {
+            hrow(ss, s[r], I1());
+            hrow(ss, s[r + 1], I0());
+        }
+    };
+
+    vpass(I0(), IM(), p.mV, p.tV, p.unV, [] {});
+    for (int st = 0;; ++st) {
+        const bool last = st == p.steps - 1;
+        const double mag = last ? p.mag : p.mag_mid;
+        h_border(I0());
+        vpass(I1(), IM(), p.mV, p.tV, p.unV, [&] { h_rest(I0()); });
+        h_border(I1());
+        h_rest(I1());
+        // the potential pass, border rows first
+        tile_ppass<T, LHY>(s[0], s[R - 1], ph[0], ph[R - 1], p.c_nl, p.c_lhy, mag);
+        h_border(I1());
+        vpass(I1(), IM(), p.mV, p.tV, p.unV, [&] {
+#pragma unroll
+            for (int r = 1; r + 1 < R; r += 2)
+                tile_ppass<T, LHY>(s[r], s[r + 1], ph[r], ph[r + 1], p.c_nl, p.c_lhy, mag);
+            h_rest(I1());
+        });
+        h_border(I0());
+        if (last) break;
+        if (p.mode2 == 0)
+            vpass(I0(), I0(), p.m2, p.t2, p.un2, [&] { h_rest(I0()); });
+        else
+            vpass(I0(), I1(), p.m2, p.t2, p.un2, [&] { h_rest(I0()); });
+    }
+    vpass(I0(), IM(), p.mV, p.tV, p.unV, [&] { h_rest(I0()); });
+}
+
+template <typename T, bool LHY, int MODE, int R>
+__global__ void __launch_bounds__(kTileWavesMax * kWave) tile_kernel(TileParams<T> p) {
+    __shared__ TileXch<T> xch;
+    const int lane = threadIdx.x & (kWave - 1);
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    const int nw = blockDim.x / kWave;
+    const int strip = blockIdx.x % p.n_strips, seg = blockIdx.x / p.n_strips;
+    const int A = kApron * p.steps;
+    const bool wrap = p.nx != 0;
+    const int X0 = strip * p.cols - A;                            // even
+    const int xl = X0 + 2 * lane;
+    // a closed tile's first rows need no apron above them
+    const int y_tile = wrap ? seg * p.rows - A : max(0, seg * p.rows - A);
+    const int y0 = y_tile + w * R;                                // even: first row of this wave
+
+    // slots of the rows above the first and below the last wave
+    if (w == 0) {
+        typename TileXch<T>::T2 z = {T(0), T(0)};
+        xch.v[0][1][0][lane] = xch.v[1][1][0][lane] = z;
+        xch.v[0][0][nw + 1][lane] = xch.v[1][0][nw + 1][lane] = z;
+    }
+
+    const unsigned bytes = (unsigned)p.pitch * (unsigned)p.H * (unsigned)sizeof(T);
+    const __amdgpu_buffer_rsrc_t r_in_re = make_rsrc(p.in_re, bytes), r_in_im = make_rsrc(p.in_im, bytes);
+    const __amdgpu_buffer_rsrc_t r_ph = make_rsrc(p.ph, bytes);
+    const __amdgpu_buffer_rsrc_t r_out_re = make_rsrc(p.out_re, bytes), r_out_im = make_rsrc(p.out_im, bytes);
+    const unsigned row_bytes = (unsigned)p.pitch * (unsigned)sizeof(T);
+    auto mod = [](int a, int n) {
+        const int r = a % n;
+        return r < 0 ? r + n : r;
+    };
+    int xs = xl;
+    bool ld_ok = xl >= 0 && xl + 2 <= p.pitch;
+    if (wrap) {
+        xs = kApron + mod(xl - kApron, p.nx);                     // even, nx even: the pair stays together
+        ld_ok = true;
+    }
+    const unsigned v_ld = ld_ok ? (unsigned)xs * (unsigned)sizeof(T) : kOffNone;
+
+    Row<T, 2> s[R];
+    T ph[R][2];
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        const int y = y0 + r;
+        const bool in = wrap || (y >= 0 && y < p.H);
+        const int ys = wrap ? kApron + mod(y - kApron, p.ny) : y;
+        const unsigned off = in ? v_ld + (unsigned)ys * row_bytes : kOffNone;
+        buf_load<T, 2>(r_in_re, off, 0u, s[r].re);
+        buf_load<T, 2>(r_in_im, off, 0u, s[r].im);
+        buf_load<T, 2>(r_ph, off, 0u, ph[r]);
+    }
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        ph[r][0] += p.dphi;
+        ph[r][1] += p.dphi;
+    }
+    __syncthreads();
+
+    const bool eh = MODE < 0 || (!wrap && (X0 < 0 || X0 + kTileCols > p.W));
+    const bool ev = MODE < 0 || (!wrap && (y0 <= 0 || y0 + R >= p.H));
+    unsigned ok = 0;
+#pragma unroll
+    for (int r = -1; r < R; ++r)
+        if (wrap || (y0 + r >= 0 && y0 + r + 1 < p.H)) ok |= 1u << (r + 1);
+    if constexpr (MODE < 0) {
+        tile_steps<T, LHY, MODE, R, true, true>(p, s, ph, xch, w, lane, xl, ok);
+    } else {
+        if (ev) tile_steps<T, LHY, MODE, R, true, true>(p, s, ph, xch, w, lane, xl, ok);
+        else if (eh) tile_steps<T, LHY, MODE, R, true, false>(p, s, ph, xch, w, lane, xl, ok);
+        else tile_steps<T, LHY, MODE, R, false, false>(p, s, ph, xch, w, lane, xl, ok);
+    }
+
+    // columns in [W, pitch) are padding and are written back as the zeros they hold
+    const bool own = lane >= A / 2 && lane < A / 2 + p.cols / 2 && xl < p.W;
+    const int y_lo = seg * p.rows, y_hi = min(p.H, y_lo + p.rows);
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        const int y = y0 + r;
+        const unsigned off =
+            own && y >= y_lo && y < y_hi ? (unsigned)xl * (unsigned)sizeof(T) + (unsigned)y * row_bytes : kOffNone;
+        buf_store<T, 2>(r_out_re, off, 0u, s[r].re);
+        buf_store<T, 2>(r_out_im, off, 0u, s[r].im);
+    }
+}
+
+}  // namespace tsmi

@@ -109,6 +109,24 @@ namespace {
         if (e_ != hipSuccess) return fail(TSMI_E_HIP, std::string(#call) + ": " + hipGetErrorString(e_)); \
     } while (0)
 
+}  // namespace
+
+int tsmi::ctx_time_mark(tsmi_ctx *c, int kind, int which) {
+    if (!c->timing) return TSMI_OK;
+    std::vector<hipEvent_t> &v = c->ev[kind][which];
+    const size_t i = c->ev_used[kind];
+    if (i >= v.size()) {
+        hipEvent_t e = nullptr;
+        TSMI_HIP(hipEventCreate(&e));
+        v.push_back(e);
+    }
+    TSMI_HIP(hipEventRecord(v[i], c->stream));
+    if (which == 1) ++c->ev_used[kind];
+    return TSMI_OK;
+}
+
+namespace {
+
 constexpr int kBlock = 256;          // 4 wavefronts per workgroup
 
 // FP32 columns per lane of the single-step and of the fused two-step kernel
@@ -313,21 +331,6 @@ int import_device(tsmi_ctx *c, void *dst, const double *src) {
     return TSMI_OK;
 }
 
-// Event pair around a step-kernel launch when timing is on (kind 1: fused).
-int time_mark(tsmi_ctx *c, int kind, int which) {
-    if (!c->timing) return TSMI_OK;
-    std::vector<hipEvent_t> &v = c->ev[kind][which];
-    const size_t i = c->ev_used[kind];
-    if (i >= v.size()) {
-        hipEvent_t e = nullptr;
-        TSMI_HIP(hipEventCreate(&e));
-        v.push_back(e);
-    }
-    TSMI_HIP(hipEventRecord(v[i], c->stream));
-    if (which == 1) ++c->ev_used[kind];
-    return TSMI_OK;
-}
-
 // The periodic halo refresh of a state (or E) allocation: the reference's
 // 4-wide exchange on the reference tile, or on the 8-wide layout the full wrap
 // of all 8 halo cells, whose inner 4 are exactly what the 4-wide exchange writes.
@@ -425,14 +428,14 @@ int launch_step2(tsmi_ctx *c) {
     p.unH = (T)c->unH; p.unV = (T)c->unV;
     p.c_nl = (T)c->c_nl_s; p.c_lhy = (T)c->c_lhy_s;
     const int blocks = (c->n_waves2 + kBlock / kWave - 1) / (kBlock / kWave);
-    if (int st = time_mark(c, 1, 0)) return st;
+    if (int st = ctx_time_mark(c, 1, 0)) return st;
     if (sizeof(T) == 8 && c->nt_out)
         hipLaunchKernelGGL((step2_kernel<T, VEC, LHY, MODE, PH, sizeof(T) == 8>), dim3(blocks), dim3(kBlock), 0,
                            c->stream, p);
     else
         hipLaunchKernelGGL((step2_kernel<T, VEC, LHY, MODE, PH>), dim3(blocks), dim3(kBlock), 0, c->stream, p);
     TSMI_HIP(hipGetLastError());
-    if (int st = time_mark(c, 1, 1)) return st;
+    if (int st = ctx_time_mark(c, 1, 1)) return st;
     c->cur = nb;
     return TSMI_OK;
 }
@@ -485,14 +488,14 @@ int launch_step(tsmi_ctx *c, int exchange) {
     }
     // the grid covers every (strip, segment) pair exactly once
     const int blocks = (c->n_waves + kBlock / kWave - 1) / (kBlock / kWave);
-    if (int st = time_mark(c, 0, 0)) return st;
+    if (int st = ctx_time_mark(c, 0, 0)) return st;
     if (!IMAG && sizeof(T) == 8 && c->nt_out)
         hipLaunchKernelGGL((step_kernel<T, IMAG, VEC, LHY, MODE, PH, !IMAG && sizeof(T) == 8>), dim3(blocks),
                            dim3(kBlock), 0, c->stream, p);
     else
         hipLaunchKernelGGL((step_kernel<T, IMAG, VEC, LHY, MODE, PH>), dim3(blocks), dim3(kBlock), 0, c->stream, p);
     TSMI_HIP(hipGetLastError());
-    if (int st = time_mark(c, 0, 1)) return st;
+    if (int st = ctx_time_mark(c, 0, 1)) return st;
     c->cur = nb;
     if (exchange) {
         const int st = exchange_halo<T>(c, c->psi_base[nb][0], c->psi_base[nb][1]);
@@ -568,12 +571,20 @@ int step_typed(tsmi_ctx *c, int exchange) {
     return lhy ? step_mode<T, false, VEC, true>(c, exchange) : step_mode<T, false, VEC, false>(c, exchange);
 }
 
-int step_once(tsmi_ctx *c, int exchange) {
+int step_rows(tsmi_ctx *c, int exchange) {
     return c->esz == 4 ? step_typed<float, kVec32, kVec32I>(c, exchange) : step_typed<double, 2, 2>(c, exchange);
 }
 
 int exchange_planes(tsmi_ctx *c, void *re, void *im) {
     return c->esz == 4 ? exchange_halo<float>(c, re, im) : exchange_halo<double>(c, re, im);
+}
+
+int exchange_current(tsmi_ctx *c) { return exchange_planes(c, c->psi_base[c->cur][0], c->psi_base[c->cur][1]); }
+
+int step_once(tsmi_ctx *c, int exchange) {
+    if (!tile_runs(c)) return step_rows(c, exchange);
+    const int st = tile_passes(c, 1, false);
+    return st || !exchange ? st : exchange_current(c);
 }
 
 // Solver::evolve(n) for one component (src/solver.cpp:186-230): n steps, the
@@ -587,6 +598,18 @@ int exchange_planes(tsmi_ctx *c, void *re, void *im) {
 int evolve_steps(tsmi_ctx *c, int n, bool exchange_last = false) {
     int st = TSMI_OK;
     const int last_ex = exchange_last ? 1 : 0;
+    if (tile_runs(c)) {
+        if (!c->d.periodic_x && !c->d.periodic_y) return tile_passes(c, n, false);
+        if (tile_wraps(c) && n >= 3) {
+            st = tile_passes(c, 1, false);
+            if (!st) st = tile_passes(c, n - 2, true);
+            return st ? st : step_once(c, last_ex);
+        }
+        // mixed axes; odd periodic extents, where the pair pattern of a halo cell
+        // differs from that of the cell it mirrors
+        for (int i = 0; i < n && !st; ++i) st = step_once(c, i != n - 1 ? 1 : last_ex);
+        return st;
+    }
     if (c->sweeps != 2 || n < 2 || (c->halo8 && n < 3)) {
         for (int i = 0; i < n && !st; ++i) st = step_once(c, i != n - 1 ? 1 : last_ex);
         return st;
@@ -1166,12 +1189,19 @@ int tsmi_evolve_checkpointed(tsmi_ctx *c, int32_t n, int32_t every) {
     // closed axes, FP32: two steps per pass wherever no checkpoint falls between
     // them (FP64 measured faster at one step per pass on a 1024^2 lattice: 32.7
     // against 34.9 ms for 2000 steps; FP32 37.7 against 30.3)
+    const bool tiles = tile_runs(c) && !c->d.periodic_x && !c->d.periodic_y;
     const bool pairs = c->sweeps == 2 && !c->halo8 && c->esz == 4;
     for (int i = 0; i < n;) {
         if (i % every == 0) {
             char *dst = (char *)c->ck + (size_t)(i / every) * 2 * pb;
             TSMI_HIP(hipMemcpyAsync(dst, c->psi_base[c->cur][0], pb, hipMemcpyDeviceToDevice, c->stream));
             TSMI_HIP(hipMemcpyAsync(dst + pb, c->psi_base[c->cur][1], pb, hipMemcpyDeviceToDevice, c->stream));
+        }
+        if (tiles) {   // up to the next checkpoint
+            const int m = std::min(n, (i / every + 1) * every) - i;
+            if (const int st = tile_passes(c, m, false)) return st;
+            i += m;
+            continue;
         }
         const bool two = pairs && i + 1 < n && (i + 1) % every != 0;
         // periodic: the halo exchange after every step but the last, as evolve

@@ -1,0 +1,174 @@
+// tsmi_tile.hip -- planning and launching the tile passes (tile_kernel.hpp):
+// several real-time steps of a small or medium lattice per launch.
+#include "tsmi_hip.h"
+
+#include <hip/hip_runtime.h>
+
+#include <algorithm>
+#include <cmath>
+#include <complex>
+#include <cstring>
+#include <string>
+
+#include "common.hpp"
+#include "context.hpp"
+#include "frame.hpp"
+#include "tile_kernel.hpp"
+
+using namespace tsmi;
+
+namespace {
+
+// Rows per wave of the compiled instances.
+constexpr int kRows32[] = {4, 8, 12}, kRows64[] = {4, 6, 8};
+
+struct Plan {
+    int r = 0, nw = 0, cols = 0, rows = 0, strips = 0, segs = 0;
+    double us = 1e30;    // modelled time per step
+};
+
+// The tile shape of a pass of `steps` steps: the one with the least modelled time.
+// A launch costs about 5 us whatever it does; a step costs each SIMD its rows
+// (about 0.17 us a row in FP32, 0.27 in FP64 with several waves per SIMD, up to
+// 60% more for a wave alone) and 0.35 us of exchanges.  Measured around it, us
+// per step: 256^2 FP64 4 rows x 8 waves 6.9, 4.9, 4.4 for 1, 2, 3 steps, 8 x 8
+// 10.7, 7.9, 7.1; 1024^2 FP32 8 x 8 9.4, 6.7, 9.8 (3 steps: more than one
+// workgroup per compute unit), 12 x 8 12.4, 8.9, 7.3, 7.2, 7.0 (5 steps).
+Plan plan(int W, int H, int esz, int steps) {
+    Plan best;
+    const int a = kApron * steps;
+    const int *rr = esz == 4 ? kRows32 : kRows64;
+    const double c_row = esz == 4 ? 0.17 : 0.27, x = 0.35, t0 = 5.0;
+    for (int i = 0; i < 3; ++i)
+        for (int nw = 4; nw <= kTileWavesMax; nw += 4) {
+            Plan p;
+            p.r = rr[i];
+            p.nw = nw;
+            p.cols = kTileCols - 2 * a;
+            p.rows = nw * p.r - 2 * a;
+            if (p.cols < 2 || p.rows < 2) continue;
+            p.strips = (W + p.cols - 1) / p.cols;
+            p.segs = (H + p.rows - 1) / p.rows;
+            const double n = p.strips * p.segs / 256.0;              // workgroups per compute unit
+            const double per_cu = n < 6 ? std::ceil(n) : n + 0.5;    // ... on the busiest one
+            const double waves = std::min(per_cu * nw / 4.0, 3.0);   // waves per SIMD
+            p.us = t0 / steps + per_cu * nw * p.r / 4.0 * c_row * (1 + 0.6 / waves) + x;
+            if (p.us < best.us) best = p;
+        }
+    return best;
+}
+
+int best_steps(int W, int H, int esz, int most) {
+    int k = 1;
+    double us = 1e30;
+    for (int s = 1; s <= std::min(most, 8); ++s) {
+        const Plan p = plan(W, H, esz, s);
+        if (p.us < us) {
+            us = p.us;
+            k = s;
+        }
+    }
+    return k;
+}
+
+template <typename T, bool LHY, int MODE, int R>
+int launch(tsmi_ctx *c, const TileParams<T> &p, const Plan &g) {
+    if (int st = ctx_time_mark(c, p.steps > 1, 0)) return st;
+    hipLaunchKernelGGL((tile_kernel<T, LHY, MODE, R>), dim3(g.strips * g.segs), dim3(g.nw * kWave), 0, c->stream, p);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return set_error(TSMI_E_HIP, std::string("tile_kernel: ") + hipGetErrorString(e));
+    return ctx_time_mark(c, p.steps > 1, 1);
+}
+
+template <typename T, bool LHY, int R>
+int launch_mode(tsmi_ctx *c, const TileParams<T> &p, const Plan &g) {
+    if (c->mode == 0) return launch<T, LHY, 0, R>(c, p, g);
+    if (c->mode == 1) return launch<T, LHY, 1, R>(c, p, g);
+    return launch<T, LHY, -1, R>(c, p, g);
+}
+
+template <typename T, bool LHY>
+int launch_rows(tsmi_ctx *c, const TileParams<T> &p, const Plan &g) {
+    constexpr const int *rr = sizeof(T) == 4 ? kRows32 : kRows64;
+    if (g.r == rr[0]) return launch_mode<T, LHY, rr[0]>(c, p, g);
+    if (g.r == rr[1]) return launch_mode<T, LHY, rr[1]>(c, p, g);
+    return launch_mode<T, LHY, rr[2]>(c, p, g);
+}
+
+template <typename T>
+int pass(tsmi_ctx *c, int steps, bool wrap) {
+    TileParams<T> p;
+    std::memset(&p, 0, sizeof(p));
+    const int nb = 1 - c->cur;
+    p.in_re = (const T *)c->psi_re[c->cur];
+    p.in_im = (const T *)c->psi_im[c->cur];
+    p.out_re = (T *)c->psi_re[nb];
+    p.out_im = (T *)c->psi_im[nb];
+    p.ph = (const T *)c->ph;
+    p.W = c->W; p.H = c->H; p.pitch = c->pitch;
+    p.nx = wrap ? c->d.dim_x : 0;
+    p.ny = wrap ? c->d.dim_y : 0;
+    p.steps = steps;
+    const Plan g = plan(c->W, c->H, c->esz, steps);
+    if (g.r == 0) return set_error(TSMI_E_INVALID, "tile pass: no tile for this many steps");
+    p.n_strips = g.strips; p.cols = g.cols; p.rows = g.rows;
+    p.mH = (T)c->mH; p.tH = (T)c->tH; p.mV = (T)c->mV; p.tV = (T)c->tV;
+    p.unH = (T)c->unH; p.unV = (T)c->unV;
+    p.c_nl = (T)c->c_nl_s; p.c_lhy = (T)c->c_lhy_s;
+    // The merged V0 V0 pass has a frame factor g2 of its own; a step followed by
+    // it applies g2 where its own and the next V0 would have applied gV^2.  The
+    // sign of g2 / gV^2 goes into the modulus (a phase near pi would leave the
+    // small-angle forms); what is left of its phase, an effect of the rounded
+    // coefficients, commutes with every pass and is spread over the k steps.
+    const double by = c->d.delta_t / (4. * c->d.mass * c->d.delta_y * c->d.delta_y);
+    const Axis one = frame_axis(c->aV, c->bV, false, c->esz);
+    const Axis two = frame_axis(std::cos(2 * by), std::sin(2 * by), false, c->esz);
+    std::complex<double> q = two.g / (one.g * one.g);
+    const double sign = q.real() < 0 ? -1.0 : 1.0;
+    q *= sign;
+    p.m2 = (T)two.m; p.t2 = (T)two.t; p.un2 = (T)two.un;
+    p.mode2 = two.form;
+    p.mag = c->corr_abs;
+    p.mag_mid = sign * c->corr_abs * std::abs(q);
+    p.dphi = (T)(-(steps - 1.0) / steps * std::arg(q));
+    const bool lhy = c->c_lhy != 0.0;
+    const int st = lhy ? launch_rows<T, true>(c, p, g) : launch_rows<T, false>(c, p, g);
+    if (!st) c->cur = nb;
+    return st;
+}
+
+}  // namespace
+
+namespace tsmi {
+
+bool tile_wraps(const tsmi_ctx *c) {
+    return c->d.periodic_x && c->d.periodic_y && c->d.dim_x % 2 == 0 && c->d.dim_y % 2 == 0;
+}
+
+// Real time with the one-plane phase, no segment height or steps per pass asked
+// for, offsets within 31 bits, and a lattice small enough that a wave's row
+// latency bounds the streaming passes: us per step, streamed against tiles, 64^2
+// FP64 17.3 / 2.8, 256^2 FP64 23.1 / 4.4, FP32 16.6 / 3.2, 512^2 FP32 14.5 / 3.9,
+// 1024^2 FP32 17.0 / 6.6, FP64 23.6 / 10.5, 2048^2 FP32 22.1 / 17.9, FP64 33.6 /
+// 43.4.
+bool tile_runs(const tsmi_ctx *c) {
+    const long most = c->esz == 4 ? 5L << 20 : 3L << 19;
+    return !c->d.imag_time && c->ph_mode && c->d.sweeps == 0 && c->d.tile_rows == 0 && c->H > 1 &&
+           (long)c->W * c->H <= most && (long)c->pitch * c->Hd * c->esz < (1L << 31);
+}
+
+int tile_steps(const tsmi_ctx *c, int most) { return best_steps(c->W, c->H, c->esz, most); }
+
+int tile_pass(tsmi_ctx *c, int steps, bool wrap) {
+    return c->esz == 4 ? pass<float>(c, steps, wrap) : pass<double>(c, steps, wrap);
+}
+
+int tile_passes(tsmi_ctx *c, int n, bool wrap) {
+    if (n <= 0) return TSMI_OK;
+    const int k = tile_steps(c, n), passes = (n + k - 1) / k;
+    int st = TSMI_OK;
+    for (int i = 0; i < passes && !st; ++i) st = tile_pass(c, n / passes + (i < n % passes ? 1 : 0), wrap);
+    return st;
+}
+
+}  // namespace tsmi
