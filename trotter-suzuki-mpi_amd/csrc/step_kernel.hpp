@@ -365,14 +365,17 @@ __device__ __forceinline__ void sincos_t(float x, float *s, float *c) {
         *c = ((q + 1) & 2) ? -b : b;
     }
 }
+__device__ __forceinline__ void sincos_t(double x, double *s, double *c) { sincos(x, s, c); }
 // The same for |x| <= 2^50: three-part Cody-Waite reduction by pi/2 with fused
 // multiply-adds (159 bits of pi/2; k is exact enough below 2^50 that |r| stays
 // within an ulp of pi/4), then the Taylor polynomials of sin (to r^17) and cos
-// (to r^16), truncation 8e-20 and 2e-18; the quadrant is k mod 4.  The device
-// sincos carries a reduction for huge arguments, inlined into every potential
-// pass: 256^2 FP64 in a harmonic trap, where angles exceed 1/64, 53.7 us per
-// two-step launch with it.
-__device__ __forceinline__ void sincos_t(double x, double *s, double *c) {
+// (to r^16), truncation 8e-20 and 2e-18; the quadrant is k mod 4.  For the
+// tile passes: the device sincos carries a reduction for huge arguments (256^2
+// FP64 in a harmonic trap, where angles exceed 1/64, 53.7 us per two-step
+// streaming launch with it).  The streaming passes keep the device sincos: this
+// one in their cold branch changes the schedule of the whole row loop (two-step
+// pass at 8192^2, where no angle exceeds 1/64: 376 -> 417 us per step, same bits).
+__device__ __forceinline__ void sincos_near(double x, double *s, double *c) {
     const double k = rint(x * 0.63661977236758134308);
     double r = fma(-k, 1.57079632679489655800, x);
     r = fma(-k, 6.12323399573676603587e-17, r);
@@ -401,7 +404,7 @@ __device__ __forceinline__ void sincos_t(double x, double *s, double *c) {
     *c = ((q + 1) & 2) ? -b : b;
 }
 // An angle above 2^50, whose own rounding (an ulp of 1/8 or more) leaves no
-// phase: brought within sincos_t's range, bounded for every finite angle; an
+// phase: brought within sincos_near's range, bounded for every finite angle; an
 // infinite one becomes NaN.
 __device__ __forceinline__ double wrap_far(double x) {
     const double n = rint(x * 0.15915494309189534561);
@@ -409,7 +412,6 @@ __device__ __forceinline__ double wrap_far(double x) {
     r = fma(-n, 2.44929359829470641435e-16, r);
     return fabs(r) <= 0x1p50 ? r : x * 0.0;
 }
-__device__ __forceinline__ float wrap_far(float x) { return x; }
 __device__ __forceinline__ float exp_t(float x) { return expf(x); }
 __device__ __forceinline__ double exp_t(double x) { return exp(x); }
 __device__ __forceinline__ float sqrt_t(float x) { return sqrtf(x); }
@@ -429,42 +431,48 @@ __device__ __forceinline__ bool wave_all_le(double v, double thr) {
 // to within the format: truncation below 2e-10 relative in FP32 (sin to x^3,
 // cos to x^4, exp to x^4) and below 1e-19 in FP64 (sin to x^7, cos to x^8,
 // exp to x^8).  Otherwise the general routines run.
-template <typename T, int VEC>
+// NEAR: the FP64 general routine is sincos_near (see there).
+template <typename T, int VEC, bool NEAR = false>
 __device__ __forceinline__ void sincos_row(const T (&x)[VEC], T (&s)[VEC], T (&c)[VEC]) {
     T m = fabs(x[0]);
 #pragma unroll
     for (int k = 1; k < VEC; ++k) m = fmax(m, fabs(x[k]));
-    if constexpr (sizeof(T) == 4) {
-        // the short polynomials always, the general routine over them in the rare
-        // wave with a large angle (no copies on the common path)
-#pragma unroll
-        for (int k = 0; k < VEC; ++k) {
-            const T r = x[k], r2 = r * r;
-            s[k] = fmaf(r * r2, -0.166666667f, r);
-            c[k] = fmaf(r2, fmaf(r2, 0.0416666667f, -0.5f), 1.0f);
-        }
-        if (__builtin_expect(!wave_all_le(m, T(0.015625)), 0)) {
-#pragma unroll
-            for (int k = 0; k < VEC; ++k) sincos_t(x[k], &s[k], &c[k]);
-        }
-    } else if (wave_all_le(m, T(0.015625))) {
-#pragma unroll
-        for (int k = 0; k < VEC; ++k) {
-            const T r = x[k], r2 = r * r;
+    auto small = [](T r, T *s, T *c) {
+        const T r2 = r * r;
+        if constexpr (sizeof(T) == 4) {
+            *s = fmaf(r * r2, -0.166666667f, r);
+            *c = fmaf(r2, fmaf(r2, 0.0416666667f, -0.5f), 1.0f);
+        } else {
             T ps = fma(r2, -1.0 / 5040.0, 1.0 / 120.0);
             ps = fma(r2, ps, -1.0 / 6.0);
-            s[k] = fma(r * r2, ps, r);
+            *s = fma(r * r2, ps, r);
             T pc = fma(r2, 1.0 / 40320.0, -1.0 / 720.0);
             pc = fma(r2, pc, 1.0 / 24.0);
             pc = fma(r2, pc, -0.5);
-            c[k] = fma(r2, pc, 1.0);
+            *c = fma(r2, pc, 1.0);
+        }
+    };
+    if constexpr (NEAR && sizeof(T) == 8) {
+        if (wave_all_le(m, T(0.015625))) {
+#pragma unroll
+            for (int k = 0; k < VEC; ++k) small(x[k], &s[k], &c[k]);
+        } else {
+            const bool far = !wave_all_le(m, T(0x1p50));
+#pragma unroll
+            for (int k = 0; k < VEC; ++k) {
+                T r = x[k];
+                if (__builtin_expect(far, 0)) r = wrap_far(r);
+                sincos_near(r, &s[k], &c[k]);
+            }
         }
     } else {
+        // the short polynomials always, the general routine over them in the rare
+        // wave with a large angle (no copies on the common path)
 #pragma unroll
-        for (int k = 0; k < VEC; ++k) {
-            T r = x[k];
-            if (__builtin_expect(!wave_all_le(m, T(0x1p50)), 0)) r = wrap_far(r);
-            sincos_t(r, &s[k], &c[k]);
+        for (int k = 0; k < VEC; ++k) small(x[k], &s[k], &c[k]);
+        if (__builtin_expect(!wave_all_le(m, T(0.015625)), 0)) {
+#pragma unroll
+            for (int k = 0; k < VEC; ++k) sincos_t(x[k], &s[k], &c[k]);
         }
     }
 }

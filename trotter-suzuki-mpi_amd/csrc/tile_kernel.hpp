@@ -77,7 +77,7 @@ __device__ __forceinline__ void tile_ppass(Row<T, 2> &a, Row<T, 2> &b, const T (
     ang[1] = angle(a, 1, pa[1]);
     ang[2] = angle(b, 0, pb[0]);
     ang[3] = angle(b, 1, pb[1]);
-    sincos_row<T, 4>(ang, sn, cs);
+    sincos_row<T, 4, true>(ang, sn, cs);
     const T ca[2] = {cs[0], cs[1]}, sa[2] = {sn[0], sn[1]}, cb[2] = {cs[2], cs[3]}, sb[2] = {sn[2], sn[3]};
     rotate_row_ph<T, 2>(a, ca, sa, mag);
     rotate_row_ph<T, 2>(b, cb, sb, mag);

@@ -96,7 +96,7 @@ int launch_rows(tsmi_ctx *c, const TileParams<T> &p, const Plan &g) {
 }
 
 template <typename T>
-int pass(tsmi_ctx *c, int steps, bool wrap) {
+int pass(tsmi_ctx *c, int steps, bool wrap, long double &drift) {
     TileParams<T> p;
     std::memset(&p, 0, sizeof(p));
     const int nb = 1 - c->cur;
@@ -115,22 +115,31 @@ int pass(tsmi_ctx *c, int steps, bool wrap) {
     p.mH = (T)c->mH; p.tH = (T)c->tH; p.mV = (T)c->mV; p.tV = (T)c->tV;
     p.unH = (T)c->unH; p.unV = (T)c->unV;
     p.c_nl = (T)c->c_nl_s; p.c_lhy = (T)c->c_lhy_s;
-    // The merged V0 V0 pass has a frame factor g2 of its own; a step followed by
-    // it applies g2 where its own and the next V0 would have applied gV^2.  The
-    // sign of g2 / gV^2 goes into the modulus (a phase near pi would leave the
-    // small-angle forms); what is left of its phase, an effect of the rounded
-    // coefficients, commutes with every pass and is spread over the k steps.
+    // The merged V0 V0 pass (factors m2, t2) stands for the square of V0's (m, t):
+    // its eigenvalue is 1/q of the exact one, q = (m + i t)^2 / (m2 + i t2), so a
+    // step followed by it applies |q| with |corr|.  The sign of q goes into the
+    // modulus (a phase near pi would leave the small-angle forms); what is left of
+    // its phase, an effect of the rounded coefficients, commutes with every pass
+    // and is spread over the k steps.  The moduli are rounded to FP64: a rounding
+    // that repeats every step would be a drift of the norm (1.8e-16 per step at
+    // 64^2), so the last step of a pass takes back what the pass's and the
+    // call's earlier ones left (drift: the log of what was applied over what was
+    // meant).
     const double by = c->d.delta_t / (4. * c->d.mass * c->d.delta_y * c->d.delta_y);
-    const Axis one = frame_axis(c->aV, c->bV, false, c->esz);
+    typedef std::complex<long double> zl;
     const Axis two = frame_axis(std::cos(2 * by), std::sin(2 * by), false, c->esz);
-    std::complex<double> q = two.g / (one.g * one.g);
-    const double sign = q.real() < 0 ? -1.0 : 1.0;
+    const zl v1(c->mV, c->tV), v2(two.m, two.t);
+    zl q = v1 * v1 / v2;
+    const long double sign = q.real() < 0 ? -1.0L : 1.0L;
     q *= sign;
     p.m2 = (T)two.m; p.t2 = (T)two.t; p.un2 = (T)two.un;
     p.mode2 = two.form;
-    p.mag = c->corr_abs;
-    p.mag_mid = sign * c->corr_abs * std::abs(q);
-    p.dphi = (T)(-(steps - 1.0) / steps * std::arg(q));
+    const long double mid = c->corr_abs * std::abs(q);
+    p.mag_mid = (double)(sign * mid);
+    drift += (steps - 1) * std::log(std::fabs((long double)p.mag_mid) / mid);
+    p.mag = (double)(c->corr_abs * (1.0L - drift));
+    drift += std::log((long double)p.mag / c->corr_abs);
+    p.dphi = (T)(-(steps - 1.0L) / steps * std::arg(q));
     const bool lhy = c->c_lhy != 0.0;
     const int st = lhy ? launch_rows<T, true>(c, p, g) : launch_rows<T, false>(c, p, g);
     if (!st) c->cur = nb;
@@ -159,15 +168,16 @@ bool tile_runs(const tsmi_ctx *c) {
 
 int tile_steps(const tsmi_ctx *c, int most) { return best_steps(c->W, c->H, c->esz, most); }
 
-int tile_pass(tsmi_ctx *c, int steps, bool wrap) {
-    return c->esz == 4 ? pass<float>(c, steps, wrap) : pass<double>(c, steps, wrap);
+static int tile_pass(tsmi_ctx *c, int steps, bool wrap, long double &drift) {
+    return c->esz == 4 ? pass<float>(c, steps, wrap, drift) : pass<double>(c, steps, wrap, drift);
 }
 
 int tile_passes(tsmi_ctx *c, int n, bool wrap) {
     if (n <= 0) return TSMI_OK;
     const int k = tile_steps(c, n), passes = (n + k - 1) / k;
+    long double drift = 0.0L;
     int st = TSMI_OK;
-    for (int i = 0; i < passes && !st; ++i) st = tile_pass(c, n / passes + (i < n % passes ? 1 : 0), wrap);
+    for (int i = 0; i < passes && !st; ++i) st = tile_pass(c, n / passes + (i < n % passes ? 1 : 0), wrap, drift);
     return st;
 }
 
