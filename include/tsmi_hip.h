@@ -75,6 +75,11 @@ int tsmi_set_stream(tsmi_ctx *ctx, void *hip_stream);
  * constructed on (CPUBlock borrows state->p_real/p_imag, src/cpukernel.cpp:244-245). */
 int tsmi_set_state(tsmi_ctx *ctx, const double *re, const double *im);
 
+/* The same from, and the whole tile into, one array of W*H complex doubles
+ * (re, im interleaved).  No reference counterpart; the get syncs. */
+int tsmi_set_state_complex(tsmi_ctx *ctx, const double *psi);
+int tsmi_get_state_complex(tsmi_ctx *ctx, double *psi);
+
 /* The same, from device memory: re/im point to W*H FP64 arrays (row stride W)
  * on the context's device.  Asynchronous on the context stream. */
 int tsmi_set_state_device(tsmi_ctx *ctx, const double *re, const double *im);
@@ -176,7 +181,7 @@ int tsmi_adjoint_device(tsmi_ctx *ctx, const double *g_re, const double *g_im, d
  * of lattice i's tile, out[3..5] strips, segments and rows per segment of its
  * dominant pass, out[6] steps per pass (1 or 2).
  * set_state / set_exp_potential / get_state take W*H FP64 host arrays of
- * lattice i; get_state syncs. */
+ * lattice i (the _complex forms one array of complex doubles); get_state syncs. */
 typedef struct tsmi_batch tsmi_batch;
 int tsmi_batch_create(const tsmi_desc *descs, int32_t n, tsmi_batch **out);
 void tsmi_batch_destroy(tsmi_batch *batch);
@@ -184,6 +189,8 @@ int tsmi_batch_set_state(tsmi_batch *batch, int32_t i, const double *re, const d
 int tsmi_batch_set_exp_potential(tsmi_batch *batch, int32_t i, const double *e_re, const double *e_im);
 int tsmi_batch_evolve(tsmi_batch *batch, int32_t n_steps);
 int tsmi_batch_get_state(tsmi_batch *batch, int32_t i, double *re, double *im);
+int tsmi_batch_set_state_complex(tsmi_batch *batch, int32_t i, const double *psi);
+int tsmi_batch_get_state_complex(tsmi_batch *batch, int32_t i, double *psi);
 int tsmi_batch_tune(tsmi_batch *batch, int32_t steps, double *ms_per_step);
 int tsmi_batch_info(const tsmi_batch *batch, int32_t i, int32_t out[7]);
 int tsmi_batch_synchronize(tsmi_batch *batch);
@@ -221,6 +228,7 @@ void tsmi_pair_destroy(tsmi_pair *pair);
  * ITrotterKernel::update_potential(..., which)), the raw potential for
  * tsmi_pair_energy. */
 int tsmi_pair_set_state(tsmi_pair *pair, int32_t which, const double *re, const double *im);
+int tsmi_pair_set_state_complex(tsmi_pair *pair, int32_t which, const double *psi);
 int tsmi_pair_set_exp_potential(tsmi_pair *pair, int32_t which, const double *e_re, const double *e_im);
 int tsmi_pair_set_potential(tsmi_pair *pair, int32_t which, const double *v);
 
@@ -248,6 +256,7 @@ int tsmi_pair_rabi(tsmi_pair *pair, double var, int32_t normalize);
 
 /* get_sample of one component, the whole tile (src/cpukernel.cpp:572-579); syncs. */
 int tsmi_pair_get_state(tsmi_pair *pair, int32_t which, double *re, double *im);
+int tsmi_pair_get_state_complex(tsmi_pair *pair, int32_t which, double *psi);
 
 /* Solver::calculate_energy_expected_values for two components
  * (src/solver.cpp:244-564, angular velocity 0): out[0..11] = total, kinetic a,

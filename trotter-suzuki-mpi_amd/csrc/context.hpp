@@ -11,6 +11,7 @@
 
 #include <vector>
 
+#include "stage.hpp"
 #include "tsmi_hip.h"
 
 struct tsmi_ctx {
@@ -72,6 +73,7 @@ struct tsmi_ctx {
     bool ck_valid = false;
     void *adj = nullptr;              // 8 planes: adjoint re/im x2, reversed state re/im x2
     double *grad = nullptr;           // FP64, pitched
+    tsmi::HostStage stage;            // pinned chunks of the host transfers
 };
 
 namespace tsmi {

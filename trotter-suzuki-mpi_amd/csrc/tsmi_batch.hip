@@ -37,6 +37,7 @@
 #include "batch_kernel.hpp"
 #include "common.hpp"
 #include "frame.hpp"
+#include "stage.hpp"
 #include "tsmi_hip.h"
 
 using namespace tsmi;
@@ -110,6 +111,7 @@ struct tsmi_batch {
     hipStream_t own = nullptr, stream = nullptr, side = nullptr;
     hipEvent_t fork = nullptr, join = nullptr;
     std::map<std::tuple<int, int, int>, GraphRec> graphs;
+    HostStage stage;                          // pinned chunks of the host transfers
 };
 
 namespace {
@@ -482,6 +484,35 @@ int reset_divisor(tsmi_batch *b, const Lattice &L) {
     return TSMI_OK;
 }
 
+// A host state of lattice L, two planes or (im null) one of complex doubles.
+int upload_state(tsmi_batch *b, const Lattice &L, const double *re, const double *im) {
+    const int buf = b->cur[L.group()];
+    void *dr = b->arena + L.psi[buf][0], *di = b->arena + L.psi[buf][1];
+    const size_t W = (size_t)L.W, H = (size_t)L.H;
+    TSMI_HIPB(b->esz == 8 ? b->stage.upload(b->stream, (double *)dr, (double *)di, (long)L.pitch, re, im, W, H, W)
+                          : b->stage.upload(b->stream, (float *)dr, (float *)di, (long)L.pitch, re, im, W, H, W));
+    return reset_divisor(b, L);
+}
+
+int download_state(tsmi_batch *b, const Lattice &L, double *re, double *im) {
+    const int buf = b->cur[L.group()];
+    double *div = nullptr;
+    if (b->imag) {
+        div = (double *)(b->arena + L.div);
+        hipLaunchKernelGGL(divisor_kernel<>, dim3(1), dim3(kWave), 0, b->stream,
+                           (const double *)(b->arena + L.partials) + (size_t)buf * (size_t)L.max_waves,
+                           (const int *)(b->arena + L.part_n) + buf, L.d.delta_x * L.d.delta_y, L.d.norm_target, div);
+        TSMI_HIPB(hipGetLastError());
+    }
+    const void *sr = b->arena + L.psi[buf][0], *si = b->arena + L.psi[buf][1];
+    const size_t W = (size_t)L.W, H = (size_t)L.H;
+    TSMI_HIPB(b->esz == 8 ? b->stage.download(b->stream, (const double *)sr, (const double *)si, (long)L.pitch, re, im,
+                                              W, H, W, div)
+                          : b->stage.download(b->stream, (const float *)sr, (const float *)si, (long)L.pitch, re, im,
+                                              W, H, W, div));
+    return TSMI_OK;
+}
+
 // The fused passes of a doubly periodic lattice read E over the whole 8-wide
 // halo: the reference-tile table with every halo cell replaced by its wrapped
 // inner cell.
@@ -643,11 +674,14 @@ int tsmi_batch_set_state(tsmi_batch *b, int32_t i, const double *re, const doubl
     Lattice *L = lattice_at(b, i, "tsmi_batch_set_state");
     if (!L) return TSMI_E_INVALID;
     if (!re || !im) return set_error(TSMI_E_INVALID, "tsmi_batch_set_state: null argument");
-    const int buf = b->cur[L->group()];
-    int st = upload_host_plane(b, *L, L->psi[buf][0], re);
-    if (!st) st = upload_host_plane(b, *L, L->psi[buf][1], im);
-    if (!st) st = reset_divisor(b, *L);
-    return st;
+    return upload_state(b, *L, re, im);
+}
+
+int tsmi_batch_set_state_complex(tsmi_batch *b, int32_t i, const double *psi) {
+    Lattice *L = lattice_at(b, i, "tsmi_batch_set_state_complex");
+    if (!L) return TSMI_E_INVALID;
+    if (!psi) return set_error(TSMI_E_INVALID, "tsmi_batch_set_state_complex: null argument");
+    return upload_state(b, *L, psi, nullptr);
 }
 
 int tsmi_batch_set_exp_potential(tsmi_batch *b, int32_t i, const double *e_re, const double *e_im) {
@@ -723,31 +757,14 @@ int tsmi_batch_get_state(tsmi_batch *b, int32_t i, double *re, double *im) {
     Lattice *L = lattice_at(b, i, "tsmi_batch_get_state");
     if (!L) return TSMI_E_INVALID;
     if (!re || !im) return set_error(TSMI_E_INVALID, "tsmi_batch_get_state: null argument");
-    const size_t n = (size_t)L->W * (size_t)L->H, es = (size_t)b->esz;
-    const int buf = b->cur[L->group()];
-    std::vector<unsigned char> tr(n * es), ti(n * es);
-    double div = 1.0;
-    TSMI_HIPB(hipMemcpy2DAsync(tr.data(), (size_t)L->W * es, b->arena + L->psi[buf][0], (size_t)L->pitch * es,
-                               (size_t)L->W * es, L->H, hipMemcpyDeviceToHost, b->stream));
-    TSMI_HIPB(hipMemcpy2DAsync(ti.data(), (size_t)L->W * es, b->arena + L->psi[buf][1], (size_t)L->pitch * es,
-                               (size_t)L->W * es, L->H, hipMemcpyDeviceToHost, b->stream));
-    if (b->imag) {
-        hipLaunchKernelGGL(divisor_kernel<>, dim3(1), dim3(kWave), 0, b->stream,
-                           (const double *)(b->arena + L->partials) + (size_t)buf * (size_t)L->max_waves,
-                           (const int *)(b->arena + L->part_n) + buf, L->d.delta_x * L->d.delta_y, L->d.norm_target,
-                           (double *)(b->arena + L->div));
-        TSMI_HIPB(hipGetLastError());
-        TSMI_HIPB(hipMemcpyAsync(&div, b->arena + L->div, sizeof(double), hipMemcpyDeviceToHost, b->stream));
-    }
-    TSMI_HIPB(hipStreamSynchronize(b->stream));
-    for (size_t k = 0; k < n; ++k) {
-        double vr, vi;
-        if (es == 8) { vr = ((const double *)tr.data())[k]; vi = ((const double *)ti.data())[k]; }
-        else         { vr = ((const float *)tr.data())[k];  vi = ((const float *)ti.data())[k]; }
-        re[k] = vr / div;
-        im[k] = vi / div;
-    }
-    return TSMI_OK;
+    return download_state(b, *L, re, im);
+}
+
+int tsmi_batch_get_state_complex(tsmi_batch *b, int32_t i, double *psi) {
+    Lattice *L = lattice_at(b, i, "tsmi_batch_get_state_complex");
+    if (!L) return TSMI_E_INVALID;
+    if (!psi) return set_error(TSMI_E_INVALID, "tsmi_batch_get_state_complex: null argument");
+    return download_state(b, *L, psi, nullptr);
 }
 
 int tsmi_batch_tune(tsmi_batch *b, int32_t steps, double *ms_per_step) {

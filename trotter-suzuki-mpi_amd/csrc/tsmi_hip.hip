@@ -183,20 +183,14 @@ int free_all(tsmi_ctx *c) {
     return TSMI_OK;
 }
 
-// Uploads W x H doubles into a pitched plane of the context precision.
-int upload_plane(tsmi_ctx *c, void *dst, const double *src) {
-    const size_t n = (size_t)c->W * (size_t)c->H;
-    if (c->esz == 8) {
-        TSMI_HIP(hipMemcpy2DAsync(dst, (size_t)c->pitch * 8, src, (size_t)c->W * 8, (size_t)c->W * 8, c->H,
-                                  hipMemcpyHostToDevice, c->stream));
-        TSMI_HIP(hipStreamSynchronize(c->stream));
-    } else {
-        std::vector<float> tmp(n);
-        for (size_t i = 0; i < n; ++i) tmp[i] = (float)src[i];   // rounded once
-        TSMI_HIP(hipMemcpy2DAsync(dst, (size_t)c->pitch * 4, tmp.data(), (size_t)c->W * 4, (size_t)c->W * 4, c->H,
-                                  hipMemcpyHostToDevice, c->stream));
-        TSMI_HIP(hipStreamSynchronize(c->stream));
-    }
+// Uploads a host state, two planes or (im null) one of complex doubles.
+int upload_state(tsmi_ctx *c, const double *re, const double *im) {
+    const size_t W = (size_t)c->W, H = (size_t)c->H;
+    void *dr = c->psi_re[c->cur], *di = c->psi_im[c->cur];
+    TSMI_HIP(c->esz == 8 ? c->stage.upload(c->stream, (double *)dr, (double *)di, (long)c->pitch, re, im, W, H, W)
+                         : c->stage.upload(c->stream, (float *)dr, (float *)di, (long)c->pitch, re, im, W, H, W));
+    c->has_state = true;
+    c->div_pending = false;
     return TSMI_OK;
 }
 
@@ -210,13 +204,17 @@ const double *pending_div(tsmi_ctx *c) {
     return c->div;
 }
 
-int current_div(tsmi_ctx *c, double *out) {
-    *out = 1.0;
-    if (const double *d = pending_div(c)) {
-        TSMI_HIP(hipGetLastError());
-        TSMI_HIP(hipMemcpyAsync(out, d, sizeof(double), hipMemcpyDeviceToHost, c->stream));
-        TSMI_HIP(hipStreamSynchronize(c->stream));
-    }
+// A window of the current state into host arrays, as upload_state takes them
+// (divided by a pending renormalisation, src/cpukernel.cpp:559-560).
+int download_state(tsmi_ctx *c, size_t stride, size_t x, size_t y, size_t w, size_t h, double *re, double *im) {
+    const double *div = pending_div(c);
+    if (div) TSMI_HIP(hipGetLastError());
+    const size_t off = y * (size_t)c->pitch + x;
+    const void *sr = c->psi_re[c->cur], *si = c->psi_im[c->cur];
+    TSMI_HIP(c->esz == 8 ? c->stage.download(c->stream, (const double *)sr + off, (const double *)si + off,
+                                             (long)c->pitch, re, im, w, h, stride, div)
+                         : c->stage.download(c->stream, (const float *)sr + off, (const float *)si + off,
+                                             (long)c->pitch, re, im, w, h, stride, div));
     return TSMI_OK;
 }
 
@@ -1034,12 +1032,13 @@ int tsmi_set_stream(tsmi_ctx *c, void *s) {
 int tsmi_set_state(tsmi_ctx *c, const double *re, const double *im) {
     if (c) c->ck_valid = false;
     if (!c || !re || !im) return fail(TSMI_E_INVALID, "tsmi_set_state: null argument");
-    int st = upload_plane(c, c->psi_re[c->cur], re);
-    if (!st) st = upload_plane(c, c->psi_im[c->cur], im);
-    if (st) return st;
-    c->has_state = true;
-    c->div_pending = false;
-    return TSMI_OK;
+    return upload_state(c, re, im);
+}
+
+int tsmi_set_state_complex(tsmi_ctx *c, const double *psi) {
+    if (c) c->ck_valid = false;
+    if (!c || !psi) return fail(TSMI_E_INVALID, "tsmi_set_state_complex: null argument");
+    return upload_state(c, psi, nullptr);
 }
 
 int tsmi_set_state_device(tsmi_ctx *c, const double *re, const double *im) {
@@ -1347,43 +1346,13 @@ int tsmi_get_sample(tsmi_ctx *c, size_t stride, size_t x, size_t y, size_t w, si
     if (x + w > (size_t)c->W || y + h > (size_t)c->H || stride < w)
         return fail(TSMI_E_INVALID, "tsmi_get_sample: window outside the tile");
     if (w == 0 || h == 0) return TSMI_OK;
-    double div = 1.0;
-    int st = current_div(c, &div);
-    if (st) return st;
-    const size_t es = (size_t)c->esz;
-    const size_t off = (y * (size_t)c->pitch + x) * es;
-    const bool scale = c->d.imag_time && c->div_pending;
-    if (es == 8 && !scale) {
-        // FP64 with nothing to apply: straight into the caller's rows
-        TSMI_HIP(hipMemcpy2DAsync(re, stride * 8, (const char *)c->psi_re[c->cur] + off, (size_t)c->pitch * 8, w * 8,
-                                  h, hipMemcpyDeviceToHost, c->stream));
-        TSMI_HIP(hipMemcpy2DAsync(im, stride * 8, (const char *)c->psi_im[c->cur] + off, (size_t)c->pitch * 8, w * 8,
-                                  h, hipMemcpyDeviceToHost, c->stream));
-        TSMI_HIP(hipStreamSynchronize(c->stream));
-        return TSMI_OK;
-    }
-    // staging (left uninitialised: the copies fill it)
-    std::unique_ptr<unsigned char[]> tr(new unsigned char[w * h * es]), ti(new unsigned char[w * h * es]);
-    TSMI_HIP(hipMemcpy2DAsync(tr.get(), w * es, (const char *)c->psi_re[c->cur] + off, (size_t)c->pitch * es, w * es,
-                              h, hipMemcpyDeviceToHost, c->stream));
-    TSMI_HIP(hipMemcpy2DAsync(ti.get(), w * es, (const char *)c->psi_im[c->cur] + off, (size_t)c->pitch * es, w * es,
-                              h, hipMemcpyDeviceToHost, c->stream));
-    TSMI_HIP(hipStreamSynchronize(c->stream));
-    for (size_t j = 0; j < h; ++j)
-        for (size_t i = 0; i < w; ++i) {
-            double vr, vi;
-            if (es == 8) {
-                vr = ((const double *)tr.get())[j * w + i];
-                vi = ((const double *)ti.get())[j * w + i];
-            } else {
-                vr = ((const float *)tr.get())[j * w + i];
-                vi = ((const float *)ti.get())[j * w + i];
-            }
-            if (scale) { vr /= div; vi /= div; }   // src/cpukernel.cpp:559-560
-            re[j * stride + i] = vr;
-            im[j * stride + i] = vi;
-        }
-    return TSMI_OK;
+    return download_state(c, stride, x, y, w, h, re, im);
+}
+
+int tsmi_get_state_complex(tsmi_ctx *c, double *psi) {
+    if (!c || !psi) return fail(TSMI_E_INVALID, "tsmi_get_state_complex: null argument");
+    if (!c->has_state) return fail(TSMI_E_INVALID, "tsmi_get_state_complex: no state");
+    return download_state(c, (size_t)c->W, 0, 0, (size_t)c->W, (size_t)c->H, psi, nullptr);
 }
 
 int tsmi_synchronize(tsmi_ctx *c) {

@@ -467,6 +467,12 @@ int tsmi_pair_set_state(tsmi_pair *p, int32_t which, const double *re, const dou
     return tsmi_set_state(c, re, im);
 }
 
+int tsmi_pair_set_state_complex(tsmi_pair *p, int32_t which, const double *psi) {
+    tsmi_ctx *c = component(p, which, "tsmi_pair_set_state_complex");
+    if (!c) return TSMI_E_INVALID;
+    return tsmi_set_state_complex(c, psi);
+}
+
 int tsmi_pair_set_exp_potential(tsmi_pair *p, int32_t which, const double *e_re, const double *e_im) {
     tsmi_ctx *c = component(p, which, "tsmi_pair_set_exp_potential");
     if (!c) return TSMI_E_INVALID;
@@ -524,6 +530,14 @@ int tsmi_pair_get_state(tsmi_pair *p, int32_t which, double *re, double *im) {
     if (!re || !im) return set_error(TSMI_E_INVALID, "tsmi_pair_get_state: null argument");
     if (int st = settle(p)) return st;
     return tsmi_get_sample(c, (size_t)c->W, 0, 0, (size_t)c->W, (size_t)c->H, re, im);
+}
+
+int tsmi_pair_get_state_complex(tsmi_pair *p, int32_t which, double *psi) {
+    tsmi_ctx *c = component(p, which, "tsmi_pair_get_state_complex");
+    if (!c) return TSMI_E_INVALID;
+    if (!psi) return set_error(TSMI_E_INVALID, "tsmi_pair_get_state_complex: null argument");
+    if (int st = settle(p)) return st;
+    return tsmi_get_state_complex(c, psi);
 }
 
 int tsmi_pair_energy(tsmi_pair *p, double out[12]) {

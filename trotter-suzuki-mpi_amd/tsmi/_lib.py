@@ -17,7 +17,9 @@ TSMI_OK = 0
 
 # Every symbol include/tsmi_hip.h declares (checked by the test suite).
 EXPORTS = (
-    "tsmi_create", "tsmi_destroy", "tsmi_set_stream", "tsmi_set_state", "tsmi_set_state_device",
+    "tsmi_create", "tsmi_destroy", "tsmi_set_stream", "tsmi_set_state", "tsmi_set_state_complex", "tsmi_get_state_complex",
+    "tsmi_set_state_device", "tsmi_batch_set_state_complex", "tsmi_batch_get_state_complex",
+    "tsmi_pair_set_state_complex", "tsmi_pair_get_state_complex",
     "tsmi_set_exp_potential", "tsmi_set_exp_potential_device", "tsmi_set_potential",
     "tsmi_set_potential_device", "tsmi_set_potential_exp_device", "tsmi_evolve", "tsmi_run_steps", "tsmi_step", "tsmi_evolve_checkpointed", "tsmi_adjoint",
     "tsmi_adjoint_device", "tsmi_batch_create", "tsmi_batch_destroy", "tsmi_batch_set_state",
@@ -80,6 +82,10 @@ def load():
     L.tsmi_destroy.restype = None
     L.tsmi_set_stream.argtypes = [C.c_void_p, C.c_void_p]
     L.tsmi_set_state.argtypes = [C.c_void_p, _dp, _dp]
+    L.tsmi_set_state_complex.argtypes = L.tsmi_get_state_complex.argtypes = [C.c_void_p, _dp]
+    for name in ("tsmi_batch", "tsmi_pair"):
+        for call in ("set", "get"):
+            getattr(L, f"{name}_{call}_state_complex").argtypes = [C.c_void_p, C.c_int32, _dp]
     L.tsmi_set_exp_potential.argtypes = [C.c_void_p, _dp, _dp]
     L.tsmi_set_potential.argtypes = [C.c_void_p, _dp]
     L.tsmi_set_state_device.argtypes = [C.c_void_p, C.c_void_p, C.c_void_p]
@@ -140,6 +146,19 @@ def check(status: int, what: str = "") -> None:
     if status != TSMI_OK:
         msg = load().tsmi_last_error().decode(errors="replace")
         raise TsmiError(f"{what}: {msg} (status {status})" if what else msg)
+
+
+def zptr(a: np.ndarray):
+    """The pointer of a complex array: interleaved doubles."""
+    assert a.dtype == np.complex128 and a.flags.c_contiguous
+    return a.ctypes.data_as(_dp)
+
+
+def complex_tile(a, shape, what: str = "") -> np.ndarray:
+    a = np.ascontiguousarray(a, dtype=np.complex128)
+    if a.shape != shape:
+        raise ValueError(f"{what}expected {shape}, got {a.shape}")
+    return a
 
 
 def dptr(a: np.ndarray):

@@ -67,8 +67,8 @@ class HipBatch:
         return a
 
     def set_state(self, i: int, psi: np.ndarray) -> None:
-        re, im = self._plane(i, psi.real), self._plane(i, psi.imag)
-        _lib.check(self._L.tsmi_batch_set_state(self._h, i, _lib.dptr(re), _lib.dptr(im)), "tsmi_batch_set_state")
+        z = _lib.complex_tile(psi, self._shape(i), f"lattice {i}: ")
+        _lib.check(self._L.tsmi_batch_set_state_complex(self._h, i, _lib.zptr(z)), "tsmi_batch_set_state")
 
     def set_exp_potential(self, i: int, e_re, e_im) -> None:
         re = self._plane(i, e_re)
@@ -83,11 +83,9 @@ class HipBatch:
         _lib.check(self._L.tsmi_batch_synchronize(self._h), "tsmi_batch_synchronize")
 
     def state(self, i: int) -> np.ndarray:
-        H, W = self._shape(i)
-        re = np.zeros((H, W))
-        im = np.zeros((H, W))
-        _lib.check(self._L.tsmi_batch_get_state(self._h, i, _lib.dptr(re), _lib.dptr(im)), "tsmi_batch_get_state")
-        return re + 1j * im
+        z = np.empty(self._shape(i), dtype=np.complex128)
+        _lib.check(self._L.tsmi_batch_get_state_complex(self._h, i, _lib.zptr(z)), "tsmi_batch_get_state")
+        return z
 
     def tune(self, steps: int = 3) -> float:
         """Autotunes the segment heights; returns the tuned ms per batch step."""

@@ -70,8 +70,8 @@ class HipKernel:
         return a
 
     def set_state(self, psi: np.ndarray) -> None:
-        re, im = self._plane(psi.real), self._plane(psi.imag)
-        _lib.check(self._L.tsmi_set_state(self._h, _lib.dptr(re), _lib.dptr(im)), "tsmi_set_state")
+        z = _lib.complex_tile(psi, (self.lattice.H, self.lattice.W), "tile: ")
+        _lib.check(self._L.tsmi_set_state_complex(self._h, _lib.zptr(z)), "tsmi_set_state")
 
     def set_exp_potential(self, e_re: np.ndarray, e_im: np.ndarray | None) -> None:
         re = self._plane(e_re)
@@ -154,6 +154,10 @@ class HipKernel:
         lat = self.lattice
         w = lat.W - x if width is None else width
         h = lat.H - y if height is None else height
+        if (x, y, w, h) == (0, 0, lat.W, lat.H):
+            z = np.empty((h, w), dtype=np.complex128)
+            _lib.check(self._L.tsmi_get_state_complex(self._h, _lib.zptr(z)), "tsmi_get_sample")
+            return z
         re = np.zeros((h, w))
         im = np.zeros((h, w))
         _lib.check(self._L.tsmi_get_sample(self._h, w, x, y, w, h, _lib.dptr(re), _lib.dptr(im)), "tsmi_get_sample")

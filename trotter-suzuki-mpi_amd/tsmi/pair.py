@@ -65,7 +65,8 @@ class HipPair:
         _lib.check(getattr(self._L, name)(self._h, int(which), *[_lib.dptr(p) for p in planes]), name)
 
     def set_state(self, which: int, psi: np.ndarray) -> None:
-        self._call("tsmi_pair_set_state", which, self._plane(psi.real), self._plane(psi.imag))
+        z = _lib.complex_tile(psi, (self.pw.lattice.H, self.pw.lattice.W))
+        _lib.check(self._L.tsmi_pair_set_state_complex(self._h, int(which), _lib.zptr(z)), "tsmi_pair_set_state")
 
     def evolve(self, n_steps: int, initial_half: bool = True) -> None:
         _lib.check(self._L.tsmi_pair_evolve(self._h, int(n_steps), int(initial_half)), "tsmi_pair_evolve")
@@ -74,12 +75,9 @@ class HipPair:
         _lib.check(self._L.tsmi_pair_synchronize(self._h), "tsmi_pair_synchronize")
 
     def state(self, which: int) -> np.ndarray:
-        lat = self.pw.lattice
-        re = np.zeros((lat.H, lat.W))
-        im = np.zeros((lat.H, lat.W))
-        _lib.check(self._L.tsmi_pair_get_state(self._h, int(which), _lib.dptr(re), _lib.dptr(im)),
-                   "tsmi_pair_get_state")
-        return re + 1j * im
+        z = np.empty((self.pw.lattice.H, self.pw.lattice.W), dtype=np.complex128)
+        _lib.check(self._L.tsmi_pair_get_state_complex(self._h, int(which), _lib.zptr(z)), "tsmi_pair_get_state")
+        return z
 
     def energy(self) -> np.ndarray:
         out = np.zeros(12)
