@@ -463,6 +463,7 @@ __device__ __forceinline__ void sincos_row(const T (&x)[VEC], T (&s)[VEC], T (&c
                 T r = x[k];
                 if (__builtin_expect(far, 0)) r = wrap_far(r);
                 sincos_near(r, &s[k], &c[k]);
+                if (k & 1) __builtin_amdgcn_sched_barrier(0);   // two at a time: registers
             }
         }
     } else {
@@ -472,7 +473,10 @@ __device__ __forceinline__ void sincos_row(const T (&x)[VEC], T (&s)[VEC], T (&c
         for (int k = 0; k < VEC; ++k) small(x[k], &s[k], &c[k]);
         if (__builtin_expect(!wave_all_le(m, T(0.015625)), 0)) {
 #pragma unroll
-            for (int k = 0; k < VEC; ++k) sincos_t(x[k], &s[k], &c[k]);
+            for (int k = 0; k < VEC; ++k) {
+                sincos_t(x[k], &s[k], &c[k]);
+                if (NEAR && (k & 1)) __builtin_amdgcn_sched_barrier(0);
+            }
         }
     }
 }

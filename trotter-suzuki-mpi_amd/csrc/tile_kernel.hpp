@@ -65,7 +65,7 @@ struct TileXch {
 
 // The potential pass of two rows: one wave-uniform test and straight-line code
 // for the four values per lane.
-template <typename T, bool LHY>
+template <typename T, bool LHY, bool IMAG = false>
 __device__ __forceinline__ void tile_ppass(Row<T, 2> &a, Row<T, 2> &b, const T (&pa)[2], const T (&pb)[2], T c, T cl,
                                            double mag) {
     T ang[4], sn[4], cs[4];
@@ -77,6 +77,18 @@ __device__ __forceinline__ void tile_ppass(Row<T, 2> &a, Row<T, 2> &b, const T (
     ang[1] = angle(a, 1, pa[1]);
     ang[2] = angle(b, 0, pb[0]);
     ang[3] = angle(b, 1, pb[1]);
+    if constexpr (IMAG) {
+        T f[4];
+        expneg_row<T, 4>(ang, f);
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+            a.re[k] *= f[k];
+            a.im[k] *= f[k];
+            b.re[k] *= f[2 + k];
+            b.im[k] *= f[2 + k];
+        }
+        return;
+    }
     sincos_row<T, 4, true>(ang, sn, cs);
     const T ca[2] = {cs[0], cs[1]}, sa[2] = {sn[0], sn[1]}, cb[2] = {cs[2], cs[3]}, sb[2] = {sn[2], sn[3]};
     rotate_row_ph<T, 2>(a, ca, sa, mag);

@@ -19,8 +19,9 @@
 #include <vector>
 
 #include "common.hpp"
-#include "context.hpp"
+#include "pair_context.hpp"
 #include "pair_kernel.hpp"
+#include "pair_tile_kernel.hpp"
 #include "tsmi_hip.h"
 
 using namespace tsmi;
@@ -40,43 +41,7 @@ constexpr int kRabiBlocksMax = 1024;
 
 }  // namespace
 
-struct tsmi_pair {
-    tsmi_ctx *c[2] = {nullptr, nullptr};
-    int esz = 0, vec = 0;
-    bool imag = false;
-    double dt = 0, c_ab = 0, omega_r = 0, omega_i = 0, g_ab = 0, tot_norm = 0;
-    int W = 0, H = 0, pitch = 0;
-    int n_strips = 0, seg_rows = 0, n_segs = 0, n_waves = 0, rabi_blocks = 0;
-    // two steps per pass (pair2_kernel) over the whole allocation, Wd x Hd
-    bool fused = false, halo8 = false;
-    int Wd = 0, Hd = 0, n_strips2 = 0, seg_rows2 = 0, n_segs2 = 0, n_waves2 = 0;
-    int ix0 = 0, ix1 = 0, iy0 = 0, iy1 = 0;
-    // device scalars: divisor pairs [2][2] (a pending pair is read while the
-    // next one is written), norm targets [2]
-    double *dv = nullptr;
-    double *partials = nullptr;
-    unsigned *counter = nullptr;
-    int slot = 0;
-    bool pending = false;
-};
-
-namespace {
-
-void free_pair(tsmi_pair *p) {
-    if (p->c[1]) tsmi_destroy(p->c[1]);   // runs on c[0]'s stream: released first
-    if (p->c[0]) tsmi_destroy(p->c[0]);
-    void *ptrs[] = {p->dv, p->partials, p->counter};
-    for (void *q : ptrs)
-        if (q) (void)hipFree(q);
-}
-
-bool same_lattice(const tsmi_desc &a, const tsmi_desc &b) {
-    return a.dim_x == b.dim_x && a.dim_y == b.dim_y && a.periodic_x == b.periodic_x &&
-           a.periodic_y == b.periodic_y && a.halo_x == b.halo_x && a.halo_y == b.halo_y &&
-           a.imag_time == b.imag_time && a.precision == b.precision && a.delta_t == b.delta_t &&
-           a.delta_x == b.delta_x && a.delta_y == b.delta_y && a.length_x == b.length_x &&
-           a.length_y == b.length_y && a.tile_rows == b.tile_rows;
-}
+namespace tsmi {
 
 // The rotation constants of CPUBlock::rabi_coupling(var, dt) (src/cpukernel.cpp:581-608).
 void rabi_coefs(const tsmi_pair *p, double var, double *cc, double *cs_r, double *cs_i) {
@@ -94,10 +59,37 @@ void rabi_coefs(const tsmi_pair *p, double var, double *cc, double *cs_r, double
     }
 }
 
-bool rabi_on(const tsmi_pair *p) { return p->omega_r != 0.0 || p->omega_i != 0.0; }
+// the periodic exchange of both components' current tiles (on the 8-wide halo
+// layout the full wrap, whose inner 4 cells are the reference's exchange)
+int exchange_both(tsmi_pair *p) {
+    for (int c = 0; c < 2; ++c) {
+        tsmi_ctx *x = p->c[c];
+        if (int st = ctx_exchange(x, x->psi_base[x->cur][0], x->psi_base[x->cur][1])) return st;
+    }
+    return TSMI_OK;
+}
+
+}  // namespace tsmi
+
+namespace {
+
+void free_pair(tsmi_pair *p) {
+    if (p->c[1]) tsmi_destroy(p->c[1]);   // runs on c[0]'s stream: released first
+    if (p->c[0]) tsmi_destroy(p->c[0]);
+    void *ptrs[] = {p->dv, p->partials, p->counter, p->tile_part, p->tile_n};
+    for (void *q : ptrs)
+        if (q) (void)hipFree(q);
+}
+
+bool same_lattice(const tsmi_desc &a, const tsmi_desc &b) {
+    return a.dim_x == b.dim_x && a.dim_y == b.dim_y && a.periodic_x == b.periodic_x &&
+           a.periodic_y == b.periodic_y && a.halo_x == b.halo_x && a.halo_y == b.halo_y &&
+           a.imag_time == b.imag_time && a.precision == b.precision && a.delta_t == b.delta_t &&
+           a.delta_x == b.delta_x && a.delta_y == b.delta_y && a.length_x == b.length_x &&
+           a.length_y == b.length_y && a.tile_rows == b.tile_rows;
+}
 
 double *div_pair(tsmi_pair *p, int s) { return p->dv + 2 * s; }
-double *norms(tsmi_pair *p) { return p->dv + 4; }
 
 // One step of both components; in real time the Rabi rotation by var leaves the
 // pipelines with the rows when rotate.
@@ -224,16 +216,6 @@ int pair_step(tsmi_pair *p, double var, bool rotate) {
     const bool ph = p->c[0]->ph_mode && p->c[1]->ph_mode;
     if (p->esz == 4) return ph ? pair_step_form<float, true>(p, var, rotate) : pair_step_form<float, false>(p, var, rotate);
     return ph ? pair_step_form<double, true>(p, var, rotate) : pair_step_form<double, false>(p, var, rotate);
-}
-
-// the periodic exchange of both components' current tiles (on the 8-wide halo
-// layout the full wrap, whose inner 4 cells are the reference's exchange)
-int exchange_both(tsmi_pair *p) {
-    for (int c = 0; c < 2; ++c) {
-        tsmi_ctx *x = p->c[c];
-        if (int st = ctx_exchange(x, x->psi_base[x->cur][0], x->psi_base[x->cur][1])) return st;
-    }
-    return TSMI_OK;
 }
 
 // Two real-time FP32 steps of both components in one pass over the allocations;
@@ -438,12 +420,19 @@ int tsmi_pair_create(const tsmi_pair_desc *pd, tsmi_pair **out) {
         p->n_waves2 = p->n_strips2 * p->n_segs2;
     }
     // norm targets at kernel construction (src/solver.cpp:153-159, src/cpukernel.cpp:321-325)
-    const double nt[6] = {1.0, 1.0, 1.0, 1.0, pd->a.norm_target, pd->b.norm_target};
+    const double nt[8] = {1.0, 1.0, 1.0, 1.0, pd->a.norm_target, pd->b.norm_target, 0.0, 0.0};
     p->tot_norm = nt[4] + nt[5];
     const size_t np = 2 * (size_t)std::max(p->n_waves, p->rabi_blocks);
     hipError_t e = hipMalloc((void **)&p->dv, sizeof(nt));
     if (e == hipSuccess) e = hipMalloc((void **)&p->partials, np * sizeof(double));
     if (e == hipSuccess) e = hipMalloc((void **)&p->counter, 64);
+    p->tiles = pair_tiles_fit(p, d.tile_rows, d.sweeps);
+    if (p->tiles && p->imag) {
+        p->part_cap = pair_tile_blocks(p);
+        if (e == hipSuccess)
+            e = hipMalloc((void **)&p->tile_part, 2 * (size_t)kPairSums * (size_t)p->part_cap * sizeof(double));
+        if (e == hipSuccess) e = hipMalloc((void **)&p->tile_n, 2 * sizeof(int));
+    }
     if (e != hipSuccess) return bail(set_error(TSMI_E_OOM, std::string("tsmi_pair_create: ") + hipGetErrorString(e)));
     hipStream_t s = c0->stream;
     e = hipMemcpyAsync(p->dv, nt, sizeof(nt), hipMemcpyHostToDevice, s);
@@ -492,7 +481,11 @@ int tsmi_pair_evolve(tsmi_pair *p, int32_t n_steps, int32_t initial_half) {
     int st = TSMI_OK;
     // src/solver.cpp:173-177
     if (initial_half && rabi) st = rabi_pass(p, 0.5, true, false);
-    // two steps per pass where both E tables have the phase form
+    // tile passes or two steps per pass where both E tables have the phase form
+    if (!st && p->tiles && p->c[0]->ph_mode && p->c[1]->ph_mode) {
+        st = settle(p);
+        return st ? st : pair_tile_evolve(p, n_steps, rabi);
+    }
     if (p->fused && p->c[0]->ph_mode && p->c[1]->ph_mode) return st ? st : evolve_fused(p, n_steps, rabi);
     for (int i = 0; i < n_steps && !st; ++i) {
         const bool last = i == n_steps - 1;

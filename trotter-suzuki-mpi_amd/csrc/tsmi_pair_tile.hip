@@ -1,0 +1,256 @@
+// tsmi_pair_tile.hip -- planning and launching the two-component tile passes
+// (pair_tile_kernel.hpp).
+#include <hip/hip_runtime.h>
+
+#include <algorithm>
+#include <cmath>
+#include <cstring>
+#include <string>
+
+#include "common.hpp"
+#include "pair_context.hpp"
+#include "pair_tile_kernel.hpp"
+#include "tsmi_hip.h"
+
+using namespace tsmi;
+
+namespace {
+
+// Rows per wave and waves of the compiled instances.
+struct Shape { int r, nw; };
+constexpr Shape kShapes32[] = {{4, 8}, {8, 8}}, kShapes64[] = {{4, 8}, {4, 4}};
+
+struct Plan {
+    int r = 0, nw = 0, cols = 0, rows = 0, strips = 0, segs = 0;
+    double us = 1e30;    // modelled time per step
+};
+
+// The tile shape of a pass of `steps` steps: the one with the least modelled time.
+// A launch costs 4.5 us and its bytes; a step costs each SIMD its rows (of both
+// components; 0.27 us a row in FP32, 0.53 in FP64 with several waves per SIMD,
+// more for a wave alone) and 0.5 us of exchanges.  Measured around it, periodic,
+// us per step: 256^2 FP32 4 rows x 8 waves 7.9, 5.6, 4.9 for 1, 2, 3 steps, 8 x 8
+// 12.6, 9.3, 8.1; 1024^2 FP32 4 x 8 13.9, 13.0, 19.2, 8 x 8 15.8, 12.2, 17.1 (3
+// steps: more than one workgroup per compute unit); 512^2 FP64 4 x 8 10.9, 8.5, 12.7.
+Plan plan(int W, int H, int esz, int steps, bool wrap) {
+    Plan best;
+    const int a = kApron * steps;
+    const Shape *sh = esz == 4 ? kShapes32 : kShapes64;
+    const double c_row = esz == 4 ? 0.27 : 0.53, x = 0.5;
+    const double t0 = 4.5 + (double)W * H * 10 * esz / 6.5e6;
+    for (int i = 0; i < 2; ++i) {
+        Plan p;
+        p.r = sh[i].r;
+        p.nw = sh[i].nw;
+        p.cols = kTileCols - 2 * a;
+        p.rows = p.nw * p.r - 2 * a;
+        if (p.cols < 2 || p.rows < 2) continue;
+        p.strips = (W + p.cols - 1) / p.cols;
+        p.segs = (H + p.rows - 1) / p.rows;
+        const double n = p.strips * p.segs / 256.0;              // workgroups per compute unit
+        const double per_cu = n < 6 ? std::ceil(n) : n + 0.5;    // ... on the busiest one
+        const double most = wrap && esz == 4 && p.r == 4 ? 4.0 : 2.0;
+        const double waves = std::min(per_cu * p.nw / 4.0, most);   // waves per SIMD
+        p.us = t0 / steps + per_cu * p.nw * p.r / 4.0 * c_row * (1 + 0.6 / waves) + x;
+        if (p.us < best.us) best = p;
+    }
+    return best;
+}
+
+int best_steps(int W, int H, int esz, int most, bool wrap) {
+    int k = 1;
+    double us = 1e30;
+    for (int s = 1; s <= std::min(most, 6); ++s) {
+        const Plan p = plan(W, H, esz, s, wrap);
+        if (p.us < us) {
+            us = p.us;
+            k = s;
+        }
+    }
+    return k;
+}
+
+template <typename T, bool IMAG, int R, int NW, bool WRAP>
+int launch_kernel(tsmi_pair *p, const PairTileParams<T> &q, const Plan &g) {
+    // one scaled form for both components on both axes, or both factors
+    const int mode = p->c[0]->mode == p->c[1]->mode ? p->c[0]->mode : -1;
+    const dim3 grid(g.strips * g.segs), block(NW * kWave);
+    hipStream_t s = p->c[0]->stream;
+    // FP64 tiles of 8 waves with an edge: the general form for all of them, as both
+    // forms in one kernel spill
+    if constexpr (!WRAP && sizeof(T) == 8 && NW == 8) {
+        hipLaunchKernelGGL((pair_tile_kernel<T, IMAG, -1, R, NW, WRAP>), grid, block, 0, s, q);
+    } else if constexpr (IMAG) {   // form A always
+        hipLaunchKernelGGL((pair_tile_kernel<T, true, 0, R, NW, WRAP>), grid, block, 0, s, q);
+    } else {
+        if (mode == 0) hipLaunchKernelGGL((pair_tile_kernel<T, false, 0, R, NW, WRAP>), grid, block, 0, s, q);
+        else if (mode == 1) hipLaunchKernelGGL((pair_tile_kernel<T, false, 1, R, NW, WRAP>), grid, block, 0, s, q);
+        else hipLaunchKernelGGL((pair_tile_kernel<T, false, -1, R, NW, WRAP>), grid, block, 0, s, q);
+    }
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return set_error(TSMI_E_HIP, std::string("pair_tile_kernel: ") + hipGetErrorString(e));
+    return TSMI_OK;
+}
+
+template <typename T, bool IMAG, int R, int NW>
+int launch(tsmi_pair *p, const PairTileParams<T> &q, const Plan &g) {
+    return q.nx ? launch_kernel<T, IMAG, R, NW, true>(p, q, g) : launch_kernel<T, IMAG, R, NW, false>(p, q, g);
+}
+
+template <typename T, bool IMAG>
+int launch_shape(tsmi_pair *p, const PairTileParams<T> &q, const Plan &g) {
+    constexpr const Shape *sh = sizeof(T) == 4 ? kShapes32 : kShapes64;
+    if (g.r == sh[0].r && g.nw == sh[0].nw) return launch<T, IMAG, sh[0].r, sh[0].nw>(p, q, g);
+    return launch<T, IMAG, sh[1].r, sh[1].nw>(p, q, g);
+}
+
+// What is pending after an imaginary-time step in slot p->slot's partial sums,
+// whose rotation is by var.
+PairNorm pending(tsmi_pair *p, double var, bool rabi) {
+    PairNorm q;
+    std::memset(&q, 0, sizeof(q));
+    q.part = p->tile_part + (size_t)p->slot * kPairSums * (size_t)p->part_cap;
+    q.n = p->tile_n + p->slot;
+    q.cap = p->part_cap;
+    q.norm_in = norms(p);
+    q.norm_out = p->dv + 4 + 2 * (1 - p->norm_slot);
+    rabi_coefs(p, var, &q.cc, &q.cs_r, &q.cs_i);
+    q.rabi = rabi ? 1 : 0;
+    q.dxdy = p->c[0]->d.delta_x * p->c[0]->d.delta_y;
+    q.tot_norm = p->tot_norm;
+    return q;
+}
+
+// `steps` steps; the rotation after the last of them is by var (1 after the
+// others).  first: nothing pending from a step before (imaginary time).
+template <typename T>
+int pass(tsmi_pair *p, int steps, bool wrap, double var, bool rabi, bool first) {
+    PairTileParams<T> q;
+    std::memset(&q, 0, sizeof(q));
+    const int cur = p->c[0]->cur, nb = 1 - cur;
+    for (int i = 0; i < 2; ++i) {
+        tsmi_ctx *c = p->c[i];
+        q.in_re[i] = (const T *)c->psi_re[cur];
+        q.in_im[i] = (const T *)c->psi_im[cur];
+        q.out_re[i] = (T *)c->psi_re[nb];
+        q.out_im[i] = (T *)c->psi_im[nb];
+        q.ph[i] = (const T *)c->ph;
+        q.mH[i] = (T)c->mH; q.tH[i] = (T)c->tH; q.mV[i] = (T)c->mV; q.tV[i] = (T)c->tV;
+        q.unH[i] = (T)c->unH; q.unV[i] = (T)c->unV;
+        q.c_self[i] = (T)c->c_nl_s;
+        q.mag[i] = p->imag ? 1.0 : c->corr_abs;
+    }
+    q.c_ab = (T)p->c_ab;
+    q.W = p->W; q.H = p->H; q.pitch = p->pitch;
+    q.nx = wrap ? p->c[0]->d.dim_x : 0;
+    q.ny = wrap ? p->c[0]->d.dim_y : 0;
+    q.steps = steps;
+    const Plan g = plan(p->W, p->H, p->esz, steps, wrap);
+    if (g.r == 0) return set_error(TSMI_E_INVALID, "pair tile pass: no tile for this many steps");
+    q.n_strips = g.strips; q.cols = g.cols; q.rows = g.rows;
+    q.ix0 = p->ix0; q.ix1 = p->ix1; q.iy0 = p->iy0; q.iy1 = p->iy1;
+    q.rabi = rabi ? 1 : 0;
+    int st;
+    if (!p->imag) {
+        rabi_coefs(p, 1.0, &q.cc, &q.cs_r, &q.cs_i);
+        rabi_coefs(p, var, &q.cc2, &q.cs_r2, &q.cs_i2);
+        st = launch_shape<T, false>(p, q, g);
+    } else {
+        if (!first) {
+            q.pend = pending(p, 1.0, rabi);
+            p->norm_slot = 1 - p->norm_slot;
+        }
+        double cc;
+        rabi_coefs(p, var, &cc, &q.s_r, &q.s_i);
+        p->slot = 1 - p->slot;
+        q.part_out = p->tile_part + (size_t)p->slot * kPairSums * (size_t)p->part_cap;
+        q.n_out = p->tile_n + p->slot;
+        q.cap = p->part_cap;
+        st = launch_shape<T, true>(p, q, g);
+    }
+    if (!st) p->c[0]->cur = p->c[1]->cur = nb;
+    return st;
+}
+
+int tile_pass(tsmi_pair *p, int steps, bool wrap, double var, bool rabi, bool first) {
+    return p->esz == 4 ? pass<float>(p, steps, wrap, var, rabi, first) : pass<double>(p, steps, wrap, var, rabi, first);
+}
+
+// The renormalisation after the last step.
+int finish(tsmi_pair *p, double var, bool rabi) {
+    const PairNorm q = pending(p, var, rabi);
+    const int cur = p->c[0]->cur;
+    const int blocks = (int)std::min<long>(256, ((long)p->W * p->H + 1023) / 1024);
+    hipStream_t s = p->c[0]->stream;
+    tsmi_ctx *a = p->c[0], *b = p->c[1];
+    if (p->esz == 4)
+        hipLaunchKernelGGL((pair_finish_kernel<float>), dim3(blocks), dim3(256), 0, s, (float *)a->psi_re[cur],
+                           (float *)a->psi_im[cur], (float *)b->psi_re[cur], (float *)b->psi_im[cur], p->W, p->H,
+                           p->pitch, q);
+    else
+        hipLaunchKernelGGL((pair_finish_kernel<double>), dim3(blocks), dim3(256), 0, s, (double *)a->psi_re[cur],
+                           (double *)a->psi_im[cur], (double *)b->psi_re[cur], (double *)b->psi_im[cur], p->W, p->H,
+                           p->pitch, q);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return set_error(TSMI_E_HIP, std::string("pair_finish_kernel: ") + hipGetErrorString(e));
+    p->norm_slot = 1 - p->norm_slot;
+    return TSMI_OK;
+}
+
+}  // namespace
+
+namespace tsmi {
+
+int pair_tile_blocks(const tsmi_pair *p) {
+    const Plan a = plan(p->W, p->H, p->esz, 1, false), b = plan(p->W, p->H, p->esz, 1, true);
+    return std::max(a.strips * a.segs, b.strips * b.segs);
+}
+
+// No segment height or steps per pass asked for, offsets within 31 bits, and a
+// lattice small enough that the row latency (real time) or the ticketed
+// reductions (imaginary time) bound the streaming passes; us per step, streamed
+// against tiles, doubly periodic / closed: real FP32 100^2 36 / 33 -> 5.5 / 5.8,
+// 512^2 37 / 33 -> 7.8 / 8.0, 1240^2 38 / 35 -> 22 / 29; FP64 100^2 61 / 55 -> 7.7 /
+// 8.6, 1240^2 64 / 59 -> 40 / 43; imaginary FP32 100^2 63 / 58 -> 11 / 12, 1240^2
+// 263 / 257 -> 26 / 33, FP64 1240^2 279 / 275 -> 54 / 54.
+bool pair_tiles_fit(const tsmi_pair *p, int tile_rows, int sweeps) {
+    const long most = p->imag ? 5L << 20 : 3L << 19;
+    return tile_rows == 0 && sweeps == 0 && p->H > 1 && (long)p->W * p->H <= most &&
+           (long)p->pitch * p->c[0]->Hd * p->esz < (1L << 31);
+}
+
+int pair_tile_evolve(tsmi_pair *p, int n, bool rabi) {
+    if (n <= 0) return TSMI_OK;
+    const tsmi_desc &d = p->c[0]->d;
+    const bool closed = !d.periodic_x && !d.periodic_y;
+    const bool wrap = d.periodic_x && d.periodic_y && d.dim_x % 2 == 0 && d.dim_y % 2 == 0 && n >= 3;
+    const int most = p->imag || !(closed || wrap) ? 1 : n;
+    int i = 0, st = TSMI_OK;
+    // n steps from step i on; the call's last rotation is by 1/2 (src/solver.cpp:222-225)
+    auto passes = [&](int m, bool w) {
+        const int k = best_steps(p->W, p->H, p->esz, std::min(m, most), w), q = (m + k - 1) / k;
+        for (int j = 0; j < q && !st; ++j) {
+            const int s = m / q + (j < m % q ? 1 : 0);
+            i += s;
+            st = tile_pass(p, s, w, i == n ? 0.5 : 1.0, rabi, i == s);
+        }
+    };
+    if (closed) {
+        passes(n, false);
+    } else if (wrap) {
+        passes(1, false);
+        passes(n - 2, true);
+        if (!st) passes(1, false);
+    } else {
+        // mixed axes; odd periodic extents, where the pair pattern of a halo cell
+        // differs from that of the cell it mirrors
+        for (int j = 0; j < n && !st; ++j) {
+            passes(1, false);
+            if (!st && j != n - 1) st = exchange_both(p);
+        }
+    }
+    if (!st && p->imag) st = finish(p, 0.5, rabi);
+    return st;
+}
+
+}  // namespace tsmi
