@@ -179,7 +179,8 @@ int tsmi_adjoint_device(tsmi_ctx *ctx, const double *g_re, const double *g_im, d
  * class (kind and tile shape) at a time; keeps the fastest, restores the states
  * and reports the tuned time per step.  tsmi_batch_info: out[0..2] W, H, pitch
  * of lattice i's tile, out[3..5] strips, segments and rows per segment of its
- * dominant pass, out[6] steps per pass (1 or 2).
+ * dominant streaming pass, out[6] that pass's steps (1 or 2); small batches run
+ * as register tiles instead, which have nothing to tune.
  * set_state / set_exp_potential / get_state take W*H FP64 host arrays of
  * lattice i (the _complex forms one array of complex doubles); get_state syncs. */
 typedef struct tsmi_batch tsmi_batch;

@@ -93,5 +93,8 @@ int ctx_time_mark(tsmi_ctx *c, int kind, int which);
 bool tile_runs(const tsmi_ctx *c);
 bool tile_wraps(const tsmi_ctx *c);
 int tile_passes(tsmi_ctx *c, int n, bool wrap);
+// n steps, each starting with the halo exchange that has not been run yet (the
+// state's halo cells are read from the cells they mirror).
+int tile_seam_steps(tsmi_ctx *c, int n);
 
 }  // namespace tsmi

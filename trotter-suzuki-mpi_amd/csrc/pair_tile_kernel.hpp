@@ -241,7 +241,7 @@ __device__ __forceinline__ void pair_tile_steps(const PairTileParams<T> &p, Row<
     auto ppass = [&](int r0, int r1) {
 #pragma unroll
         for (int c = 0; c < 2; ++c) {
-            tile_ppass<T, false, IMAG>(s[c][r0], s[c][r1], base[c][r0], base[c][r1], p.c_self[c], T(0), p.mag[c]);
+            tile_ppass<T, false, IMAG, 2>(s[c][r0], s[c][r1], base[c][r0], base[c][r1], p.c_self[c], T(0), p.mag[c]);
         }
         __builtin_amdgcn_sched_barrier(0);   // one group of rows at a time: fewer registers at once
     };

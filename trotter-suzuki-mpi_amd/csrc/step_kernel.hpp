@@ -431,8 +431,9 @@ __device__ __forceinline__ bool wave_all_le(double v, double thr) {
 // to within the format: truncation below 2e-10 relative in FP32 (sin to x^3,
 // cos to x^4, exp to x^4) and below 1e-19 in FP64 (sin to x^7, cos to x^8,
 // exp to x^8).  Otherwise the general routines run.
-// NEAR: the FP64 general routine is sincos_near (see there).
-template <typename T, int VEC, bool NEAR = false>
+// NEAR: the FP64 general routine is sincos_near (see there); 2: in either
+// precision two general values at a time, for kernels short of registers.
+template <typename T, int VEC, int NEAR = 0>
 __device__ __forceinline__ void sincos_row(const T (&x)[VEC], T (&s)[VEC], T (&c)[VEC]) {
     T m = fabs(x[0]);
 #pragma unroll
@@ -452,7 +453,7 @@ __device__ __forceinline__ void sincos_row(const T (&x)[VEC], T (&s)[VEC], T (&c
             *c = fma(r2, pc, 1.0);
         }
     };
-    if constexpr (NEAR && sizeof(T) == 8) {
+    if constexpr (NEAR != 0 && sizeof(T) == 8) {
         if (wave_all_le(m, T(0.015625))) {
 #pragma unroll
             for (int k = 0; k < VEC; ++k) small(x[k], &s[k], &c[k]);
@@ -463,7 +464,7 @@ __device__ __forceinline__ void sincos_row(const T (&x)[VEC], T (&s)[VEC], T (&c
                 T r = x[k];
                 if (__builtin_expect(far, 0)) r = wrap_far(r);
                 sincos_near(r, &s[k], &c[k]);
-                if (k & 1) __builtin_amdgcn_sched_barrier(0);   // two at a time: registers
+                if (NEAR == 2 && (k & 1)) __builtin_amdgcn_sched_barrier(0);
             }
         }
     } else {
@@ -475,7 +476,7 @@ __device__ __forceinline__ void sincos_row(const T (&x)[VEC], T (&s)[VEC], T (&c
 #pragma unroll
             for (int k = 0; k < VEC; ++k) {
                 sincos_t(x[k], &s[k], &c[k]);
-                if (NEAR && (k & 1)) __builtin_amdgcn_sched_barrier(0);
+                if (NEAR == 2 && (k & 1)) __builtin_amdgcn_sched_barrier(0);
             }
         }
     }

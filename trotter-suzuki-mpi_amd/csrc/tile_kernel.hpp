@@ -29,7 +29,9 @@
 // Otherwise W and H are the tile of a doubly periodic lattice of nx x ny inner
 // cells, both even (the pair pattern then is periodic too): rows and columns are
 // read from the inner cells they mirror, every cell of the tile is written, and
-// the halo is left as the exchange would leave it.
+// the halo is left as the exchange would leave it.  Mixed axes and odd periodic
+// extents run one step per pass on the closed tile, the state's halo cells read
+// from the cells they mirror (seam): no exchange runs between the steps.
 #pragma once
 #include "step_kernel.hpp"
 
@@ -46,6 +48,7 @@ struct TileParams {
     int W, H, pitch;
     int nx, ny;                      // inner extents of a doubly periodic lattice, or 0
     int steps;                       // k
+    int seam, px, py;                // 1: one step on the reference tile, the state's halo read through seam_off
     int n_strips, cols, rows;        // output columns and rows per tile
     T mH, tH, mV, tV, unH, unV;      // scaled-frame pair factors (StepParams)
     T m2, t2, un2;                   // the merged V0 V0 pass
@@ -54,6 +57,42 @@ struct TileParams {
     double mag, mag_mid;             // |corr| of the last step and of the steps before it
     T dphi;                          // phase of the merged frame, added to every phase
 };
+
+// A cell of the reference tile whose halo exchange has not run: where its value
+// is (a byte offset), as exchange_cell would have copied it.  The copy's own
+// quirk is kept: with a closed y axis the x halo of the last 2 halo rows stays.
+struct SeamTile {
+    int W, H, px, py;
+};
+__device__ __forceinline__ unsigned seam_off(const SeamTile &q, int x, int y, unsigned row_bytes, unsigned esz) {
+    if (x < 0 || x >= q.W || y < 0 || y >= q.H) return kOffNone;
+    const int lo = q.py ? kApron : 0, hi = lo + max(0, q.H - 2 * kApron);   // rows whose x halo is refreshed
+    int sx = x, sy = y;
+    if (q.py && y < kApron) sy = y + q.H - 2 * kApron;
+    if (q.py && y >= q.H - kApron) sy = y - (q.H - 2 * kApron);
+    if (q.px && sy >= lo && sy < hi) {
+        if (x < kApron) sx = x + q.W - 2 * kApron;
+        if (x >= q.W - kApron) sx = x - (q.W - 2 * kApron);
+    }
+    return (unsigned)sx * esz + (unsigned)sy * row_bytes;
+}
+__device__ __forceinline__ float buf_load1(__amdgpu_buffer_rsrc_t r, unsigned off, float) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, off, 0u, 0));
+}
+__device__ __forceinline__ double buf_load1(__amdgpu_buffer_rsrc_t r, unsigned off, double) {
+    return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(r, off, 0u, 0));
+}
+// Two cells of a row, each from where it is.
+template <typename T>
+__device__ __forceinline__ void seam_load(const SeamTile &q, __amdgpu_buffer_rsrc_t re, __amdgpu_buffer_rsrc_t im, int x,
+                                          int y, unsigned row_bytes, Row<T, 2> &s) {
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+        const unsigned off = seam_off(q, x + k, y, row_bytes, (unsigned)sizeof(T));
+        s.re[k] = buf_load1(re, off, T(0));
+        s.im[k] = buf_load1(im, off, T(0));
+    }
+}
 
 template <typename T>
 struct TileXch {
@@ -65,7 +104,7 @@ struct TileXch {
 
 // The potential pass of two rows: one wave-uniform test and straight-line code
 // for the four values per lane.
-template <typename T, bool LHY, bool IMAG = false>
+template <typename T, bool LHY, bool IMAG = false, int NEAR = 1>
 __device__ __forceinline__ void tile_ppass(Row<T, 2> &a, Row<T, 2> &b, const T (&pa)[2], const T (&pb)[2], T c, T cl,
                                            double mag) {
     T ang[4], sn[4], cs[4];
@@ -89,7 +128,7 @@ __device__ __forceinline__ void tile_ppass(Row<T, 2> &a, Row<T, 2> &b, const T (
         }
         return;
     }
-    sincos_row<T, 4, true>(ang, sn, cs);
+    sincos_row<T, 4, NEAR>(ang, sn, cs);
     const T ca[2] = {cs[0], cs[1]}, sa[2] = {sn[0], sn[1]}, cb[2] = {cs[2], cs[3]}, sb[2] = {sn[2], sn[3]};
     rotate_row_ph<T, 2>(a, ca, sa, mag);
     rotate_row_ph<T, 2>(b, cb, sb, mag);
@@ -212,13 +251,13 @@ __device__ __forceinline__ void tile_steps(const TileParams<T> &p, Row<T, 2> (&s
     vpass(I0(), IM(), p.mV, p.tV, p.unV, [&] { h_rest(I0()); });
 }
 
+// Tile `tile` of the pass p by a workgroup of nw waves.
 template <typename T, bool LHY, int MODE, int R>
-__global__ void __launch_bounds__(kTileWavesMax * kWave) tile_kernel(TileParams<T> p) {
-    __shared__ TileXch<T> xch;
+__device__ __forceinline__ void tile_group(const TileParams<T> &p, int tile, TileXch<T> &xch) {
     const int lane = threadIdx.x & (kWave - 1);
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     const int nw = blockDim.x / kWave;
-    const int strip = blockIdx.x % p.n_strips, seg = blockIdx.x / p.n_strips;
+    const int strip = tile % p.n_strips, seg = tile / p.n_strips;
     const int A = kApron * p.steps;
     const bool wrap = p.nx != 0;
     const int X0 = strip * p.cols - A;                            // even
@@ -253,16 +292,25 @@ __global__ void __launch_bounds__(kTileWavesMax * kWave) tile_kernel(TileParams<
 
     Row<T, 2> s[R];
     T ph[R][2];
+    auto load = [&](auto seam) {
+        const SeamTile q = {p.W, p.H, p.px, p.py};
 #pragma unroll
-    for (int r = 0; r < R; ++r) {
-        const int y = y0 + r;
-        const bool in = wrap || (y >= 0 && y < p.H);
-        const int ys = wrap ? kApron + mod(y - kApron, p.ny) : y;
-        const unsigned off = in ? v_ld + (unsigned)ys * row_bytes : kOffNone;
-        buf_load<T, 2>(r_in_re, off, 0u, s[r].re);
-        buf_load<T, 2>(r_in_im, off, 0u, s[r].im);
-        buf_load<T, 2>(r_ph, off, 0u, ph[r]);
-    }
+        for (int r = 0; r < R; ++r) {
+            const int y = y0 + r;
+            const bool in = wrap || (y >= 0 && y < p.H);
+            const int ys = wrap ? kApron + mod(y - kApron, p.ny) : y;
+            const unsigned off = in ? v_ld + (unsigned)ys * row_bytes : kOffNone;
+            if constexpr (decltype(seam)::value) {
+                seam_load<T>(q, r_in_re, r_in_im, xl, y, row_bytes, s[r]);
+            } else {
+                buf_load<T, 2>(r_in_re, off, 0u, s[r].re);
+                buf_load<T, 2>(r_in_im, off, 0u, s[r].im);
+            }
+            buf_load<T, 2>(r_ph, off, 0u, ph[r]);
+        }
+    };
+    if (p.seam) load(std::true_type());
+    else load(std::false_type());
 #pragma unroll
     for (int r = 0; r < R; ++r) {
         ph[r][0] += p.dphi;
@@ -295,6 +343,23 @@ __global__ void __launch_bounds__(kTileWavesMax * kWave) tile_kernel(TileParams<
         buf_store<T, 2>(r_out_re, off, 0u, s[r].re);
         buf_store<T, 2>(r_out_im, off, 0u, s[r].im);
     }
+}
+
+template <typename T, bool LHY, int MODE, int R>
+__global__ void __launch_bounds__(kTileWavesMax * kWave) tile_kernel(TileParams<T> p) {
+    __shared__ TileXch<T> xch;
+    tile_group<T, LHY, MODE, R>(p, blockIdx.x, xch);
+}
+
+// One pass of many lattices: a workgroup per item (lattice, tile).
+template <typename T, bool LHY, int MODE, int R>
+__global__ void __launch_bounds__(kTileWavesMax * kWave) tile_batch_kernel(const TileParams<T> *__restrict__ params,
+                                                                           const int2 *__restrict__ items) {
+    __shared__ TileXch<T> xch;
+    const int2 it = items[blockIdx.x];
+    const int i = __builtin_amdgcn_readfirstlane(it.x), tile = __builtin_amdgcn_readfirstlane(it.y);
+    const TileParams<T> p = params[i];
+    tile_group<T, LHY, MODE, R>(p, tile, xch);
 }
 
 }  // namespace tsmi

@@ -38,6 +38,7 @@
 #include "common.hpp"
 #include "frame.hpp"
 #include "stage.hpp"
+#include "tile_plan.hpp"
 #include "tsmi_hip.h"
 
 using namespace tsmi;
@@ -45,8 +46,10 @@ using namespace tsmi;
 namespace {
 
 constexpr int kBlock = 256;
+constexpr int kGroups = 4;                     // see the top
 constexpr int kDefaultSegRows = 64;
 constexpr int kVecF = 2;                       // elements per lane of the fused passes
+constexpr long kTileCells32 = 7L << 19, kTileCells64 = 3L << 19;   // most cells of a batch run as tiles
 constexpr int kExchChunks = 64;                // most workgroups per lattice of an exchange launch
 
 #define TSMI_HIPB(call)                                                                              \
@@ -78,7 +81,9 @@ struct Lattice {
     // imaginary time: partial sums of |psi|^2 per buffer parity (max_waves
     // each), their two counts, and a divisor for host-side readers
     size_t partials = 0, div = 0, part_n = 0;
-    int group() const { return fused ? 1 : 0; }
+    int tile = 0;                             // 2, 3: in that tile group now; 0: not in one
+    int tile_group = 0;                       // the tile group it takes when every E has the phase form (0: none)
+    int group() const { return tile ? tile : (fused ? 1 : 0); }
 };
 
 size_t align256(size_t x) { return (x + 255) / 256 * 256; }
@@ -86,8 +91,17 @@ size_t align256(size_t x) { return (x + 255) / 256 * 256; }
 struct GraphRec {
     hipGraph_t g = nullptr;
     hipGraphExec_t x = nullptr;
-    int end[2] = {0, 0};
+    int end[kGroups] = {0, 0, 0, 0};
 };
+
+// One tile pass over a tile group: its shape, parameters per buffer parity, items.
+struct TilePass {
+    TilePlan g;
+    void *params[2] = {nullptr, nullptr};
+    int2 *items = nullptr;
+    int n_items = 0;
+};
+enum TileHow { kClosed, kWrap, kSeam };   // as tsmi_tile.hip's passes
 
 }  // namespace
 
@@ -105,7 +119,9 @@ struct tsmi_batch {
     int n_items[3] = {0, 0, 0}, items_cap[3] = {0, 0, 0};
     void *exch[2][2] = {{nullptr, nullptr}, {nullptr, nullptr}};   // [group][buffer holding the state]
     int n_exch[2] = {0, 0}, exch_chunks[2] = {1, 1};
-    int cur[2] = {0, 0};                      // buffer holding the states, per group
+    int cur[kGroups] = {0, 0, 0, 0};          // buffer holding the states, per group
+    int n_tiled[kGroups] = {0, 0, 0, 0};      // lattices in the tile groups
+    std::map<std::tuple<int, int, int>, TilePass> tile_passes;   // by (group, how, steps)
     bool ph = false;                          // every lattice's E has the one-plane form
     int grid[2] = {0, 0}, grid2[2] = {0, 0};   // persistent grids of the E form [0] and the phase form [1]
     hipStream_t own = nullptr, stream = nullptr, side = nullptr;
@@ -124,12 +140,22 @@ void drop_graphs(tsmi_batch *b) {
     b->graphs.clear();
 }
 
+void drop_tile_passes(tsmi_batch *b) {
+    for (auto &t : b->tile_passes) {
+        void *ptrs[] = {t.second.params[0], t.second.params[1], t.second.items};
+        for (void *p : ptrs)
+            if (p) (void)hipFree(p);
+    }
+    b->tile_passes.clear();
+}
+
 void free_batch(tsmi_batch *b) {
     drop_graphs(b);
     void *ptrs[] = {b->arena,    b->params[0], b->params[1], b->params2[0], b->params2[1], b->items[0], b->items[1],
                     b->items[2], b->exch[0][0], b->exch[0][1], b->exch[1][0], b->exch[1][1]};
     for (void *p : ptrs)
         if (p) (void)hipFree(p);
+    drop_tile_passes(b);
     if (b->fork) (void)hipEventDestroy(b->fork);
     if (b->join) (void)hipEventDestroy(b->join);
     if (b->side) (void)hipStreamDestroy(b->side);
@@ -237,7 +263,7 @@ int upload_item_list(tsmi_batch *b, int list) {
     std::vector<int> rows;
     for (int i = 0; i < b->n; ++i) {
         const Lattice &L = b->lat[i];
-        if ((list == 0 && L.fused) || (list > 0 && !L.fused)) continue;
+        if (L.group() != (list == 0 ? 0 : 1)) continue;
         const int waves = list == 2 ? L.n_waves2 : L.n_waves;
         for (int w = 0; w < waves; ++w) items.push_back(make_int2(i, w));
     }
@@ -393,10 +419,139 @@ int fused_pass(tsmi_batch *b, hipStream_t s, int *cur) {
     return exchange(b, s, 1, cur[1]);
 }
 
-// n steps of every lattice, eagerly; cur[] is updated to the buffers holding
-// the results.  Group 0 goes to the side stream when both groups have work.
+// ---------------------------------------------------------------------------
+// tile groups
+// ---------------------------------------------------------------------------
+std::vector<std::pair<int, int>> tile_sizes(const tsmi_batch *b, int group) {
+    std::vector<std::pair<int, int>> v;
+    for (const Lattice &L : b->lat)
+        if (L.tile == group) v.emplace_back(L.W, L.H);
+    return v;
+}
+
+template <typename T>
+int build_tile_pass(tsmi_batch *b, int group, TileHow how, int steps, TilePass *out) {
+    TilePass t;
+    t.g = tile_plan(tile_sizes(b, group), b->esz, steps);
+    if (t.g.r == 0) return set_error(TSMI_E_INVALID, "batch tile pass: no tile for this many steps");
+    std::vector<TileParams<T>> h[2];
+    std::vector<int2> items;
+    char *a = b->arena;
+    for (const Lattice &L : b->lat) {
+        if (L.tile != group) continue;
+        const StepCoefs &k = L.k;
+        const TileFactors f = {k.mH, k.tH, k.mV, k.tV, k.unH, k.unV, k.c_nl_s, k.c_lhy_s, k.corr_abs,
+                               L.d.delta_t / (4. * L.d.mass * L.d.delta_y * L.d.delta_y)};
+        const bool wrap = how == kWrap && L.d.periodic_x;
+        long double drift = 0.0L;   // within the pass
+        TileParams<T> p;
+        std::memset(&p, 0, sizeof(p));
+        tile_params<T>(p, f, t.g, L.W, L.H, L.pitch, wrap ? L.d.dim_x : 0, wrap ? L.d.dim_y : 0, steps, drift);
+        p.seam = how == kSeam;
+        p.px = L.d.periodic_x != 0; p.py = L.d.periodic_y != 0;
+        p.ph = (const T *)(a + L.ph);
+        const int i = (int)h[0].size(), tiles = p.n_strips * ((L.H + p.rows - 1) / p.rows);
+        for (int c = 0; c < 2; ++c) {
+            p.in_re = (const T *)(a + L.psi[c][0]);
+            p.in_im = (const T *)(a + L.psi[c][1]);
+            p.out_re = (T *)(a + L.psi[1 - c][0]);
+            p.out_im = (T *)(a + L.psi[1 - c][1]);
+            h[c].push_back(p);
+        }
+        for (int j = 0; j < tiles; ++j) items.push_back(make_int2(i, j));
+    }
+    t.n_items = (int)items.size();
+    const size_t pb = h[0].size() * sizeof(TileParams<T>), ib = items.size() * sizeof(int2);
+    hipError_t e = hipMalloc((void **)&t.items, ib);
+    for (int c = 0; c < 2 && e == hipSuccess; ++c) {
+        e = hipMalloc(&t.params[c], pb);
+        if (e == hipSuccess) e = hipMemcpyAsync(t.params[c], h[c].data(), pb, hipMemcpyHostToDevice, b->stream);
+    }
+    if (e == hipSuccess) e = hipMemcpyAsync(t.items, items.data(), ib, hipMemcpyHostToDevice, b->stream);
+    if (e == hipSuccess) e = hipStreamSynchronize(b->stream);
+    if (e != hipSuccess) {
+        void *ptrs[] = {t.params[0], t.params[1], t.items};
+        for (void *p : ptrs)
+            if (p) (void)hipFree(p);
+        return set_error(TSMI_E_HIP, std::string("batch tile pass: ") + hipGetErrorString(e));
+    }
+    *out = t;
+    return TSMI_OK;
+}
+
+// The tile passes of an n-step call of one group, in order: as tile_passes and
+// tile_seam_steps run a single lattice.  `run` is called with each.
+template <typename F>
+int tile_sequence(tsmi_batch *b, int group, int n, F &&run) {
+    bool periodic = false;
+    for (const Lattice &L : b->lat) periodic = periodic || (L.tile == group && L.d.periodic_x);
+    int st = TSMI_OK;
+    auto several = [&](int m, TileHow how) {
+        if (m <= 0) return;
+        const int k = tile_best_steps(tile_sizes(b, group), b->esz, m), q = (m + k - 1) / k;
+        for (int j = 0; j < q && !st; ++j) st = run(how, m / q + (j < m % q ? 1 : 0));
+    };
+    if (group == 2 && !periodic) {
+        several(n, kClosed);
+    } else if (group == 2 && n >= 3) {
+        st = run(kClosed, 1);
+        if (!st) several(n - 2, kWrap);
+        if (!st) st = run(kClosed, 1);
+    } else {
+        for (int j = 0; j < n && !st; ++j) st = run(j == 0 ? kClosed : kSeam, 1);
+    }
+    return st;
+}
+
+// Builds what an n-step call needs (allocates; not inside a capture).
+int prepare_tiles(tsmi_batch *b, int n) {
+    for (int group = 2; group < kGroups; ++group) {
+        if (b->n_tiled[group] == 0) continue;
+        const int st = tile_sequence(b, group, n, [&](TileHow how, int steps) -> int {
+            const auto key = std::make_tuple(group, (int)how, steps);
+            if (b->tile_passes.count(key)) return TSMI_OK;
+            TilePass t;
+            const int s = b->esz == 4 ? build_tile_pass<float>(b, group, how, steps, &t)
+                                      : build_tile_pass<double>(b, group, how, steps, &t);
+            if (!s) b->tile_passes.emplace(key, t);
+            return s;
+        });
+        if (st) return st;
+    }
+    return TSMI_OK;
+}
+
+int run_tiles(tsmi_batch *b, hipStream_t s, int group, int n, int *cur) {
+    if (b->n_tiled[group] == 0) return TSMI_OK;
+    return tile_sequence(b, group, n, [&](TileHow how, int steps) -> int {
+        const TilePass &t = b->tile_passes.at(std::make_tuple(group, (int)how, steps));
+        const int st = tile_batch_launch(b->esz, b->lhy, b->mode, t.g, t.params[cur[group]], t.items, t.n_items, s);
+        cur[group] ^= 1;
+        return st;
+    });
+}
+
+// Brings every lattice's state into the buffer group 0's is in, so that a
+// lattice that changes group finds its state where its new group looks.
+int unify_buffers(tsmi_batch *b) {
+    for (const Lattice &L : b->lat) {
+        const int from = b->cur[L.group()];
+        if (from == b->cur[0]) continue;
+        const size_t pb = (size_t)L.pitch * (size_t)L.Hd * (size_t)b->esz;
+        for (int c = 0; c < 2; ++c)
+            TSMI_HIPB(hipMemcpyAsync(b->arena + L.psi[b->cur[0]][c] - L.shift, b->arena + L.psi[from][c] - L.shift, pb,
+                                     hipMemcpyDeviceToDevice, b->stream));
+    }
+    for (int g = 1; g < kGroups; ++g) b->cur[g] = b->cur[0];
+    drop_graphs(b);
+    return TSMI_OK;
+}
+
+// n steps of every lattice, eagerly (after prepare_tiles(n)); cur[] is updated to
+// the buffers holding the results.  Groups 0 and 3 (one step per pass) go to the
+// side stream when the others have work too.
 int batch_run(tsmi_batch *b, int n, int *cur) {
-    const bool both = b->n_items[0] > 0 && b->n_items[1] > 0;
+    const bool both = (b->n_items[0] > 0 || b->n_tiled[3] > 0) && (b->n_items[1] > 0 || b->n_tiled[2] > 0);
     hipStream_t s0 = both ? b->side : b->stream;
     if (both) {
         TSMI_HIPB(hipEventRecord(b->fork, b->stream));
@@ -404,6 +559,7 @@ int batch_run(tsmi_batch *b, int n, int *cur) {
     }
     int st = TSMI_OK;
     for (int i = 0; i < n && !st; ++i) st = single_pass(b, s0, 0, cur, i != n - 1);
+    if (!st) st = run_tiles(b, s0, 3, n, cur);
     if (!st && b->n_items[1] > 0) {
         if (n < 3) {
             for (int i = 0; i < n && !st; ++i) st = single_pass(b, b->stream, 1, cur, i != n - 1);
@@ -415,6 +571,7 @@ int batch_run(tsmi_batch *b, int n, int *cur) {
             if (!st) st = single_pass(b, b->stream, 1, cur, false);
         }
     }
+    if (!st) st = run_tiles(b, b->stream, 2, n, cur);
     if (both) {
         // join even after an error, so that a capture in progress stays well formed
         TSMI_HIPB(hipEventRecord(b->join, b->side));
@@ -448,6 +605,23 @@ hipError_t occupancy2_of(const tsmi_batch *b, int *blocks) {
                       : q((const void *)batch_step2_kernel<float, kVecF, false, 0, PH>);
     return b->lhy ? q((const void *)batch_step2_kernel<double, kVecF, true, 0, PH>)
                   : q((const void *)batch_step2_kernel<double, kVecF, false, 0, PH>);
+}
+
+// Puts the lattices that may run as tiles into their groups (every E has the
+// phase form) or back.
+int set_tiles(tsmi_batch *b) {
+    bool any = false;
+    for (const Lattice &L : b->lat) any = any || L.tile_group != 0;
+    if (!any) return TSMI_OK;
+    if (int st = unify_buffers(b)) return st;
+    drop_tile_passes(b);
+    for (int g = 0; g < kGroups; ++g) b->n_tiled[g] = 0;
+    for (Lattice &L : b->lat) {
+        L.tile = b->ph ? L.tile_group : 0;
+        if (L.tile) ++b->n_tiled[L.tile];
+    }
+    const int st = b->esz == 4 ? upload_exchange<float>(b) : upload_exchange<double>(b);
+    return st ? st : upload_layout(b);
 }
 
 Lattice *lattice_at(tsmi_batch *b, int i, const char *who) {
@@ -619,6 +793,21 @@ int tsmi_batch_create(const tsmi_desc *descs, int32_t n, tsmi_batch **out) {
     }
     b->mode = mode;
     b->arena_bytes = off;
+    // Tiles: real time, neither segment heights nor steps per pass asked for, and
+    // few enough cells in all that a wave's row latency bounds the streaming passes
+    // (us per step, streamed with 64-row segments against tiles: 4 x 100^2 periodic
+    // FP32 32 -> 2.7, FP64 33 -> 3.4, 32 x 256^2 FP32 36 -> 12, 12 x 512^2 FP32 35 ->
+    // 15; FP64 32 x 256^2, past the line, 38 -> 32).  Above it the streaming passes,
+    // which autotuning helps and tiles not, are near their memory time.
+    long cells = 0;
+    for (const Lattice &L : b->lat) cells += (long)L.W * L.H;
+    if (!b->imag && cells <= (b->esz == 4 ? kTileCells32 : kTileCells64))
+        for (Lattice &L : b->lat) {
+            const tsmi_desc &d = L.d;
+            if (d.sweeps != 0 || d.tile_rows > 0 || L.H < 2) continue;
+            const bool even = d.dim_x % 2 == 0 && d.dim_y % 2 == 0;
+            L.tile_group = (!d.periodic_x && !d.periodic_y) || (d.periodic_x && d.periodic_y && even) ? 2 : 3;
+        }
     auto bail = [&](int code) {
         free_batch(b);
         delete b;
@@ -716,6 +905,7 @@ int tsmi_batch_set_exp_potential(tsmi_batch *b, int32_t i, const double *e_re, c
     if (all != b->ph) {
         b->ph = all;
         drop_graphs(b);   // recorded with the other form's kernels
+        return set_tiles(b);
     }
     return TSMI_OK;
 }
@@ -724,12 +914,12 @@ int tsmi_batch_evolve(tsmi_batch *b, int32_t n) {
     if (!b) return set_error(TSMI_E_INVALID, "tsmi_batch_evolve: null batch");
     if (n < 0) return set_error(TSMI_E_INVALID, "tsmi_batch_evolve: negative step count");
     if (n == 0) return TSMI_OK;
-    const std::tuple<int, int, int> key(n, b->cur[0], b->cur[1]);
+    const std::tuple<int, int, int> key(n, b->cur[0] + 2 * b->cur[1], b->cur[2] + 2 * b->cur[3]);
     auto it = b->graphs.find(key);
     if (it == b->graphs.end()) {
+        if (int st = prepare_tiles(b, n)) return st;
         GraphRec rec;
-        rec.end[0] = b->cur[0];
-        rec.end[1] = b->cur[1];
+        std::copy(b->cur, b->cur + kGroups, rec.end);
         TSMI_HIPB(hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal));
         const int st = batch_run(b, n, rec.end);
         hipGraph_t captured = nullptr;
@@ -748,8 +938,7 @@ int tsmi_batch_evolve(tsmi_batch *b, int32_t n) {
         it = b->graphs.emplace(key, rec).first;
     }
     TSMI_HIPB(hipGraphLaunch(it->second.x, b->stream));
-    b->cur[0] = it->second.end[0];
-    b->cur[1] = it->second.end[1];
+    std::copy(it->second.end, it->second.end + kGroups, b->cur);
     return TSMI_OK;
 }
 
@@ -778,19 +967,8 @@ int tsmi_batch_tune(tsmi_batch *b, int32_t steps, double *ms_per_step) {
     // has 2 (or 3) single steps beside its fused passes: comparing one with two
     // steps per pass takes trials long enough for the passes to dominate.
     const int tsteps = any_tunable ? std::max(steps, 24) : (any_fusable ? std::max(steps, 6) : steps);
-    // A lattice may change group: first bring both groups' states into the same
-    // buffer, so that every membership finds its state where its group looks.
-    if (b->cur[1] != b->cur[0]) {
-        for (const Lattice &L : b->lat) {
-            if (L.group() != 1) continue;
-            const size_t pb = (size_t)L.pitch * (size_t)L.Hd * (size_t)b->esz;
-            for (int c = 0; c < 2; ++c)
-                TSMI_HIPB(hipMemcpyAsync(b->arena + L.psi[b->cur[0]][c] - L.shift, b->arena + L.psi[b->cur[1]][c] - L.shift,
-                                         pb, hipMemcpyDeviceToDevice, b->stream));
-        }
-        b->cur[1] = b->cur[0];
-        drop_graphs(b);
-    }
+    // a lattice may change group
+    if (int us = unify_buffers(b)) return us;
     auto relayout = [&]() -> int {
         const int st = b->esz == 4 ? upload_exchange<float>(b) : upload_exchange<double>(b);
         return st ? st : upload_layout(b);
@@ -811,9 +989,12 @@ int tsmi_batch_tune(tsmi_batch *b, int32_t steps, double *ms_per_step) {
         restore();
         return set_error(TSMI_E_HIP, std::string("tsmi_batch_tune: ") + hipGetErrorString(e));
     }
-    int cur[2] = {b->cur[0], b->cur[1]};
+    int cur[kGroups];
+    std::copy(b->cur, b->cur + kGroups, cur);
     auto trial = [&](float *ms) -> int {
         if (int st = relayout()) return st;
+        if (int st = prepare_tiles(b, 1)) return st;
+        if (int st = prepare_tiles(b, tsteps)) return st;
         if (int st = batch_run(b, 1, cur)) return st;   // warm-up
         TSMI_HIPB(hipEventRecord(t0, b->stream));
         if (int st = batch_run(b, tsteps, cur)) return st;
@@ -827,6 +1008,7 @@ int tsmi_batch_tune(tsmi_batch *b, int32_t steps, double *ms_per_step) {
     std::map<std::tuple<int, int, int>, std::vector<int>> classes;
     for (int i = 0; i < b->n; ++i) {
         const Lattice &L = b->lat[i];
+        if (L.tile) continue;   // tiles have no segment heights
         if (!L.fixed_rows || L.tunable) classes[std::make_tuple(L.tunable ? 2 : L.group(), L.Hd, L.Wd)].push_back(i);
     }
     std::vector<std::tuple<int, int, int>> order;
@@ -882,7 +1064,7 @@ int tsmi_batch_tune(tsmi_batch *b, int32_t steps, double *ms_per_step) {
         apply(best_kind, best_rows);
         best_all = best;
     }
-    if (!st) st = relayout();
+    if (!st) st = order.empty() ? trial(&best_all) : relayout();
     (void)hipEventDestroy(t0);
     (void)hipEventDestroy(t1);
     restore();

@@ -605,8 +605,9 @@ int evolve_steps(tsmi_ctx *c, int n, bool exchange_last = false) {
         }
         // mixed axes; odd periodic extents, where the pair pattern of a halo cell
         // differs from that of the cell it mirrors
-        for (int i = 0; i < n && !st; ++i) st = step_once(c, i != n - 1 ? 1 : last_ex);
-        return st;
+        if (n > 0) st = tile_passes(c, 1, false);
+        if (!st) st = tile_seam_steps(c, n - 1);
+        return st || !last_ex || n <= 0 ? st : exchange_current(c);
     }
     if (c->sweeps != 2 || n < 2 || (c->halo8 && n < 3)) {
         for (int i = 0; i < n && !st; ++i) st = step_once(c, i != n - 1 ? 1 : last_ex);

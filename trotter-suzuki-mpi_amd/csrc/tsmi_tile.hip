@@ -14,6 +14,7 @@
 #include "context.hpp"
 #include "frame.hpp"
 #include "tile_kernel.hpp"
+#include "tile_plan.hpp"
 
 using namespace tsmi;
 
@@ -22,11 +23,6 @@ namespace {
 // Rows per wave of the compiled instances.
 constexpr int kRows32[] = {4, 8, 12}, kRows64[] = {4, 6, 8};
 
-struct Plan {
-    int r = 0, nw = 0, cols = 0, rows = 0, strips = 0, segs = 0;
-    double us = 1e30;    // modelled time per step
-};
-
 // The tile shape of a pass of `steps` steps: the one with the least modelled time.
 // A launch costs about 5 us whatever it does; a step costs each SIMD its rows
 // (about 0.17 us a row in FP32, 0.27 in FP64 with several waves per SIMD, up to
@@ -34,22 +30,22 @@ struct Plan {
 // per step: 256^2 FP64 4 rows x 8 waves 6.9, 4.9, 4.4 for 1, 2, 3 steps, 8 x 8
 // 10.7, 7.9, 7.1; 1024^2 FP32 8 x 8 9.4, 6.7, 9.8 (3 steps: more than one
 // workgroup per compute unit), 12 x 8 12.4, 8.9, 7.3, 7.2, 7.0 (5 steps).
-Plan plan(int W, int H, int esz, int steps) {
-    Plan best;
+TilePlan plan(const std::pair<int, int> *size, size_t count, int esz, int steps) {
+    TilePlan best;
     const int a = kApron * steps;
     const int *rr = esz == 4 ? kRows32 : kRows64;
     const double c_row = esz == 4 ? 0.17 : 0.27, x = 0.35, t0 = 5.0;
     for (int i = 0; i < 3; ++i)
         for (int nw = 4; nw <= kTileWavesMax; nw += 4) {
-            Plan p;
+            TilePlan p;
             p.r = rr[i];
             p.nw = nw;
-            p.cols = kTileCols - 2 * a;
-            p.rows = nw * p.r - 2 * a;
-            if (p.cols < 2 || p.rows < 2) continue;
-            p.strips = (W + p.cols - 1) / p.cols;
-            p.segs = (H + p.rows - 1) / p.rows;
-            const double n = p.strips * p.segs / 256.0;              // workgroups per compute unit
+            const int cols = kTileCols - 2 * a, rows = nw * p.r - 2 * a;
+            if (cols < 2 || rows < 2) continue;
+            long tiles = 0;
+            for (size_t j = 0; j < count; ++j)
+                tiles += (long)((size[j].first + cols - 1) / cols) * ((size[j].second + rows - 1) / rows);
+            const double n = tiles / 256.0;                          // workgroups per compute unit
             const double per_cu = n < 6 ? std::ceil(n) : n + 0.5;    // ... on the busiest one
             const double waves = std::min(per_cu * nw / 4.0, 3.0);   // waves per SIMD
             p.us = t0 / steps + per_cu * nw * p.r / 4.0 * c_row * (1 + 0.6 / waves) + x;
@@ -58,11 +54,11 @@ Plan plan(int W, int H, int esz, int steps) {
     return best;
 }
 
-int best_steps(int W, int H, int esz, int most) {
+int best_steps(const std::pair<int, int> *size, size_t count, int esz, int most) {
     int k = 1;
     double us = 1e30;
     for (int s = 1; s <= std::min(most, 8); ++s) {
-        const Plan p = plan(W, H, esz, s);
+        const TilePlan p = plan(size, count, esz, s);
         if (p.us < us) {
             us = p.us;
             k = s;
@@ -71,50 +67,94 @@ int best_steps(int W, int H, int esz, int most) {
     return k;
 }
 
+// Launches tile_kernel, or (items) tile_batch_kernel.
 template <typename T, bool LHY, int MODE, int R>
-int launch(tsmi_ctx *c, const TileParams<T> &p, const Plan &g) {
-    if (int st = ctx_time_mark(c, p.steps > 1, 0)) return st;
-    hipLaunchKernelGGL((tile_kernel<T, LHY, MODE, R>), dim3(g.strips * g.segs), dim3(g.nw * kWave), 0, c->stream, p);
-    const hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return set_error(TSMI_E_HIP, std::string("tile_kernel: ") + hipGetErrorString(e));
-    return ctx_time_mark(c, p.steps > 1, 1);
+void launch(const TilePlan &g, int blocks, const TileParams<T> *p, const int2 *items, hipStream_t s) {
+    if (items)
+        hipLaunchKernelGGL((tile_batch_kernel<T, LHY, MODE, R>), dim3(blocks), dim3(g.nw * kWave), 0, s, p, items);
+    else
+        hipLaunchKernelGGL((tile_kernel<T, LHY, MODE, R>), dim3(blocks), dim3(g.nw * kWave), 0, s, *p);
 }
 
 template <typename T, bool LHY, int R>
-int launch_mode(tsmi_ctx *c, const TileParams<T> &p, const Plan &g) {
-    if (c->mode == 0) return launch<T, LHY, 0, R>(c, p, g);
-    if (c->mode == 1) return launch<T, LHY, 1, R>(c, p, g);
-    return launch<T, LHY, -1, R>(c, p, g);
+void launch_mode(int mode, const TilePlan &g, int blocks, const TileParams<T> *p, const int2 *items, hipStream_t s) {
+    if (mode == 0) launch<T, LHY, 0, R>(g, blocks, p, items, s);
+    else if (mode == 1) launch<T, LHY, 1, R>(g, blocks, p, items, s);
+    else launch<T, LHY, -1, R>(g, blocks, p, items, s);
 }
 
 template <typename T, bool LHY>
-int launch_rows(tsmi_ctx *c, const TileParams<T> &p, const Plan &g) {
+int launch_rows(int mode, const TilePlan &g, int blocks, const TileParams<T> *p, const int2 *items, hipStream_t s) {
     constexpr const int *rr = sizeof(T) == 4 ? kRows32 : kRows64;
-    if (g.r == rr[0]) return launch_mode<T, LHY, rr[0]>(c, p, g);
-    if (g.r == rr[1]) return launch_mode<T, LHY, rr[1]>(c, p, g);
-    return launch_mode<T, LHY, rr[2]>(c, p, g);
+    if (g.r == rr[0]) launch_mode<T, LHY, rr[0]>(mode, g, blocks, p, items, s);
+    else if (g.r == rr[1]) launch_mode<T, LHY, rr[1]>(mode, g, blocks, p, items, s);
+    else launch_mode<T, LHY, rr[2]>(mode, g, blocks, p, items, s);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return set_error(TSMI_E_HIP, std::string("tile_kernel: ") + hipGetErrorString(e));
+    return TSMI_OK;
 }
 
 template <typename T>
-int pass(tsmi_ctx *c, int steps, bool wrap, long double &drift) {
+int launch_any(bool lhy, int mode, const TilePlan &g, int blocks, const TileParams<T> *p, const int2 *items,
+               hipStream_t s) {
+    return lhy ? launch_rows<T, true>(mode, g, blocks, p, items, s)
+               : launch_rows<T, false>(mode, g, blocks, p, items, s);
+}
+
+// One pass of context c.  how: kClosed, kWrap, kSeam.
+enum How { kClosed, kWrap, kSeam };
+
+template <typename T>
+int pass(tsmi_ctx *c, int steps, How how, long double &drift) {
     TileParams<T> p;
     std::memset(&p, 0, sizeof(p));
     const int nb = 1 - c->cur;
+    const std::pair<int, int> size(c->W, c->H);
+    const TilePlan g = plan(&size, 1, c->esz, steps);
+    if (g.r == 0) return set_error(TSMI_E_INVALID, "tile pass: no tile for this many steps");
+    const TileFactors f = {c->mH, c->tH, c->mV, c->tV, c->unH, c->unV, c->c_nl_s, c->c_lhy_s, c->corr_abs,
+                           c->d.delta_t / (4. * c->d.mass * c->d.delta_y * c->d.delta_y)};
+    const bool wrap = how == kWrap;
+    tile_params<T>(p, f, g, c->W, c->H, c->pitch, wrap ? c->d.dim_x : 0, wrap ? c->d.dim_y : 0, steps, drift);
+    p.seam = how == kSeam;
+    p.px = c->d.periodic_x != 0; p.py = c->d.periodic_y != 0;
     p.in_re = (const T *)c->psi_re[c->cur];
     p.in_im = (const T *)c->psi_im[c->cur];
     p.out_re = (T *)c->psi_re[nb];
     p.out_im = (T *)c->psi_im[nb];
     p.ph = (const T *)c->ph;
-    p.W = c->W; p.H = c->H; p.pitch = c->pitch;
-    p.nx = wrap ? c->d.dim_x : 0;
-    p.ny = wrap ? c->d.dim_y : 0;
+    const int blocks = p.n_strips * ((c->H + p.rows - 1) / p.rows);
+    if (int st = ctx_time_mark(c, steps > 1, 0)) return st;
+    if (int st = launch_any<T>(c->c_lhy != 0.0, c->mode, g, blocks, &p, nullptr, c->stream)) return st;
+    c->cur = nb;
+    return ctx_time_mark(c, steps > 1, 1);
+}
+
+}  // namespace
+
+namespace tsmi {
+
+TilePlan tile_plan(const std::vector<std::pair<int, int>> &sizes, int esz, int steps) {
+    return plan(sizes.data(), sizes.size(), esz, steps);
+}
+
+int tile_best_steps(const std::vector<std::pair<int, int>> &sizes, int esz, int most) {
+    return best_steps(sizes.data(), sizes.size(), esz, most);
+}
+
+template <typename T>
+void tile_params(TileParams<T> &p, const TileFactors &f, const TilePlan &g, int W, int H, int pitch, int nx, int ny,
+                 int steps, long double &drift) {
+    p.W = W; p.H = H; p.pitch = pitch;
+    p.nx = nx;
+    p.ny = ny;
     p.steps = steps;
-    const Plan g = plan(c->W, c->H, c->esz, steps);
-    if (g.r == 0) return set_error(TSMI_E_INVALID, "tile pass: no tile for this many steps");
-    p.n_strips = g.strips; p.cols = g.cols; p.rows = g.rows;
-    p.mH = (T)c->mH; p.tH = (T)c->tH; p.mV = (T)c->mV; p.tV = (T)c->tV;
-    p.unH = (T)c->unH; p.unV = (T)c->unV;
-    p.c_nl = (T)c->c_nl_s; p.c_lhy = (T)c->c_lhy_s;
+    p.cols = kTileCols - 2 * kApron * steps;
+    p.rows = g.nw * g.r - 2 * kApron * steps;
+    p.n_strips = (W + p.cols - 1) / p.cols;
+    p.mH = (T)f.mH; p.tH = (T)f.tH; p.mV = (T)f.mV; p.tV = (T)f.tV;
+    p.unH = (T)f.unH; p.unV = (T)f.unV;
+    p.c_nl = (T)f.c_nl_s; p.c_lhy = (T)f.c_lhy_s;
     // The merged V0 V0 pass (factors m2, t2) stands for the square of V0's (m, t):
     // its eigenvalue is 1/q of the exact one, q = (m + i t)^2 / (m2 + i t2), so a
     // step followed by it applies |q| with |corr|.  The sign of q goes into the
@@ -125,30 +165,32 @@ int pass(tsmi_ctx *c, int steps, bool wrap, long double &drift) {
     // 64^2), so the last step of a pass takes back what the pass's and the
     // call's earlier ones left (drift: the log of what was applied over what was
     // meant).
-    const double by = c->d.delta_t / (4. * c->d.mass * c->d.delta_y * c->d.delta_y);
     typedef std::complex<long double> zl;
-    const Axis two = frame_axis(std::cos(2 * by), std::sin(2 * by), false, c->esz);
-    const zl v1(c->mV, c->tV), v2(two.m, two.t);
+    const Axis two = frame_axis(std::cos(2 * f.by), std::sin(2 * f.by), false, (int)sizeof(T));
+    const zl v1(f.mV, f.tV), v2(two.m, two.t);
     zl q = v1 * v1 / v2;
     const long double sign = q.real() < 0 ? -1.0L : 1.0L;
     q *= sign;
     p.m2 = (T)two.m; p.t2 = (T)two.t; p.un2 = (T)two.un;
     p.mode2 = two.form;
-    const long double mid = c->corr_abs * std::abs(q);
+    const long double mid = f.corr_abs * std::abs(q);
     p.mag_mid = (double)(sign * mid);
     drift += (steps - 1) * std::log(std::fabs((long double)p.mag_mid) / mid);
-    p.mag = (double)(c->corr_abs * (1.0L - drift));
-    drift += std::log((long double)p.mag / c->corr_abs);
+    p.mag = (double)(f.corr_abs * (1.0L - drift));
+    drift += std::log((long double)p.mag / f.corr_abs);
     p.dphi = (T)(-(steps - 1.0L) / steps * std::arg(q));
-    const bool lhy = c->c_lhy != 0.0;
-    const int st = lhy ? launch_rows<T, true>(c, p, g) : launch_rows<T, false>(c, p, g);
-    if (!st) c->cur = nb;
-    return st;
 }
 
-}  // namespace
+template void tile_params<float>(TileParams<float> &, const TileFactors &, const TilePlan &, int, int, int, int, int,
+                                 int, long double &);
+template void tile_params<double>(TileParams<double> &, const TileFactors &, const TilePlan &, int, int, int, int, int,
+                                  int, long double &);
 
-namespace tsmi {
+int tile_batch_launch(int esz, bool lhy, int mode, const TilePlan &g, const void *params, const int2 *items,
+                      int n_items, hipStream_t stream) {
+    return esz == 4 ? launch_any<float>(lhy, mode, g, n_items, (const TileParams<float> *)params, items, stream)
+                    : launch_any<double>(lhy, mode, g, n_items, (const TileParams<double> *)params, items, stream);
+}
 
 bool tile_wraps(const tsmi_ctx *c) {
     return c->d.periodic_x && c->d.periodic_y && c->d.dim_x % 2 == 0 && c->d.dim_y % 2 == 0;
@@ -166,18 +208,25 @@ bool tile_runs(const tsmi_ctx *c) {
            (long)c->W * c->H <= most && (long)c->pitch * c->Hd * c->esz < (1L << 31);
 }
 
-int tile_steps(const tsmi_ctx *c, int most) { return best_steps(c->W, c->H, c->esz, most); }
-
-static int tile_pass(tsmi_ctx *c, int steps, bool wrap, long double &drift) {
-    return c->esz == 4 ? pass<float>(c, steps, wrap, drift) : pass<double>(c, steps, wrap, drift);
+static int tile_pass(tsmi_ctx *c, int steps, How how, long double &drift) {
+    return c->esz == 4 ? pass<float>(c, steps, how, drift) : pass<double>(c, steps, how, drift);
 }
 
 int tile_passes(tsmi_ctx *c, int n, bool wrap) {
     if (n <= 0) return TSMI_OK;
-    const int k = tile_steps(c, n), passes = (n + k - 1) / k;
+    const std::pair<int, int> size(c->W, c->H);
+    const int k = best_steps(&size, 1, c->esz, n), passes = (n + k - 1) / k;
     long double drift = 0.0L;
     int st = TSMI_OK;
-    for (int i = 0; i < passes && !st; ++i) st = tile_pass(c, n / passes + (i < n % passes ? 1 : 0), wrap, drift);
+    for (int i = 0; i < passes && !st; ++i)
+        st = tile_pass(c, n / passes + (i < n % passes ? 1 : 0), wrap ? kWrap : kClosed, drift);
+    return st;
+}
+
+int tile_seam_steps(tsmi_ctx *c, int n) {
+    long double drift = 0.0L;
+    int st = TSMI_OK;
+    for (int i = 0; i < n && !st; ++i) st = tile_pass(c, 1, kSeam, drift);
     return st;
 }
 
