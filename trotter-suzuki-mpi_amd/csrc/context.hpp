@@ -97,4 +97,15 @@ int tile_passes(tsmi_ctx *c, int n, bool wrap);
 // state's halo cells are read from the cells they mirror).
 int tile_seam_steps(tsmi_ctx *c, int n);
 
+// Reverse sweep as tile passes (tsmi_adjoint_tile.hip): whether it runs so; the
+// steps of a pass, at most `most`; one pass of that many reverse steps, field 0 the
+// state, field 1 the adjoint state, planes (re, im) of the reference tile.
+struct AdjTileIo {
+    const void *in[2][2];
+    void *out[2][2];
+};
+bool adjoint_tiles_run(const tsmi_ctx *c);
+int adjoint_tile_steps(const tsmi_ctx *c, int most);
+int adjoint_tile_pass(tsmi_ctx *c, int steps, const AdjTileIo &io);
+
 }  // namespace tsmi

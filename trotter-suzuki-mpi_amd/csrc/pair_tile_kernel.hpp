@@ -128,6 +128,7 @@ struct PairTileParams {
     const T *ph[2];
     int W, H, pitch;
     int nx, ny;                      // as TileParams
+    int seam, px, py;                // as TileParams
     int steps;
     int n_strips, cols, rows;
     T mH[2], tH[2], mV[2], tV[2], unH[2], unV[2];
@@ -151,10 +152,16 @@ struct PairXch {
     T4 v[2][2][NW + 2][kWave];   // as TileXch: (a re, a im, b re, b im)
 };
 
-template <typename T, bool IMAG, int MODE, int R, bool EH, bool EV, int NW, typename LoadPh>
-__device__ __forceinline__ void pair_tile_steps(const PairTileParams<T> &p, Row<T, 2> (&s)[2][R],
-                                                PairXch<T, NW> &x, int w, int lane, int xl, unsigned ok,
-                                                LoadPh &&load_ph) {
+// p.steps steps of two fields on a tile held in registers (p: pair factors per
+// field, extents).  EH: the strip reaches past the tile's left or right edge
+// (per-lane factors); EV: so do the wave's rows at the top or bottom (bit r + 1 of
+// ok: rows r and r + 1 of the wave are both inside).  begin(st) runs before a step
+// changes the state, mid(r0, r1) is the potential stage of two rows, used(st) runs
+// after the last of them, end(st) after the step.
+template <typename T, bool IMAG, int MODE, int R, bool EH, bool EV, int NW, typename P, typename Begin, typename Mid,
+          typename Used, typename End>
+__device__ __forceinline__ void two_field_steps(const P &p, Row<T, 2> (&s)[2][R], PairXch<T, NW> &x, int w, int lane,
+                                                int xl, unsigned ok, Begin &&begin, Mid &&mid, Used &&used, End &&end) {
     static_assert(R % 2 == 0 && R >= 4, "row parities are fixed per register");
     typedef typename PairXch<T, NW>::T4 T4;
     constexpr int M = MODE < 0 ? 0 : MODE;
@@ -166,10 +173,6 @@ __device__ __forceinline__ void pair_tile_steps(const PairTileParams<T> &p, Row<
         hc1 = make_hcoef<T, 2>(xe, lane, We, p.mH[1], p.tH[1], p.unH[1]);
     }
     const T kH[2] = {M == 0 ? p.tH[0] : p.mH[0], M == 0 ? p.tH[1] : p.mH[1]};
-    // phase plane, plus the other component's start-of-step density; the plane is
-    // read anew for each step as soon as the potential pass of the one before has
-    // used it (it stays in the L2), which holds one set of registers, not two
-    T base[2][R][2];
     int buf = 0;
 
     auto hrow = [&](auto ss, auto rr, int r) {
@@ -238,17 +241,39 @@ __device__ __forceinline__ void pair_tile_steps(const PairTileParams<T> &p, Row<
             hrow(ss, I0(), r + 1);
         }
     };
-    auto ppass = [&](int r0, int r1) {
-#pragma unroll
-        for (int c = 0; c < 2; ++c) {
-            tile_ppass<T, false, IMAG, 2>(s[c][r0], s[c][r1], base[c][r0], base[c][r1], p.c_self[c], T(0), p.mag[c]);
-        }
-        __builtin_amdgcn_sched_barrier(0);   // one group of rows at a time: fewer registers at once
-    };
-
-    load_ph(base);
     for (int st = 0; st < p.steps; ++st) {
-        vpass(I0(), [&] {
+        vpass(I0(), [&] { begin(st); });
+        h_border(I0());
+        vpass(I1(), [&] { h_rest(I0()); });
+        h_border(I1());
+        h_rest(I1());
+        mid(0, R - 1);
+        h_border(I1());
+        vpass(I1(), [&] {
+#pragma unroll
+            for (int r = 1; r + 1 < R; r += 2) mid(r, r + 1);
+            used(st);
+            h_rest(I1());
+        });
+        h_border(I0());
+        vpass(I0(), [&] { h_rest(I0()); });
+        end(st);
+    }
+}
+
+// The steps of the two components.
+template <typename T, bool IMAG, int MODE, int R, bool EDGE, int NW, typename LoadPh>
+__device__ __forceinline__ void pair_tile_steps(const PairTileParams<T> &p, Row<T, 2> (&s)[2][R],
+                                                PairXch<T, NW> &x, int w, int lane, int xl, unsigned ok,
+                                                LoadPh &&load_ph) {
+    // phase plane, plus the other component's start-of-step density; the plane is
+    // read anew for each step as soon as the potential pass of the one before has
+    // used it (it stays in the L2), which holds one set of registers, not two
+    T base[2][R][2];
+    load_ph(base);
+    two_field_steps<T, IMAG, MODE, R, EDGE, EDGE, NW>(
+        p, s, x, w, lane, xl, ok,
+        [&](int) {
 #pragma unroll
             for (int r = 0; r < R; ++r) {
                 T na[2], nb[2];
@@ -260,33 +285,29 @@ __device__ __forceinline__ void pair_tile_steps(const PairTileParams<T> &p, Row<
                     base[1][r][k] += p.c_ab * na[k];
                 }
             }
-        });
-        h_border(I0());
-        vpass(I1(), [&] { h_rest(I0()); });
-        h_border(I1());
-        h_rest(I1());
-        ppass(0, R - 1);
-        h_border(I1());
-        vpass(I1(), [&] {
+        },
+        [&](int r0, int r1) {
 #pragma unroll
-            for (int r = 1; r + 1 < R; r += 2) ppass(r, r + 1);
+            for (int c = 0; c < 2; ++c)
+                tile_ppass<T, false, IMAG, 2>(s[c][r0], s[c][r1], base[c][r0], base[c][r1], p.c_self[c], T(0), p.mag[c]);
+            __builtin_amdgcn_sched_barrier(0);   // one group of rows at a time: fewer registers at once
+        },
+        [&](int st) {
             if (st + 1 < p.steps) load_ph(base);
-            h_rest(I1());
-        });
-        h_border(I0());
-        vpass(I0(), [&] { h_rest(I0()); });
-        // always, by the identity when there is no coupling: a branch would merge
-        // two versions of the state, and did so in copies of every register
-        if constexpr (!IMAG) {
-            const bool last = st == p.steps - 1;
-            const double cc = last ? p.cc2 : p.cc, sr = last ? p.cs_r2 : p.cs_r, si = last ? p.cs_i2 : p.cs_i;
+        },
+        [&](int st) {
+            // always, by the identity when there is no coupling: a branch would merge
+            // two versions of the state, and did so in copies of every register
+            if constexpr (!IMAG) {
+                const bool last = st == p.steps - 1;
+                const double cc = last ? p.cc2 : p.cc, sr = last ? p.cs_r2 : p.cs_r, si = last ? p.cs_i2 : p.cs_i;
 #pragma unroll
-            for (int r = 0; r < R; ++r) {
-                rabi_rows<T, 2>(s[0][r], s[1][r], cc, sr, si);
-                __builtin_amdgcn_sched_barrier(0);
+                for (int r = 0; r < R; ++r) {
+                    rabi_rows<T, 2>(s[0][r], s[1][r], cc, sr, si);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
             }
-        }
-    }
+        });
 }
 
 template <typename T, bool IMAG, int MODE, int R, int NW, bool WRAP>
@@ -346,9 +367,19 @@ __global__ void __launch_bounds__(NW * kWave, (kPairWaves<T, R, NW, WRAP && MODE
         const unsigned off = in ? v_ld + so[r] : kOffNone;
 #pragma unroll
         for (int c = 0; c < 2; ++c) {
+            if (!WRAP && p.seam) continue;
             buf_load<T, 2>(make_rsrc(p.in_re[c], bytes), off, 0u, s[c][r].re);
             buf_load<T, 2>(make_rsrc(p.in_im[c], bytes), off, 0u, s[c][r].im);
         }
+    }
+    if (!WRAP && p.seam) {
+        const SeamTile q = {p.W, p.H, p.px, p.py};
+#pragma unroll
+        for (int r = 0; r < R; ++r)
+#pragma unroll
+            for (int c = 0; c < 2; ++c)
+                seam_load<T>(q, make_rsrc(p.in_re[c], bytes), make_rsrc(p.in_im[c], bytes), xl, y0 + r, row_bytes,
+                             s[c][r]);
     }
     if constexpr (IMAG) {
         if (p.pend.part) {
@@ -363,7 +394,7 @@ __global__ void __launch_bounds__(NW * kWave, (kPairWaves<T, R, NW, WRAP && MODE
     __syncthreads();
 
     if constexpr (WRAP && MODE >= 0) {
-        pair_tile_steps<T, IMAG, MODE, R, false, false>(p, s, xch, w, lane, xl, 0u, load_ph);
+        pair_tile_steps<T, IMAG, MODE, R, false>(p, s, xch, w, lane, xl, 0u, load_ph);
     } else {
         unsigned ok = 0;
 #pragma unroll
@@ -371,9 +402,9 @@ __global__ void __launch_bounds__(NW * kWave, (kPairWaves<T, R, NW, WRAP && MODE
             if (wrap || (y0 + r >= 0 && y0 + r + 1 < p.H)) ok |= 1u << (r + 1);
         const bool edge = X0 < 0 || X0 + kTileCols > p.W || y0 <= 0 || y0 + R >= p.H;
         if (MODE < 0 || edge) {
-            pair_tile_steps<T, IMAG, MODE, R, true, true>(p, s, xch, w, lane, xl, ok, load_ph);
+            pair_tile_steps<T, IMAG, MODE, R, true>(p, s, xch, w, lane, xl, ok, load_ph);
         } else if constexpr (MODE >= 0) {
-            pair_tile_steps<T, IMAG, MODE, R, false, false>(p, s, xch, w, lane, xl, ok, load_ph);
+            pair_tile_steps<T, IMAG, MODE, R, false>(p, s, xch, w, lane, xl, ok, load_ph);
         }
     }
 

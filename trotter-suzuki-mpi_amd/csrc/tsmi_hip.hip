@@ -745,9 +745,13 @@ int reverse_sweep(tsmi_ctx *c, const double *g_re, const double *g_im, void **g0
     if (!st) st = import_device(c, L[0][1], g_im);
     if (st) return st;
     const void *s_re = c->psi_re[c->cur], *s_im = c->psi_im[c->cur];
+    const bool tiles = adjoint_tiles_run(c);   // passes that read through the periodic wrap
     if (per) {
         st = c->esz == 4 ? view_fold<float>(c, L[0][0], L[0][1]) : view_fold<double>(c, L[0][0], L[0][1]);
-        if (!st) st = view_exchange_any(c, L[0][0], L[0][1]);
+        if (st) return st;
+    }
+    if (per && !tiles) {
+        st = view_exchange_any(c, L[0][0], L[0][1]);
         const size_t row = (size_t)c->pitch * c->esz;
         TSMI_HIP(hipMemcpy2DAsync(S[0][0], row, s_re, row, (size_t)c->W * c->esz, c->H, hipMemcpyDeviceToDevice,
                                   c->stream));
@@ -759,7 +763,25 @@ int reverse_sweep(tsmi_ctx *c, const double *g_re, const double *g_im, void **g0
         s_im = S[0][1];
     }
     int k = 0;
-    for (int n = c->ck_steps - 1; n >= 0; --n) {
+    for (int n = c->ck_steps - 1; n >= 0 && tiles;) {
+        // down to the checkpoint below, in passes of about the same length
+        int m = n % c->ck_every + 1;
+        const int q = (m + adjoint_tile_steps(c, m) - 1) / adjoint_tile_steps(c, m);
+        for (int j = 0; j < q; ++j) {
+            const int o = 1 - k, steps = (m + q - j - 1) / (q - j);
+            const AdjTileIo io = {{{s_re, s_im}, {L[k][0], L[k][1]}}, {{S[o][0], S[o][1]}, {L[o][0], L[o][1]}}};
+            if ((st = adjoint_tile_pass(c, steps, io))) return st;
+            s_re = S[o][0];
+            s_im = S[o][1];
+            k = o;
+            m -= steps;
+            n -= steps;
+        }
+        const char *ck = (const char *)c->ck + (size_t)((n + 1) / c->ck_every) * 2 * pb + view_off;
+        s_re = ck;
+        s_im = ck + pb;
+    }
+    for (int n = tiles ? -1 : c->ck_steps - 1; n >= 0; --n) {
         const int o = 1 - k;
         st = adjoint_step(c, s_re, s_im, L[k][0], L[k][1], S[o][0], S[o][1], L[o][0], L[o][1]);
         if (!st && per) st = view_exchange_any(c, L[o][0], L[o][1]);

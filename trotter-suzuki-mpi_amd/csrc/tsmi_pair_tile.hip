@@ -10,68 +10,18 @@
 #include "common.hpp"
 #include "pair_context.hpp"
 #include "pair_tile_kernel.hpp"
+#include "two_field_plan.hpp"
 #include "tsmi_hip.h"
 
 using namespace tsmi;
 
 namespace {
 
-// Rows per wave and waves of the compiled instances.
-struct Shape { int r, nw; };
-constexpr Shape kShapes32[] = {{4, 8}, {8, 8}}, kShapes64[] = {{4, 8}, {4, 4}};
-
-struct Plan {
-    int r = 0, nw = 0, cols = 0, rows = 0, strips = 0, segs = 0;
-    double us = 1e30;    // modelled time per step
-};
-
-// The tile shape of a pass of `steps` steps: the one with the least modelled time.
-// A launch costs 4.5 us and its bytes; a step costs each SIMD its rows (of both
-// components; 0.27 us a row in FP32, 0.53 in FP64 with several waves per SIMD,
-// more for a wave alone) and 0.5 us of exchanges.  Measured around it, periodic,
-// us per step: 256^2 FP32 4 rows x 8 waves 7.9, 5.6, 4.9 for 1, 2, 3 steps, 8 x 8
-// 12.6, 9.3, 8.1; 1024^2 FP32 4 x 8 13.9, 13.0, 19.2, 8 x 8 15.8, 12.2, 17.1 (3
-// steps: more than one workgroup per compute unit); 512^2 FP64 4 x 8 10.9, 8.5, 12.7.
-Plan plan(int W, int H, int esz, int steps, bool wrap) {
-    Plan best;
-    const int a = kApron * steps;
-    const Shape *sh = esz == 4 ? kShapes32 : kShapes64;
-    const double c_row = esz == 4 ? 0.27 : 0.53, x = 0.5;
-    const double t0 = 4.5 + (double)W * H * 10 * esz / 6.5e6;
-    for (int i = 0; i < 2; ++i) {
-        Plan p;
-        p.r = sh[i].r;
-        p.nw = sh[i].nw;
-        p.cols = kTileCols - 2 * a;
-        p.rows = p.nw * p.r - 2 * a;
-        if (p.cols < 2 || p.rows < 2) continue;
-        p.strips = (W + p.cols - 1) / p.cols;
-        p.segs = (H + p.rows - 1) / p.rows;
-        const double n = p.strips * p.segs / 256.0;              // workgroups per compute unit
-        const double per_cu = n < 6 ? std::ceil(n) : n + 0.5;    // ... on the busiest one
-        const double most = wrap && esz == 4 && p.r == 4 ? 4.0 : 2.0;
-        const double waves = std::min(per_cu * p.nw / 4.0, most);   // waves per SIMD
-        p.us = t0 / steps + per_cu * p.nw * p.r / 4.0 * c_row * (1 + 0.6 / waves) + x;
-        if (p.us < best.us) best = p;
-    }
-    return best;
-}
-
-int best_steps(int W, int H, int esz, int most, bool wrap) {
-    int k = 1;
-    double us = 1e30;
-    for (int s = 1; s <= std::min(most, 6); ++s) {
-        const Plan p = plan(W, H, esz, s, wrap);
-        if (p.us < us) {
-            us = p.us;
-            k = s;
-        }
-    }
-    return k;
-}
+// Modelled us of a row of both components, and planes moved per launch.
+TwoFieldCost cost(int esz) { return esz == 4 ? TwoFieldCost{0.27, 10} : TwoFieldCost{0.53, 10}; }
 
 template <typename T, bool IMAG, int R, int NW, bool WRAP>
-int launch_kernel(tsmi_pair *p, const PairTileParams<T> &q, const Plan &g) {
+int launch_kernel(tsmi_pair *p, const PairTileParams<T> &q, const TwoFieldPlan &g) {
     // one scaled form for both components on both axes, or both factors
     const int mode = p->c[0]->mode == p->c[1]->mode ? p->c[0]->mode : -1;
     const dim3 grid(g.strips * g.segs), block(NW * kWave);
@@ -93,15 +43,14 @@ int launch_kernel(tsmi_pair *p, const PairTileParams<T> &q, const Plan &g) {
 }
 
 template <typename T, bool IMAG, int R, int NW>
-int launch(tsmi_pair *p, const PairTileParams<T> &q, const Plan &g) {
+int launch(tsmi_pair *p, const PairTileParams<T> &q, const TwoFieldPlan &g) {
     return q.nx ? launch_kernel<T, IMAG, R, NW, true>(p, q, g) : launch_kernel<T, IMAG, R, NW, false>(p, q, g);
 }
 
 template <typename T, bool IMAG>
-int launch_shape(tsmi_pair *p, const PairTileParams<T> &q, const Plan &g) {
-    constexpr const Shape *sh = sizeof(T) == 4 ? kShapes32 : kShapes64;
-    if (g.r == sh[0].r && g.nw == sh[0].nw) return launch<T, IMAG, sh[0].r, sh[0].nw>(p, q, g);
-    return launch<T, IMAG, sh[1].r, sh[1].nw>(p, q, g);
+int launch_shape(tsmi_pair *p, const PairTileParams<T> &q, const TwoFieldPlan &g) {
+    if constexpr (sizeof(T) == 4) return g.r == 4 ? launch<T, IMAG, 4, 8>(p, q, g) : launch<T, IMAG, 8, 8>(p, q, g);
+    else return g.nw == 8 ? launch<T, IMAG, 4, 8>(p, q, g) : launch<T, IMAG, 4, 4>(p, q, g);
 }
 
 // What is pending after an imaginary-time step in slot p->slot's partial sums,
@@ -121,10 +70,15 @@ PairNorm pending(tsmi_pair *p, double var, bool rabi) {
     return q;
 }
 
+// How a pass reads the state: the closed tile, the periodic lattice, or the tile
+// whose halo exchange has not been run (one step; seam_off).
+enum How { kClosed, kWrap, kSeam };
+
 // `steps` steps; the rotation after the last of them is by var (1 after the
 // others).  first: nothing pending from a step before (imaginary time).
 template <typename T>
-int pass(tsmi_pair *p, int steps, bool wrap, double var, bool rabi, bool first) {
+int pass(tsmi_pair *p, int steps, How how, double var, bool rabi, bool first) {
+    const bool wrap = how == kWrap;
     PairTileParams<T> q;
     std::memset(&q, 0, sizeof(q));
     const int cur = p->c[0]->cur, nb = 1 - cur;
@@ -144,8 +98,10 @@ int pass(tsmi_pair *p, int steps, bool wrap, double var, bool rabi, bool first) 
     q.W = p->W; q.H = p->H; q.pitch = p->pitch;
     q.nx = wrap ? p->c[0]->d.dim_x : 0;
     q.ny = wrap ? p->c[0]->d.dim_y : 0;
+    q.seam = how == kSeam;
+    q.px = p->c[0]->d.periodic_x != 0; q.py = p->c[0]->d.periodic_y != 0;
     q.steps = steps;
-    const Plan g = plan(p->W, p->H, p->esz, steps, wrap);
+    const TwoFieldPlan g = two_field_plan(p->W, p->H, p->esz, steps, wrap, cost(p->esz));
     if (g.r == 0) return set_error(TSMI_E_INVALID, "pair tile pass: no tile for this many steps");
     q.n_strips = g.strips; q.cols = g.cols; q.rows = g.rows;
     q.ix0 = p->ix0; q.ix1 = p->ix1; q.iy0 = p->iy0; q.iy1 = p->iy1;
@@ -172,8 +128,8 @@ int pass(tsmi_pair *p, int steps, bool wrap, double var, bool rabi, bool first) 
     return st;
 }
 
-int tile_pass(tsmi_pair *p, int steps, bool wrap, double var, bool rabi, bool first) {
-    return p->esz == 4 ? pass<float>(p, steps, wrap, var, rabi, first) : pass<double>(p, steps, wrap, var, rabi, first);
+int tile_pass(tsmi_pair *p, int steps, How how, double var, bool rabi, bool first) {
+    return p->esz == 4 ? pass<float>(p, steps, how, var, rabi, first) : pass<double>(p, steps, how, var, rabi, first);
 }
 
 // The renormalisation after the last step.
@@ -202,7 +158,8 @@ int finish(tsmi_pair *p, double var, bool rabi) {
 namespace tsmi {
 
 int pair_tile_blocks(const tsmi_pair *p) {
-    const Plan a = plan(p->W, p->H, p->esz, 1, false), b = plan(p->W, p->H, p->esz, 1, true);
+    const TwoFieldPlan a = two_field_plan(p->W, p->H, p->esz, 1, false, cost(p->esz)),
+                       b = two_field_plan(p->W, p->H, p->esz, 1, true, cost(p->esz));
     return std::max(a.strips * a.segs, b.strips * b.segs);
 }
 
@@ -227,27 +184,25 @@ int pair_tile_evolve(tsmi_pair *p, int n, bool rabi) {
     const int most = p->imag || !(closed || wrap) ? 1 : n;
     int i = 0, st = TSMI_OK;
     // n steps from step i on; the call's last rotation is by 1/2 (src/solver.cpp:222-225)
-    auto passes = [&](int m, bool w) {
-        const int k = best_steps(p->W, p->H, p->esz, std::min(m, most), w), q = (m + k - 1) / k;
+    auto passes = [&](int m, How how) {
+        const int k = two_field_best_steps(p->W, p->H, p->esz, std::min(m, most), how == kWrap, cost(p->esz));
+        const int q = (m + k - 1) / k;
         for (int j = 0; j < q && !st; ++j) {
             const int s = m / q + (j < m % q ? 1 : 0);
             i += s;
-            st = tile_pass(p, s, w, i == n ? 0.5 : 1.0, rabi, i == s);
+            st = tile_pass(p, s, how, i == n ? 0.5 : 1.0, rabi, i == s);
         }
     };
     if (closed) {
-        passes(n, false);
+        passes(n, kClosed);
     } else if (wrap) {
-        passes(1, false);
-        passes(n - 2, true);
-        if (!st) passes(1, false);
+        passes(1, kClosed);
+        passes(n - 2, kWrap);
+        if (!st) passes(1, kClosed);
     } else {
         // mixed axes; odd periodic extents, where the pair pattern of a halo cell
-        // differs from that of the cell it mirrors
-        for (int j = 0; j < n && !st; ++j) {
-            passes(1, false);
-            if (!st && j != n - 1) st = exchange_both(p);
-        }
+        // differs from that of the cell it mirrors; a call of two steps
+        for (int j = 0; j < n && !st; ++j) passes(1, j == 0 ? kClosed : kSeam);
     }
     if (!st && p->imag) st = finish(p, 0.5, rabi);
     return st;
