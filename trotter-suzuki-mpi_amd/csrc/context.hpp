@@ -50,6 +50,7 @@ struct tsmi_ctx {
     double *div = nullptr;
     double *partials = nullptr;
     int *part_n = nullptr;
+    int part_cap = 0;                    // partial sums per slot
     double *obs_partials = nullptr;      // kObsBlocksMax * OBS_COUNT block partials
     double *obs_out = nullptr;           // kObsOut results of the last observables pass
     int obs_blocks = 0;
@@ -86,8 +87,8 @@ int ctx_exchange(tsmi_ctx *c, void *re, void *im);
 // several steps per launch; which 0: before, 1: after).
 int ctx_time_mark(tsmi_ctx *c, int kind, int which);
 
-// Tile passes (tsmi_tile.hip), asynchronous on c's stream: whether c's real-time
-// steps run as them; whether c is a doubly periodic lattice whose passes may wrap
+// Tile passes (tsmi_tile.hip), asynchronous on c's stream: whether c's steps run
+// as them; whether c is a doubly periodic lattice whose passes may wrap
 // (several steps per launch); n steps as one or several passes, on the tile
 // closed at its edges or (wrap) on the periodic lattice, the halo refreshed.
 bool tile_runs(const tsmi_ctx *c);
@@ -96,6 +97,8 @@ int tile_passes(tsmi_ctx *c, int n, bool wrap);
 // n steps, each starting with the halo exchange that has not been run yet (the
 // state's halo cells are read from the cells they mirror).
 int tile_seam_steps(tsmi_ctx *c, int n);
+// Workgroups of a pass of one step.
+int tile_blocks(const tsmi_ctx *c);
 
 // Reverse sweep as tile passes (tsmi_adjoint_tile.hip): whether it runs so; the
 // steps of a pass, at most `most`; one pass of that many reverse steps, field 0 the

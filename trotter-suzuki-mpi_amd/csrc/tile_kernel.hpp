@@ -24,6 +24,11 @@
 // 2.8, 256^2 FP64 23.1 -> 4.4, 1024^2 FP32 17.0 -> 6.6, FP64 23.6 -> 10.5.  Now
 // bound by instruction issue (and by the launch, some 4 us of a pass).
 //
+// Imaginary time (kTileImag) takes one step per pass, as every step ends in a
+// renormalisation by the whole lattice's norm: the partial sums of a step's
+// workgroups are added by every wave of the next, which scales its rows as it
+// loads them (256^2 closed FP32 12.8 -> 7.0 us per step, FP64 15.3 -> 7.0).
+//
 // Two uses, by p.nx: 0: the tile W x H is closed at its edges (closed axes, or
 // one step on the reference tile of a periodic lattice, its halo as it is).
 // Otherwise W and H are the tile of a doubly periodic lattice of nx x ny inner
@@ -39,6 +44,7 @@ namespace tsmi {
 
 constexpr int kTileWavesMax = 8;     // waves per workgroup, at most
 constexpr int kTileCols = 2 * kWave; // columns of a tile
+constexpr int kTileImag = 2;         // MODE of imaginary time
 
 template <typename T>
 struct TileParams {
@@ -56,6 +62,13 @@ struct TileParams {
     T c_nl, c_lhy;
     double mag, mag_mid;             // |corr| of the last step and of the steps before it
     T dphi;                          // phase of the merged frame, added to every phase
+    // imaginary time, as StepParams; one partial sum per workgroup
+    const double *part_in;
+    const int *n_in;
+    double *part_out;
+    int *n_out;
+    double norm_target, dxdy;
+    int ix0, ix1, iy0, iy1;
 };
 
 // A cell of the reference tile whose halo exchange has not run: where its value
@@ -137,13 +150,15 @@ __device__ __forceinline__ void tile_ppass(Row<T, 2> &a, Row<T, 2> &b, const T (
 // EH: the strip reaches past the tile's left or right edge (per-lane pair
 // coefficients); EV: so do the wave's rows at the top or bottom (bit r + 1 of ok:
 // rows r and r + 1 of the wave are both inside the tile).
+// MODE: kTileImag is one step in imaginary time (form A).
 template <typename T, bool LHY, int MODE, int R, bool EH, bool EV>
 __device__ __forceinline__ void tile_steps(const TileParams<T> &p, Row<T, 2> (&s)[R], const T (&ph)[R][2],
                                            TileXch<T> &x, int w, int lane, int xl,
                                            unsigned ok) {
     static_assert(R % 2 == 0 && R >= 4, "row parities are fixed per register");
     typedef typename TileXch<T>::T2 T2;
-    constexpr int M = MODE < 0 ? 0 : MODE;
+    constexpr bool IMAG = MODE == kTileImag;
+    constexpr int M = MODE < 0 || IMAG ? 0 : MODE;
     const T kH = M == 0 ? p.tH : p.mH;
     HCoef<T, 2> hc = {};
     // a periodic lattice has no edge: every column far from one
@@ -153,8 +168,8 @@ __device__ __forceinline__ void tile_steps(const TileParams<T> &p, Row<T, 2> (&s
 
     auto hrow = [&](auto ss, Row<T, 2> &r, auto rr) {
         constexpr int PAR = (decltype(ss)::value + decltype(rr)::value) & 1;
-        if constexpr (EH) hpass<PAR, false>(r, hc);
-        else hpass_fast<PAR, false, M>(r, kH);
+        if constexpr (EH) hpass<PAR, IMAG>(r, hc);
+        else hpass_fast<PAR, IMAG, M>(r, kH);
     };
     // the vertical pass V(S), factors (m, t) in the scaled form FM (-1: both
     // factors) and un for unpaired cells; `first` has run on the border rows and
@@ -182,9 +197,9 @@ __device__ __forceinline__ void tile_steps(const TileParams<T> &p, Row<T, 2> (&s
                 s[r + 1].re[c] *= un;
                 s[r + 1].im[c] *= un;
             } else if constexpr (FM < 0) {
-                rot<false>(m, t, s[r].re[c], s[r].im[c], s[r + 1].re[c], s[r + 1].im[c]);
+                rot<IMAG>(m, t, s[r].re[c], s[r].im[c], s[r + 1].re[c], s[r + 1].im[c]);
             } else {
-                fpair<false, FM>(FM == 0 ? t : m, s[r].re[c], s[r].im[c], s[r + 1].re[c], s[r + 1].im[c]);
+                fpair<IMAG, FM>(FM == 0 ? t : m, s[r].re[c], s[r].im[c], s[r + 1].re[c], s[r + 1].im[c]);
             }
         };
 #pragma unroll
@@ -196,22 +211,22 @@ __device__ __forceinline__ void tile_steps(const TileParams<T> &p, Row<T, 2> (&s
             f.re[CX] *= un;
             f.im[CX] *= un;
         } else if constexpr (FM < 0) {
-            rot_q<false>(m, t, up[0], up[1], f.re[CX], f.im[CX]);
+            rot_q<IMAG>(m, t, up[0], up[1], f.re[CX], f.im[CX]);
         } else {
-            fpair_q<false, FM>(FM == 0 ? t : m, up[0], up[1], f.re[CX], f.im[CX]);
+            fpair_q<IMAG, FM>(FM == 0 ? t : m, up[0], up[1], f.re[CX], f.im[CX]);
         }
         if (EV && __builtin_expect(!(ok >> R & 1u), 0)) {
             l.re[CX] *= un;
             l.im[CX] *= un;
         } else if constexpr (FM < 0) {
-            rot_p<false>(m, t, l.re[CX], l.im[CX], dn[0], dn[1]);
+            rot_p<IMAG>(m, t, l.re[CX], l.im[CX], dn[0], dn[1]);
         } else {
-            fpair_p<false, FM>(FM == 0 ? t : m, l.re[CX], l.im[CX], dn[0], dn[1]);
+            fpair_p<IMAG, FM>(FM == 0 ? t : m, l.re[CX], l.im[CX], dn[0], dn[1]);
         }
     };
     using I0 = std::integral_constant<int, 0>;
     using I1 = std::integral_constant<int, 1>;
-    using IM = std::integral_constant<int, MODE>;
+    using IM = std::integral_constant<int, IMAG ? 0 : MODE>;
     auto h_border = [&](auto ss) {
         hrow(ss, s[0], I0());
         hrow(ss, s[R - 1], I1());                    // R - 1 is odd
@@ -233,16 +248,16 @@ __device__ __forceinline__ void tile_steps(const TileParams<T> &p, Row<T, 2> (&s
         h_border(I1());
         h_rest(I1());
         // the potential pass, border rows first
-        tile_ppass<T, LHY>(s[0], s[R - 1], ph[0], ph[R - 1], p.c_nl, p.c_lhy, mag);
+        tile_ppass<T, LHY, IMAG>(s[0], s[R - 1], ph[0], ph[R - 1], p.c_nl, p.c_lhy, mag);
         h_border(I1());
         vpass(I1(), IM(), p.mV, p.tV, p.unV, [&] {
 #pragma unroll
             for (int r = 1; r + 1 < R; r += 2)
-                tile_ppass<T, LHY>(s[r], s[r + 1], ph[r], ph[r + 1], p.c_nl, p.c_lhy, mag);
+                tile_ppass<T, LHY, IMAG>(s[r], s[r + 1], ph[r], ph[r + 1], p.c_nl, p.c_lhy, mag);
             h_rest(I1());
         });
         h_border(I0());
-        if (last) break;
+        if (IMAG || last) break;
         if (p.mode2 == 0)
             vpass(I0(), I0(), p.m2, p.t2, p.un2, [&] { h_rest(I0()); });
         else
@@ -311,6 +326,15 @@ __device__ __forceinline__ void tile_group(const TileParams<T> &p, int tile, Til
     };
     if (p.seam) load(std::true_type());
     else load(std::false_type());
+    if constexpr (MODE == kTileImag) {
+        // the pending renormalisation, as step_kernel applies it
+        if (p.part_in) {
+            const int n = __builtin_amdgcn_readfirstlane(*p.n_in);
+            const double inv = 1.0 / renorm_divisor(p.part_in, n, p.dxdy, p.norm_target, lane);
+#pragma unroll
+            for (int r = 0; r < R; ++r) scale_row<T, 2>(s[r], inv);
+        }
+    }
 #pragma unroll
     for (int r = 0; r < R; ++r) {
         ph[r][0] += p.dphi;
@@ -342,6 +366,38 @@ __device__ __forceinline__ void tile_group(const TileParams<T> &p, int tile, Til
             own && y >= y_lo && y < y_hi ? (unsigned)xl * (unsigned)sizeof(T) + (unsigned)y * row_bytes : kOffNone;
         buf_store<T, 2>(r_out_re, off, 0u, s[r].re);
         buf_store<T, 2>(r_out_im, off, 0u, s[r].im);
+    }
+    if constexpr (MODE == kTileImag) {
+        double q = 0.0, e = 0.0;
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            const int y = y0 + r;
+            if (!(y >= y_lo && y < y_hi && y >= p.iy0 && y < p.iy1)) continue;   // uniform
+            double v = 0.0;
+#pragma unroll
+            for (int k = 0; k < 2; ++k) {
+                const double re = s[r].re[k], im = s[r].im[k];
+                v += own && xl + k >= p.ix0 && xl + k < p.ix1 ? re * re + im * im : 0.0;
+            }
+            const double t = q + v;
+            e += fabs(q) >= fabs(v) ? (q - t) + v : (v - t) + q;
+            q = t;
+        }
+        double t = q + e;
+        for (int o = kWave / 2; o > 0; o >>= 1) t += __shfl_xor(t, o, kWave);
+        __shared__ double red[kTileWavesMax];
+        if (lane == 0) red[w] = t;
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            double a = 0.0, c = 0.0;
+            for (int i = 0; i < nw; ++i) {
+                const double u = a + red[i];
+                c += fabs(a) >= fabs(red[i]) ? (a - u) + red[i] : (red[i] - u) + a;
+                a = u;
+            }
+            p.part_out[tile] = a + c;
+            if (tile == 0) *p.n_out = gridDim.x;
+        }
     }
 }
 

@@ -199,7 +199,7 @@ int upload_state(tsmi_ctx *c, const double *re, const double *im) {
 const double *pending_div(tsmi_ctx *c) {
     if (!c->d.imag_time || !c->div_pending) return nullptr;
     hipLaunchKernelGGL(divisor_kernel<>, dim3(1), dim3(kWave), 0, c->stream,
-                       (const double *)(c->partials + (size_t)c->div_slot * c->n_waves),
+                       (const double *)(c->partials + (size_t)c->div_slot * c->part_cap),
                        (const int *)(c->part_n + c->div_slot), c->d.delta_x * c->d.delta_y, c->d.norm_target, c->div);
     return c->div;
 }
@@ -476,10 +476,9 @@ int launch_step(tsmi_ctx *c, int exchange) {
     p.c_nl = (T)c->c_nl_s; p.c_lhy = (T)c->c_lhy_s;
     p.ix0 = c->ix0; p.ix1 = c->ix1; p.iy0 = c->iy0; p.iy1 = c->iy1;
     if (IMAG) {
-        const size_t nw = (size_t)c->n_waves;
-        p.part_in = c->div_pending ? c->partials + (size_t)c->div_slot * nw : nullptr;
+        p.part_in = c->div_pending ? c->partials + (size_t)c->div_slot * c->part_cap : nullptr;
         p.n_in = c->part_n + c->div_slot;
-        p.part_out = c->partials + (size_t)(1 - c->div_slot) * nw;
+        p.part_out = c->partials + (size_t)(1 - c->div_slot) * c->part_cap;
         p.n_out = c->part_n + (1 - c->div_slot);
         p.norm_target = c->d.norm_target;
         p.dxdy = c->d.delta_x * c->d.delta_y;
@@ -1001,13 +1000,14 @@ int tsmi_create(const tsmi_desc *desc, tsmi_ctx **out) {
     const size_t pb = plane_bytes(c);
     const size_t pd = (size_t)c->pitch * (size_t)c->Hd * sizeof(double);
     c->obs_blocks = std::min(kObsBlocksMax, c->H);
+    c->part_cap = std::max(c->n_waves, d.imag_time ? tile_blocks(c) : 0);
     struct { void **p; size_t n; } allocs[] = {
         {&c->psi_base[0][0], pb}, {&c->psi_base[0][1], pb}, {&c->psi_base[1][0], pb}, {&c->psi_base[1][1], pb},
         {&c->e_base[0], pb}, {&c->e_base[1], pb}, {&c->e8[0], halo8 ? pb : 0}, {&c->e8[1], halo8 ? pb : 0},
         {&c->ph_base, pb}, {&c->ph8, halo8 ? pb : 0}, {(void **)&c->flag, 64},
         {(void **)&c->v_base, pd},
         {(void **)&c->xc, (size_t)c->W * sizeof(double)}, {(void **)&c->yc, (size_t)c->H * sizeof(double)},
-        {(void **)&c->div, 2 * sizeof(double)}, {(void **)&c->partials, 2 * (size_t)c->n_waves * sizeof(double)},
+        {(void **)&c->div, 2 * sizeof(double)}, {(void **)&c->partials, 2 * (size_t)c->part_cap * sizeof(double)},
         {(void **)&c->part_n, 64}, {(void **)&c->obs_partials, (size_t)kObsBlocksMax * OBS_COUNT * sizeof(double)},
         {(void **)&c->obs_out, kObsOut * sizeof(double)},
     };
