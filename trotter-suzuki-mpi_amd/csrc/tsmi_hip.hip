@@ -218,28 +218,52 @@ int download_state(tsmi_ctx *c, size_t stride, size_t x, size_t y, size_t w, siz
     return TSMI_OK;
 }
 
-// W x H FP64 (row stride W) -> pitched plane of T, rounding once.
-template <typename T>
-__global__ void import_plane(const double *__restrict__ src, T *__restrict__ dst, int W, int H, int pitch) {
-    const long n = (long)W * H;
-    for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x) {
-        const long y = i / W, x = i - y * W;
-        dst[y * pitch + x] = (T)src[i];
+// Tile-wide kernels between W x H FP64 arrays (row stride W) and pitched planes:
+// a workgroup takes 256 columns of a row at a time, so a cell's row and column
+// cost no division, and both planes of a state go in one launch (50 steps of 64^2
+// with import and export 150 -> 146 us).
+constexpr int kCols = 256;
+
+template <typename F>
+__device__ __forceinline__ void for_cells(int W, int H, F &&f) {
+    const unsigned chunks = ((unsigned)W + kCols - 1) / kCols;
+    const unsigned items = chunks * (unsigned)H;   // a plane this size is far beyond any memory
+    for (unsigned i = blockIdx.x; i < items; i += gridDim.x) {
+        const unsigned y = i / chunks, x = (i - y * chunks) * kCols + threadIdx.x;
+        if (x < (unsigned)W) f((long)y, (long)x);
     }
 }
 
-// pitched plane of T -> W x H FP64, divided by *div when given
+int cell_blocks(int W, int H) {
+    return (int)std::min<long long>(4096, (long long)((W + kCols - 1) / kCols) * H);
+}
+
+// FP64 -> T, rounding once
 template <typename T>
-__global__ void export_plane(const T *__restrict__ src, double *__restrict__ dst, int W, int H, int pitch,
-                             const double *__restrict__ div) {
-    const long n = (long)W * H;
+__global__ void __launch_bounds__(kCols) import_planes(const double *__restrict__ sre, const double *__restrict__ sim,
+                                                       T *__restrict__ dre, T *__restrict__ dim, int W, int H, int pitch) {
+    for_cells(W, H, [&](long y, long x) {
+        const double re = sre[y * W + x], im = sim[y * W + x];
+        dre[y * pitch + x] = (T)re;
+        dim[y * pitch + x] = (T)im;
+    });
+}
+
+// T -> FP64, divided by *div when given; either destination may be null
+template <typename T>
+__global__ void __launch_bounds__(kCols) export_planes(const T *__restrict__ sre, const T *__restrict__ sim,
+                                                       double *__restrict__ dre, double *__restrict__ dim, int W, int H,
+                                                       int pitch, const double *__restrict__ div) {
     const double d = div ? *div : 1.0;
-    for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x) {
-        const long y = i / W, x = i - y * W;
-        double v = (double)src[y * pitch + x];
-        if (div) v /= d;
-        dst[i] = v;
-    }
+    for_cells(W, H, [&](long y, long x) {
+        double re = (double)sre[y * pitch + x], im = (double)sim[y * pitch + x];
+        if (div) {
+            re /= d;
+            im /= d;
+        }
+        if (dre) dre[y * W + x] = re;
+        if (dim) dim[y * W + x] = im;
+    });
 }
 
 // E table of the step: E*corr computed in FP64, each component then rounded
@@ -249,14 +273,12 @@ __global__ void export_plane(const T *__restrict__ src, double *__restrict__ dst
 // (real time), lambda = -ln(E corr) when E > 0 (imaginary time); a cell without
 // that form sets *bad.
 template <typename T>
-__global__ void import_exp(const double *__restrict__ sre, const double *__restrict__ sim, double cr, double ci,
+__global__ void __launch_bounds__(kCols) import_exp(const double *__restrict__ sre, const double *__restrict__ sim, double cr, double ci,
                            T *__restrict__ dre, T *__restrict__ dim, T *__restrict__ dph, unsigned *bad, int W,
                            int H, int pitch) {
-    const long n = (long)W * H;
     bool ok = true;
-    for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x) {
-        const long y = i / W, x = i - y * W;
-        const double er = sre[i], ei = sim ? sim[i] : 0.0;
+    for_cells(W, H, [&](long y, long x) {
+        const double er = sre[y * W + x], ei = sim ? sim[y * W + x] : 0.0;
         const double zr = er * cr - ei * ci, zi = er * ci + ei * cr;
         dre[y * pitch + x] = (T)zr;
         dim[y * pitch + x] = (T)zi;
@@ -269,7 +291,7 @@ __global__ void import_exp(const double *__restrict__ sre, const double *__restr
             ph = zr > 0.0 ? -log(zr) : 0.0;
         }
         dph[y * pitch + x] = (T)ph;
-    }
+    });
     if (!ok) atomicOr(bad, 1u);
 }
 
@@ -278,10 +300,10 @@ __global__ void import_exp(const double *__restrict__ sre, const double *__restr
 int launch_import_exp(tsmi_ctx *c, const double *re, const double *im) {
     TSMI_HIP(hipMemsetAsync(c->flag, 0, sizeof(unsigned), c->stream));
     if (c->esz == 4)
-        hipLaunchKernelGGL(import_exp<float>, dim3(2048), dim3(256), 0, c->stream, re, im, c->corr_re, c->corr_im,
+        hipLaunchKernelGGL(import_exp<float>, dim3(cell_blocks(c->W, c->H)), dim3(kCols), 0, c->stream, re, im, c->corr_re, c->corr_im,
                            (float *)c->e_re, (float *)c->e_im, (float *)c->ph, c->flag, c->W, c->H, c->pitch);
     else
-        hipLaunchKernelGGL(import_exp<double>, dim3(2048), dim3(256), 0, c->stream, re, im, c->corr_re, c->corr_im,
+        hipLaunchKernelGGL(import_exp<double>, dim3(cell_blocks(c->W, c->H)), dim3(kCols), 0, c->stream, re, im, c->corr_re, c->corr_im,
                            (double *)c->e_re, (double *)c->e_im, (double *)c->ph, c->flag, c->W, c->H, c->pitch);
     TSMI_HIP(hipGetLastError());
     unsigned bad = 1;
@@ -296,15 +318,13 @@ int launch_import_exp(tsmi_ctx *c, const double *re, const double *im) {
 // it (src/solver.cpp:74-109), times the frame factor, rounded once; the raw V
 // goes to the pitched FP64 plane used by the energies.
 template <typename T>
-__global__ void exp_from_potential(const double *__restrict__ v, double dt, int imag, double cr, double ci,
+__global__ void __launch_bounds__(kCols) exp_from_potential(const double *__restrict__ v, double dt, int imag, double cr, double ci,
                                    T *__restrict__ dre, T *__restrict__ dim, T *__restrict__ dph,
                                    double *__restrict__ vout, int W, int H, int pitch) {
-    const long n = (long)W * H;
     // one-plane form: phi = dt V - arg(corr), lambda = dt V - ln(corr)
     const double shift = imag ? log(cr) : atan2(ci, cr);
-    for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x) {
-        const long y = i / W, x = i - y * W;
-        const double vi = v[i];
+    for_cells(W, H, [&](long y, long x) {
+        const double vi = v[y * W + x];
         double er, ei;
         if (imag) {
             er = exp(-dt * vi);
@@ -316,15 +336,31 @@ __global__ void exp_from_potential(const double *__restrict__ v, double dt, int 
         dim[y * pitch + x] = (T)(er * ci + ei * cr);
         dph[y * pitch + x] = (T)(dt * vi - shift);
         vout[y * pitch + x] = vi;
-    }
+    });
 }
 
-int import_device(tsmi_ctx *c, void *dst, const double *src) {
-    const int blocks = 2048;
+int import_device(tsmi_ctx *c, void *dre, void *dim, const double *re, const double *im) {
+    const dim3 grid(cell_blocks(c->W, c->H));
     if (c->esz == 8)
-        hipLaunchKernelGGL(import_plane<double>, dim3(blocks), dim3(256), 0, c->stream, src, (double *)dst, c->W, c->H, c->pitch);
+        hipLaunchKernelGGL(import_planes<double>, grid, dim3(kCols), 0, c->stream, re, im, (double *)dre, (double *)dim,
+                           c->W, c->H, c->pitch);
     else
-        hipLaunchKernelGGL(import_plane<float>, dim3(blocks), dim3(256), 0, c->stream, src, (float *)dst, c->W, c->H, c->pitch);
+        hipLaunchKernelGGL(import_planes<float>, grid, dim3(kCols), 0, c->stream, re, im, (float *)dre, (float *)dim, c->W,
+                           c->H, c->pitch);
+    TSMI_HIP(hipGetLastError());
+    return TSMI_OK;
+}
+
+// pitched planes of the context precision -> W x H FP64 on the device (either may
+// be null), divided by *div when given
+int export_device(tsmi_ctx *c, const void *sre, const void *sim, double *dre, double *dim, const double *div) {
+    const dim3 grid(cell_blocks(c->W, c->H));
+    if (c->esz == 8)
+        hipLaunchKernelGGL(export_planes<double>, grid, dim3(kCols), 0, c->stream, (const double *)sre,
+                           (const double *)sim, dre, dim, c->W, c->H, c->pitch, div);
+    else
+        hipLaunchKernelGGL(export_planes<float>, grid, dim3(kCols), 0, c->stream, (const float *)sre, (const float *)sim,
+                           dre, dim, c->W, c->H, c->pitch, div);
     TSMI_HIP(hipGetLastError());
     return TSMI_OK;
 }
@@ -631,7 +667,9 @@ int evolve_steps(tsmi_ctx *c, int n, bool exchange_last = false) {
 // The fused passes read E over the whole 8-wide halo: the reference-tile table
 // with every halo cell replaced by its wrapped inner cell.
 int wrap_exp(tsmi_ctx *c) {
-    if (!c->halo8) return TSMI_OK;
+    // tile passes read the reference tile's table (whether they run depends on the
+    // descriptor and the table's form alone)
+    if (!c->halo8 || tile_runs(c)) return TSMI_OK;
     const size_t pb = plane_bytes(c);
     TSMI_HIP(hipMemcpyAsync(c->e8[0], c->e_base[0], pb, hipMemcpyDeviceToDevice, c->stream));
     TSMI_HIP(hipMemcpyAsync(c->e8[1], c->e_base[1], pb, hipMemcpyDeviceToDevice, c->stream));
@@ -740,8 +778,7 @@ int reverse_sweep(tsmi_ctx *c, const double *g_re, const double *g_im, void **g0
     // rows are padded; the padding of every plane must read as zero
     TSMI_HIP(hipMemsetAsync(c->adj, 0, 8 * pb, c->stream));
     TSMI_HIP(hipMemsetAsync(c->grad, 0, pd, c->stream));
-    int st = import_device(c, L[0][0], g_re);
-    if (!st) st = import_device(c, L[0][1], g_im);
+    int st = import_device(c, L[0][0], L[0][1], g_re, g_im);
     if (st) return st;
     const void *s_re = c->psi_re[c->cur], *s_im = c->psi_im[c->cur];
     const bool tiles = adjoint_tiles_run(c);   // passes that read through the periodic wrap
@@ -804,19 +841,6 @@ int reverse_sweep(tsmi_ctx *c, const double *g_re, const double *g_im, void **g0
     }
     *g0_re = L[k][0];
     *g0_im = L[k][1];
-    return TSMI_OK;
-}
-
-// pitched plane of the context precision -> W x H FP64 on the device
-int export_device(tsmi_ctx *c, const void *src, double *dst) {
-    const int blocks = 2048;
-    if (c->esz == 8)
-        hipLaunchKernelGGL(export_plane<double>, dim3(blocks), dim3(256), 0, c->stream, (const double *)src, dst,
-                           c->W, c->H, c->pitch, (const double *)nullptr);
-    else
-        hipLaunchKernelGGL(export_plane<float>, dim3(blocks), dim3(256), 0, c->stream, (const float *)src, dst,
-                           c->W, c->H, c->pitch, (const double *)nullptr);
-    TSMI_HIP(hipGetLastError());
     return TSMI_OK;
 }
 
@@ -1067,9 +1091,7 @@ int tsmi_set_state_complex(tsmi_ctx *c, const double *psi) {
 int tsmi_set_state_device(tsmi_ctx *c, const double *re, const double *im) {
     if (c) c->ck_valid = false;
     if (!c || !re || !im) return fail(TSMI_E_INVALID, "tsmi_set_state_device: null argument");
-    int st = import_device(c, c->psi_re[c->cur], re);
-    if (!st) st = import_device(c, c->psi_im[c->cur], im);
-    if (st) return st;
+    if (int st = import_device(c, c->psi_re[c->cur], c->psi_im[c->cur], re, im)) return st;
     c->has_state = true;
     c->div_pending = false;
     return TSMI_OK;
@@ -1092,10 +1114,10 @@ int tsmi_set_potential_exp_device(tsmi_ctx *c, const double *v) {
     const double dt = c->d.delta_t;
     const int imag = c->d.imag_time ? 1 : 0;
     if (c->esz == 4)
-        hipLaunchKernelGGL(exp_from_potential<float>, dim3(2048), dim3(256), 0, c->stream, v, dt, imag, c->corr_re,
+        hipLaunchKernelGGL(exp_from_potential<float>, dim3(cell_blocks(c->W, c->H)), dim3(kCols), 0, c->stream, v, dt, imag, c->corr_re,
                            c->corr_im, (float *)c->e_re, (float *)c->e_im, (float *)c->ph, c->v, c->W, c->H, c->pitch);
     else
-        hipLaunchKernelGGL(exp_from_potential<double>, dim3(2048), dim3(256), 0, c->stream, v, dt, imag, c->corr_re,
+        hipLaunchKernelGGL(exp_from_potential<double>, dim3(cell_blocks(c->W, c->H)), dim3(kCols), 0, c->stream, v, dt, imag, c->corr_re,
                            c->corr_im, (double *)c->e_re, (double *)c->e_im, (double *)c->ph, c->v, c->W, c->H,
                            c->pitch);
     TSMI_HIP(hipGetLastError());
@@ -1119,19 +1141,7 @@ int tsmi_get_state_device(tsmi_ctx *c, double *re, double *im) {
     if (!c->has_state) return fail(TSMI_E_INVALID, "tsmi_get_state_device: no state");
     const double *div = pending_div(c);
     if (div) TSMI_HIP(hipGetLastError());
-    const int blocks = 2048;
-    for (int k = 0; k < 2; ++k) {
-        const void *src = k ? c->psi_im[c->cur] : c->psi_re[c->cur];
-        double *dst = k ? im : re;
-        if (c->esz == 8)
-            hipLaunchKernelGGL(export_plane<double>, dim3(blocks), dim3(256), 0, c->stream, (const double *)src, dst,
-                               c->W, c->H, c->pitch, div);
-        else
-            hipLaunchKernelGGL(export_plane<float>, dim3(blocks), dim3(256), 0, c->stream, (const float *)src, dst,
-                               c->W, c->H, c->pitch, div);
-        TSMI_HIP(hipGetLastError());
-    }
-    return TSMI_OK;
+    return export_device(c, c->psi_re[c->cur], c->psi_im[c->cur], re, im, div);
 }
 
 int tsmi_set_exp_potential(tsmi_ctx *c, const double *e_re, const double *e_im) {
@@ -1247,8 +1257,7 @@ int tsmi_adjoint_device(tsmi_ctx *c, const double *g_re, const double *g_im, dou
     if (st) return st;
     TSMI_HIP(hipMemcpy2DAsync(grad_v, (size_t)c->W * 8, c->grad, (size_t)c->pitch * 8, (size_t)c->W * 8, c->H,
                               hipMemcpyDeviceToDevice, c->stream));
-    if (g0_re) st = export_device(c, l_re, g0_re);
-    if (!st && g0_im) st = export_device(c, l_im, g0_im);
+    if (g0_re || g0_im) st = export_device(c, l_re, l_im, g0_re, g0_im, nullptr);
     return st;
 }
 
