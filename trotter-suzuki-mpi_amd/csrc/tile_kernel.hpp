@@ -107,12 +107,12 @@ __device__ __forceinline__ void seam_load(const SeamTile &q, __amdgpu_buffer_rsr
     }
 }
 
-template <typename T>
+template <typename T, int NW>
 struct TileXch {
     typedef T __attribute__((ext_vector_type(2))) T2;
     // [buffer][first / last row of a wave][wave + 1][lane]; the slots of waves -1
     // and NW hold zeros (no row there)
-    T2 v[2][2][kTileWavesMax + 2][kWave];
+    T2 v[2][2][NW + 2][kWave];
 };
 
 // The potential pass of two rows: one wave-uniform test and straight-line code
@@ -151,12 +151,12 @@ __device__ __forceinline__ void tile_ppass(Row<T, 2> &a, Row<T, 2> &b, const T (
 // coefficients); EV: so do the wave's rows at the top or bottom (bit r + 1 of ok:
 // rows r and r + 1 of the wave are both inside the tile).
 // MODE: kTileImag is one step in imaginary time (form A).
-template <typename T, bool LHY, int MODE, int R, bool EH, bool EV>
+template <typename T, bool LHY, int MODE, int R, bool EH, bool EV, int NW>
 __device__ __forceinline__ void tile_steps(const TileParams<T> &p, Row<T, 2> (&s)[R], const T (&ph)[R][2],
-                                           TileXch<T> &x, int w, int lane, int xl,
+                                           TileXch<T, NW> &x, int w, int lane, int xl,
                                            unsigned ok) {
     static_assert(R % 2 == 0 && R >= 4, "row parities are fixed per register");
-    typedef typename TileXch<T>::T2 T2;
+    typedef typename TileXch<T, NW>::T2 T2;
     constexpr bool IMAG = MODE == kTileImag;
     constexpr int M = MODE < 0 || IMAG ? 0 : MODE;
     const T kH = M == 0 ? p.tH : p.mH;
@@ -266,9 +266,9 @@ __device__ __forceinline__ void tile_steps(const TileParams<T> &p, Row<T, 2> (&s
     vpass(I0(), IM(), p.mV, p.tV, p.unV, [&] { h_rest(I0()); });
 }
 
-// Tile `tile` of the pass p by a workgroup of nw waves.
-template <typename T, bool LHY, int MODE, int R>
-__device__ __forceinline__ void tile_group(const TileParams<T> &p, int tile, TileXch<T> &xch) {
+// Tile `tile` of the pass p by a workgroup of nw waves, at most NW.
+template <typename T, bool LHY, int MODE, int R, int NW>
+__device__ __forceinline__ void tile_group(const TileParams<T> &p, int tile, TileXch<T, NW> &xch) {
     const int lane = threadIdx.x & (kWave - 1);
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     const int nw = blockDim.x / kWave;
@@ -283,7 +283,7 @@ __device__ __forceinline__ void tile_group(const TileParams<T> &p, int tile, Til
 
     // slots of the rows above the first and below the last wave
     if (w == 0) {
-        typename TileXch<T>::T2 z = {T(0), T(0)};
+        typename TileXch<T, NW>::T2 z = {T(0), T(0)};
         xch.v[0][1][0][lane] = xch.v[1][1][0][lane] = z;
         xch.v[0][0][nw + 1][lane] = xch.v[1][0][nw + 1][lane] = z;
     }
@@ -309,14 +309,14 @@ __device__ __forceinline__ void tile_group(const TileParams<T> &p, int tile, Til
     T ph[R][2];
     auto load = [&](auto seam) {
         const SeamTile q = {p.W, p.H, p.px, p.py};
+        int ys = wrap ? mod(y0 - kApron, p.ny) : y0;              // one division, then row by row
 #pragma unroll
         for (int r = 0; r < R; ++r) {
-            const int y = y0 + r;
-            const bool in = wrap || (y >= 0 && y < p.H);
-            const int ys = wrap ? kApron + mod(y - kApron, p.ny) : y;
-            const unsigned off = in ? v_ld + (unsigned)ys * row_bytes : kOffNone;
+            const bool in = wrap || (ys >= 0 && ys < p.H);
+            const unsigned off = in ? v_ld + (unsigned)(wrap ? ys + kApron : ys) * row_bytes : kOffNone;
+            ys = wrap && ys + 1 == p.ny ? 0 : ys + 1;
             if constexpr (decltype(seam)::value) {
-                seam_load<T>(q, r_in_re, r_in_im, xl, y, row_bytes, s[r]);
+                seam_load<T>(q, r_in_re, r_in_im, xl, y0 + r, row_bytes, s[r]);
             } else {
                 buf_load<T, 2>(r_in_re, off, 0u, s[r].re);
                 buf_load<T, 2>(r_in_im, off, 0u, s[r].im);
@@ -349,11 +349,11 @@ __device__ __forceinline__ void tile_group(const TileParams<T> &p, int tile, Til
     for (int r = -1; r < R; ++r)
         if (wrap || (y0 + r >= 0 && y0 + r + 1 < p.H)) ok |= 1u << (r + 1);
     if constexpr (MODE < 0) {
-        tile_steps<T, LHY, MODE, R, true, true>(p, s, ph, xch, w, lane, xl, ok);
+        tile_steps<T, LHY, MODE, R, true, true, NW>(p, s, ph, xch, w, lane, xl, ok);
     } else {
-        if (ev) tile_steps<T, LHY, MODE, R, true, true>(p, s, ph, xch, w, lane, xl, ok);
-        else if (eh) tile_steps<T, LHY, MODE, R, true, false>(p, s, ph, xch, w, lane, xl, ok);
-        else tile_steps<T, LHY, MODE, R, false, false>(p, s, ph, xch, w, lane, xl, ok);
+        if (ev) tile_steps<T, LHY, MODE, R, true, true, NW>(p, s, ph, xch, w, lane, xl, ok);
+        else if (eh) tile_steps<T, LHY, MODE, R, true, false, NW>(p, s, ph, xch, w, lane, xl, ok);
+        else tile_steps<T, LHY, MODE, R, false, false, NW>(p, s, ph, xch, w, lane, xl, ok);
     }
 
     // columns in [W, pitch) are padding and are written back as the zeros they hold
@@ -385,7 +385,7 @@ __device__ __forceinline__ void tile_group(const TileParams<T> &p, int tile, Til
         }
         double t = q + e;
         for (int o = kWave / 2; o > 0; o >>= 1) t += __shfl_xor(t, o, kWave);
-        __shared__ double red[kTileWavesMax];
+        __shared__ double red[NW];
         if (lane == 0) red[w] = t;
         __syncthreads();
         if (threadIdx.x == 0) {
@@ -401,21 +401,21 @@ __device__ __forceinline__ void tile_group(const TileParams<T> &p, int tile, Til
     }
 }
 
-template <typename T, bool LHY, int MODE, int R>
-__global__ void __launch_bounds__(kTileWavesMax * kWave) tile_kernel(TileParams<T> p) {
-    __shared__ TileXch<T> xch;
-    tile_group<T, LHY, MODE, R>(p, blockIdx.x, xch);
+template <typename T, bool LHY, int MODE, int R, int NW>
+__global__ void __launch_bounds__(NW * kWave) tile_kernel(TileParams<T> p) {
+    __shared__ TileXch<T, NW> xch;
+    tile_group<T, LHY, MODE, R, NW>(p, blockIdx.x, xch);
 }
 
 // One pass of many lattices: a workgroup per item (lattice, tile).
-template <typename T, bool LHY, int MODE, int R>
-__global__ void __launch_bounds__(kTileWavesMax * kWave) tile_batch_kernel(const TileParams<T> *__restrict__ params,
+template <typename T, bool LHY, int MODE, int R, int NW>
+__global__ void __launch_bounds__(NW * kWave) tile_batch_kernel(const TileParams<T> *__restrict__ params,
                                                                            const int2 *__restrict__ items) {
-    __shared__ TileXch<T> xch;
+    __shared__ TileXch<T, NW> xch;
     const int2 it = items[blockIdx.x];
     const int i = __builtin_amdgcn_readfirstlane(it.x), tile = __builtin_amdgcn_readfirstlane(it.y);
     const TileParams<T> p = params[i];
-    tile_group<T, LHY, MODE, R>(p, tile, xch);
+    tile_group<T, LHY, MODE, R, NW>(p, tile, xch);
 }
 
 }  // namespace tsmi

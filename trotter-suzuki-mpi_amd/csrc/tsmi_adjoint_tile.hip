@@ -20,14 +20,18 @@ namespace {
 // Modelled us of a row of both fields, and planes moved per launch: two states in
 // and out, E, and the FP64 gradient in and out.
 TwoFieldCost cost(const tsmi_ctx *c) {
-    return c->esz == 4 ? TwoFieldCost{0.27, 14} : TwoFieldCost{0.40, 12};
+    const bool wide = c->c_nl == 0.0 && c->c_lhy == 0.0 && c->mode >= 0;   // 120 VGPRs; the others need more
+    return c->esz == 4 ? TwoFieldCost{0.27, 14, wide} : TwoFieldCost{0.40, 12, false};
 }
 
 template <typename T, bool NL, int R, int NW, bool WRAP>
 int launch_kernel(tsmi_ctx *c, const AdjTileParams<T> &q, int blocks) {
     const dim3 grid(blocks), block(NW * kWave);
     // tiles with an edge, 8 FP64 waves: as in tsmi_pair_tile.hip
-    if constexpr (!WRAP && sizeof(T) == 8 && NW == 8) {
+    if constexpr (NW == 16) {
+        if (c->mode == 0) hipLaunchKernelGGL((adj_tile_kernel<T, NL, 0, R, NW, WRAP>), grid, block, 0, c->stream, q);
+        else hipLaunchKernelGGL((adj_tile_kernel<T, NL, 1, R, NW, WRAP>), grid, block, 0, c->stream, q);
+    } else if constexpr (!WRAP && sizeof(T) == 8 && NW == 8) {
         hipLaunchKernelGGL((adj_tile_kernel<T, NL, -1, R, NW, WRAP>), grid, block, 0, c->stream, q);
     } else {
         if (c->mode == 0) hipLaunchKernelGGL((adj_tile_kernel<T, NL, 0, R, NW, WRAP>), grid, block, 0, c->stream, q);
@@ -42,6 +46,9 @@ int launch_kernel(tsmi_ctx *c, const AdjTileParams<T> &q, int blocks) {
 template <typename T, bool NL, bool WRAP>
 int launch(tsmi_ctx *c, const AdjTileParams<T> &q, const TwoFieldPlan &g) {
     const int blocks = g.strips * g.segs;
+    if constexpr (sizeof(T) == 4 && !NL) {
+        if (g.nw == 16) return launch_kernel<T, NL, 4, 16, WRAP>(c, q, blocks);
+    }
     if constexpr (sizeof(T) == 4)
         return g.r == 4 ? launch_kernel<T, NL, 4, 8, WRAP>(c, q, blocks) : launch_kernel<T, NL, 8, 8, WRAP>(c, q, blocks);
     else

@@ -17,8 +17,13 @@ using namespace tsmi;
 
 namespace {
 
+// One scaled form for both components on both axes.
+bool one_form(const tsmi_pair *p) { return p->c[0]->mode == p->c[1]->mode && p->c[0]->mode >= 0; }
+
 // Modelled us of a row of both components, and planes moved per launch.
-TwoFieldCost cost(int esz) { return esz == 4 ? TwoFieldCost{0.27, 10} : TwoFieldCost{0.53, 10}; }
+TwoFieldCost cost(int esz, bool wide) {
+    return esz == 4 ? TwoFieldCost{0.27, 10, wide} : TwoFieldCost{0.53, 10, false};
+}
 
 template <typename T, bool IMAG, int R, int NW, bool WRAP>
 int launch_kernel(tsmi_pair *p, const PairTileParams<T> &q, const TwoFieldPlan &g) {
@@ -49,8 +54,24 @@ int launch(tsmi_pair *p, const PairTileParams<T> &q, const TwoFieldPlan &g) {
 
 template <typename T, bool IMAG>
 int launch_shape(tsmi_pair *p, const PairTileParams<T> &q, const TwoFieldPlan &g) {
-    if constexpr (sizeof(T) == 4) return g.r == 4 ? launch<T, IMAG, 4, 8>(p, q, g) : launch<T, IMAG, 8, 8>(p, q, g);
-    else return g.nw == 8 ? launch<T, IMAG, 4, 8>(p, q, g) : launch<T, IMAG, 4, 4>(p, q, g);
+    if constexpr (sizeof(T) == 4) {
+        if (g.nw == 16) {   // WRAP and one form only: the other kernels need more registers
+            hipStream_t s = p->c[0]->stream;
+            const dim3 grid(g.strips * g.segs), block(16 * kWave);
+            if constexpr (IMAG) {
+                hipLaunchKernelGGL((pair_tile_kernel<T, true, 0, 4, 16, true>), grid, block, 0, s, q);
+            } else {
+                if (p->c[0]->mode == 0)
+                    hipLaunchKernelGGL((pair_tile_kernel<T, false, 0, 4, 16, true>), grid, block, 0, s, q);
+                else
+                    hipLaunchKernelGGL((pair_tile_kernel<T, false, 1, 4, 16, true>), grid, block, 0, s, q);
+            }
+            const hipError_t e = hipGetLastError();
+            if (e != hipSuccess) return set_error(TSMI_E_HIP, std::string("pair_tile_kernel: ") + hipGetErrorString(e));
+            return TSMI_OK;
+        }
+        return g.r == 4 ? launch<T, IMAG, 4, 8>(p, q, g) : launch<T, IMAG, 8, 8>(p, q, g);
+    } else return g.nw == 8 ? launch<T, IMAG, 4, 8>(p, q, g) : launch<T, IMAG, 4, 4>(p, q, g);
 }
 
 // What is pending after an imaginary-time step in slot p->slot's partial sums,
@@ -101,7 +122,7 @@ int pass(tsmi_pair *p, int steps, How how, double var, bool rabi, bool first) {
     q.seam = how == kSeam;
     q.px = p->c[0]->d.periodic_x != 0; q.py = p->c[0]->d.periodic_y != 0;
     q.steps = steps;
-    const TwoFieldPlan g = two_field_plan(p->W, p->H, p->esz, steps, wrap, cost(p->esz));
+    const TwoFieldPlan g = two_field_plan(p->W, p->H, p->esz, steps, wrap, cost(p->esz, wrap && one_form(p)));
     if (g.r == 0) return set_error(TSMI_E_INVALID, "pair tile pass: no tile for this many steps");
     q.n_strips = g.strips; q.cols = g.cols; q.rows = g.rows;
     q.ix0 = p->ix0; q.ix1 = p->ix1; q.iy0 = p->iy0; q.iy1 = p->iy1;
@@ -158,8 +179,8 @@ int finish(tsmi_pair *p, double var, bool rabi) {
 namespace tsmi {
 
 int pair_tile_blocks(const tsmi_pair *p) {
-    const TwoFieldPlan a = two_field_plan(p->W, p->H, p->esz, 1, false, cost(p->esz)),
-                       b = two_field_plan(p->W, p->H, p->esz, 1, true, cost(p->esz));
+    const TwoFieldPlan a = two_field_plan(p->W, p->H, p->esz, 1, false, cost(p->esz, false)),
+                       b = two_field_plan(p->W, p->H, p->esz, 1, true, cost(p->esz, one_form(p)));
     return std::max(a.strips * a.segs, b.strips * b.segs);
 }
 
@@ -185,7 +206,8 @@ int pair_tile_evolve(tsmi_pair *p, int n, bool rabi) {
     int i = 0, st = TSMI_OK;
     // n steps from step i on; the call's last rotation is by 1/2 (src/solver.cpp:222-225)
     auto passes = [&](int m, How how) {
-        const int k = two_field_best_steps(p->W, p->H, p->esz, std::min(m, most), how == kWrap, cost(p->esz));
+        const int k = two_field_best_steps(p->W, p->H, p->esz, std::min(m, most), how == kWrap,
+                                           cost(p->esz, how == kWrap && one_form(p)));
         const int q = (m + k - 1) / k;
         for (int j = 0; j < q && !st; ++j) {
             const int s = m / q + (j < m % q ? 1 : 0);

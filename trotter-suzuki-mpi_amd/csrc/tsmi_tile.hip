@@ -36,7 +36,9 @@ TilePlan plan(const std::pair<int, int> *size, size_t count, int esz, int steps)
     const int *rr = esz == 4 ? kRows32 : kRows64;
     const double c_row = esz == 4 ? 0.17 : 0.27, x = 0.35, t0 = 5.0;
     for (int i = 0; i < 3; ++i)
-        for (int nw = 4; nw <= kTileWavesMax; nw += 4) {
+        for (int nw : {4, 8, 16}) {
+            // 16 waves: FP32 with 4 rows, the only instance of at most 128 VGPRs
+            if (nw == 16 && (esz != 4 || i != 0)) continue;
             TilePlan p;
             p.r = rr[i];
             p.nw = nw;
@@ -47,7 +49,7 @@ TilePlan plan(const std::pair<int, int> *size, size_t count, int esz, int steps)
                 tiles += (long)((size[j].first + cols - 1) / cols) * ((size[j].second + rows - 1) / rows);
             const double n = tiles / 256.0;                          // workgroups per compute unit
             const double per_cu = n < 6 ? std::ceil(n) : n + 0.5;    // ... on the busiest one
-            const double waves = std::min(per_cu * nw / 4.0, 3.0);   // waves per SIMD
+            const double waves = std::min(per_cu * nw / 4.0, nw == 16 ? 4.0 : 3.0);   // waves per SIMD
             p.us = t0 / steps + per_cu * nw * p.r / 4.0 * c_row * (1 + 0.6 / waves) + x;
             if (p.us < best.us) best = p;
         }
@@ -68,29 +70,35 @@ int best_steps(const std::pair<int, int> *size, size_t count, int esz, int most)
 }
 
 // Launches tile_kernel, or (items) tile_batch_kernel.
-template <typename T, bool LHY, int MODE, int R>
+template <typename T, bool LHY, int MODE, int R, int NW>
 void launch(const TilePlan &g, int blocks, const TileParams<T> *p, const int2 *items, hipStream_t s) {
-    if (items)
-        hipLaunchKernelGGL((tile_batch_kernel<T, LHY, MODE, R>), dim3(blocks), dim3(g.nw * kWave), 0, s, p, items);
-    else
-        hipLaunchKernelGGL((tile_kernel<T, LHY, MODE, R>), dim3(blocks), dim3(g.nw * kWave), 0, s, *p);
+    if constexpr (MODE != kTileImag)
+        if (items) {
+            hipLaunchKernelGGL((tile_batch_kernel<T, LHY, MODE, R, NW>), dim3(blocks), dim3(g.nw * kWave), 0, s, p, items);
+            return;
+        }
+    hipLaunchKernelGGL((tile_kernel<T, LHY, MODE, R, NW>), dim3(blocks), dim3(g.nw * kWave), 0, s, *p);
 }
 
-template <typename T, bool LHY, int R>
+template <typename T, bool LHY, int R, int NW>
 void launch_mode(int mode, const TilePlan &g, int blocks, const TileParams<T> *p, const int2 *items, hipStream_t s) {
-    if (mode == kTileImag)
-        hipLaunchKernelGGL((tile_kernel<T, LHY, kTileImag, R>), dim3(blocks), dim3(g.nw * kWave), 0, s, *p);
-    else if (mode == 0) launch<T, LHY, 0, R>(g, blocks, p, items, s);
-    else if (mode == 1) launch<T, LHY, 1, R>(g, blocks, p, items, s);
-    else launch<T, LHY, -1, R>(g, blocks, p, items, s);
+    if (mode == kTileImag) launch<T, LHY, kTileImag, R, NW>(g, blocks, p, items, s);
+    else if (mode == 0) launch<T, LHY, 0, R, NW>(g, blocks, p, items, s);
+    else if (mode == 1) launch<T, LHY, 1, R, NW>(g, blocks, p, items, s);
+    else launch<T, LHY, -1, R, NW>(g, blocks, p, items, s);
 }
 
 template <typename T, bool LHY>
 int launch_rows(int mode, const TilePlan &g, int blocks, const TileParams<T> *p, const int2 *items, hipStream_t s) {
     constexpr const int *rr = sizeof(T) == 4 ? kRows32 : kRows64;
-    if (g.r == rr[0]) launch_mode<T, LHY, rr[0]>(mode, g, blocks, p, items, s);
-    else if (g.r == rr[1]) launch_mode<T, LHY, rr[1]>(mode, g, blocks, p, items, s);
-    else launch_mode<T, LHY, rr[2]>(mode, g, blocks, p, items, s);
+    constexpr int N = kTileWavesMax;
+    if constexpr (sizeof(T) == 4) {
+        if (g.nw == 16) launch_mode<T, LHY, rr[0], 16>(mode, g, blocks, p, items, s);
+    }
+    if (g.nw == 16) (void)0;   // launched above
+    else if (g.r == rr[0]) launch_mode<T, LHY, rr[0], N>(mode, g, blocks, p, items, s);
+    else if (g.r == rr[1]) launch_mode<T, LHY, rr[1], N>(mode, g, blocks, p, items, s);
+    else launch_mode<T, LHY, rr[2], N>(mode, g, blocks, p, items, s);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return set_error(TSMI_E_HIP, std::string("tile_kernel: ") + hipGetErrorString(e));
     return TSMI_OK;

@@ -19,9 +19,11 @@ struct TwoFieldPlan {
 struct TwoFieldCost {
     double row;
     int planes;
+    bool wide;                       // 4 rows x 16 waves is compiled (FP32)
 };
 
-// The compiled instances: FP32 4 rows x 8 waves and 8 x 8, FP64 4 x 8 and 4 x 4.
+// The compiled instances: FP32 4 rows x 8 waves, 8 x 8 and (wide) 4 x 16, FP64 4 x 8
+// and 4 x 4.
 //
 // The shape of a pass of `steps` steps is the one with the least modelled time.  A
 // launch costs 4.5 us and its bytes (at 6.5 TB/s); a step costs each SIMD its rows
@@ -29,13 +31,16 @@ struct TwoFieldCost {
 // components of a periodic lattice in real time, us per step: 256^2 FP32 4 rows x
 // 8 waves 7.9, 5.6, 4.9 for 1, 2, 3 steps, 8 x 8 12.6, 9.3, 8.1; 1024^2 FP32 4 x 8
 // 13.9, 13.0, 19.2, 8 x 8 15.8, 12.2, 17.1 (3 steps: more than one workgroup per
-// compute unit); 512^2 FP64 4 x 8 10.9, 8.5, 12.7.
+// compute unit); 512^2 FP64 4 x 8 10.9, 8.5, 12.7.  4 rows x 16 waves, the tile of
+// 8 x 8 with twice the waves to hide each other's latency, 119 VGPRs at most: 1024^2
+// 12.1 -> 11.1, 800^2 10.7 -> 9.7.
 inline TwoFieldPlan two_field_plan(int W, int H, int esz, int steps, bool wrap, const TwoFieldCost &cost) {
-    static const int shapes[2][2][2] = {{{4, 8}, {8, 8}}, {{4, 8}, {4, 4}}};
+    static const int shapes[2][3][2] = {{{4, 8}, {8, 8}, {4, 16}}, {{4, 8}, {4, 4}, {0, 0}}};
     TwoFieldPlan best;
     const int a = kApron * steps;
     const double x = 0.5, t0 = 4.5 + (double)W * H * cost.planes * esz / 6.5e6;
     for (const auto &sh : shapes[esz == 4 ? 0 : 1]) {
+        if (sh[1] == 0 || (sh[1] == 16 && !cost.wide)) continue;
         TwoFieldPlan p;
         p.r = sh[0];
         p.nw = sh[1];
@@ -46,7 +51,7 @@ inline TwoFieldPlan two_field_plan(int W, int H, int esz, int steps, bool wrap, 
         p.segs = (H + p.rows - 1) / p.rows;
         const double n = p.strips * p.segs / 256.0;                 // workgroups per compute unit
         const double per_cu = n < 6 ? std::ceil(n) : n + 0.5;       // ... on the busiest one
-        const double most = wrap && esz == 4 && p.r == 4 ? 4.0 : 2.0;
+        const double most = p.nw == 16 || (wrap && esz == 4 && p.r == 4) ? 4.0 : 2.0;
         const double waves = std::min(per_cu * p.nw / 4.0, most);   // waves per SIMD
         p.us = t0 / steps + per_cu * p.nw * p.r / 4.0 * cost.row * (1 + 0.6 / waves) + x;
         if (p.us < best.us) best = p;
