@@ -266,6 +266,33 @@ __global__ void __launch_bounds__(kCols) export_planes(const T *__restrict__ sre
     });
 }
 
+// One plane of a large tile, cell by cell: these copies are bound by memory, where
+// one stream in and one out measured faster than two (import and export of 8192^2:
+// 73 us less in FP32 and FP64).
+constexpr long kLargeCells = 4L << 20;
+
+template <typename T>
+__global__ void import_plane(const double *__restrict__ src, T *__restrict__ dst, int W, int H, int pitch) {
+    const long n = (long)W * H;
+    for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x) {
+        const long y = i / W, x = i - y * W;
+        dst[y * pitch + x] = (T)src[i];
+    }
+}
+
+template <typename T>
+__global__ void export_plane(const T *__restrict__ src, double *__restrict__ dst, int W, int H, int pitch,
+                             const double *__restrict__ div) {
+    const long n = (long)W * H;
+    const double d = div ? *div : 1.0;
+    for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x) {
+        const long y = i / W, x = i - y * W;
+        double v = (double)src[y * pitch + x];
+        if (div) v /= d;
+        dst[i] = v;
+    }
+}
+
 // E table of the step: E*corr computed in FP64, each component then rounded
 // once to the kernel precision.  corr is the step's product of the scaled-frame
 // factors (see tsmi_create).  sim may be null (imaginary time: E is real).
@@ -339,30 +366,44 @@ __global__ void __launch_bounds__(kCols) exp_from_potential(const double *__rest
     });
 }
 
-int import_device(tsmi_ctx *c, void *dre, void *dim, const double *re, const double *im) {
-    const dim3 grid(cell_blocks(c->W, c->H));
-    if (c->esz == 8)
-        hipLaunchKernelGGL(import_planes<double>, grid, dim3(kCols), 0, c->stream, re, im, (double *)dre, (double *)dim,
+template <typename T>
+int import_typed(tsmi_ctx *c, T *dre, T *dim, const double *re, const double *im) {
+    if ((long)c->W * c->H > kLargeCells) {
+        hipLaunchKernelGGL(import_plane<T>, dim3(2048), dim3(256), 0, c->stream, re, dre, c->W, c->H, c->pitch);
+        hipLaunchKernelGGL(import_plane<T>, dim3(2048), dim3(256), 0, c->stream, im, dim, c->W, c->H, c->pitch);
+    } else {
+        hipLaunchKernelGGL(import_planes<T>, dim3(cell_blocks(c->W, c->H)), dim3(kCols), 0, c->stream, re, im, dre, dim,
                            c->W, c->H, c->pitch);
-    else
-        hipLaunchKernelGGL(import_planes<float>, grid, dim3(kCols), 0, c->stream, re, im, (float *)dre, (float *)dim, c->W,
-                           c->H, c->pitch);
+    }
     TSMI_HIP(hipGetLastError());
     return TSMI_OK;
 }
 
+int import_device(tsmi_ctx *c, void *dre, void *dim, const double *re, const double *im) {
+    return c->esz == 8 ? import_typed(c, (double *)dre, (double *)dim, re, im)
+                       : import_typed(c, (float *)dre, (float *)dim, re, im);
+}
+
 // pitched planes of the context precision -> W x H FP64 on the device (either may
 // be null), divided by *div when given
-int export_device(tsmi_ctx *c, const void *sre, const void *sim, double *dre, double *dim, const double *div) {
-    const dim3 grid(cell_blocks(c->W, c->H));
-    if (c->esz == 8)
-        hipLaunchKernelGGL(export_planes<double>, grid, dim3(kCols), 0, c->stream, (const double *)sre,
-                           (const double *)sim, dre, dim, c->W, c->H, c->pitch, div);
-    else
-        hipLaunchKernelGGL(export_planes<float>, grid, dim3(kCols), 0, c->stream, (const float *)sre, (const float *)sim,
-                           dre, dim, c->W, c->H, c->pitch, div);
+template <typename T>
+int export_typed(tsmi_ctx *c, const T *sre, const T *sim, double *dre, double *dim, const double *div) {
+    if ((long)c->W * c->H > kLargeCells) {
+        if (dre)
+            hipLaunchKernelGGL(export_plane<T>, dim3(2048), dim3(256), 0, c->stream, sre, dre, c->W, c->H, c->pitch, div);
+        if (dim)
+            hipLaunchKernelGGL(export_plane<T>, dim3(2048), dim3(256), 0, c->stream, sim, dim, c->W, c->H, c->pitch, div);
+    } else {
+        hipLaunchKernelGGL(export_planes<T>, dim3(cell_blocks(c->W, c->H)), dim3(kCols), 0, c->stream, sre, sim, dre, dim,
+                           c->W, c->H, c->pitch, div);
+    }
     TSMI_HIP(hipGetLastError());
     return TSMI_OK;
+}
+
+int export_device(tsmi_ctx *c, const void *sre, const void *sim, double *dre, double *dim, const double *div) {
+    return c->esz == 8 ? export_typed(c, (const double *)sre, (const double *)sim, dre, dim, div)
+                       : export_typed(c, (const float *)sre, (const float *)sim, dre, dim, div);
 }
 
 // The periodic halo refresh of a state (or E) allocation: the reference's

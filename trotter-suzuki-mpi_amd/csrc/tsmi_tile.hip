@@ -225,13 +225,14 @@ bool tile_wraps(const tsmi_ctx *c) {
 // for, offsets within 31 bits, and a lattice small enough that a wave's row
 // latency bounds the streaming passes: us per step, streamed against tiles, 64^2
 // FP64 17.3 / 2.8, 256^2 FP64 23.1 / 4.4, FP32 16.6 / 3.2, 512^2 FP32 14.5 / 3.9,
-// 1024^2 FP32 17.0 / 6.6, FP64 23.6 / 10.5, 2048^2 FP32 22.1 / 17.9, FP64 33.6 /
-// 43.4.  Imaginary time, one step per pass, gives out earlier: closed FP32 100^2
+// 1024^2 FP32 17.0 / 6.6, FP64 23.6 / 10.5, 1600^2 FP64 36.0 / 19.6, 1700^2 FP64
+// 35.8 / 30.0, 1800^2 37.1 / 32.6, 2000^2 FP32 23.7 / 18.3, 2200^2 FP32 24.7 / 31.3,
+// 2048^2 FP64 33.6 / 43.4.  Imaginary time, one step per pass, gives out earlier: closed FP32 100^2
 // 12.4 / 6.9, 1200^2 15.0 / 13.1, 2048^2 23.1 / 28.8, FP64 100^2 14.7 / 6.8, 1024^2
 // 20.7 / 14.8, 1200^2 21.3 / 22.6.
 bool tile_runs(const tsmi_ctx *c) {
     const bool imag = c->d.imag_time != 0;
-    const long most = imag ? (c->esz == 4 ? 3L << 19 : 9L << 17) : (c->esz == 4 ? 5L << 20 : 3L << 19);
+    const long most = imag ? (c->esz == 4 ? 3L << 19 : 9L << 17) : (c->esz == 4 ? 9L << 19 : 5L << 19);
     return c->ph_mode && c->d.sweeps == 0 && c->d.tile_rows == 0 && c->H > 1 && (long)c->W * c->H <= most &&
            (long)c->pitch * c->Hd * c->esz < (1L << 31);
 }
