@@ -27,7 +27,7 @@
 // leaves FP32 tiles of 4 rows 119 VGPRs (two workgroups per CU) instead of 153,
 // and those of 8 rows 231 instead of spilling (1024^2 FP32 17.1 -> 12.2 us per step).
 //
-// Measured, us per step, streamed -> tiles: 1024^2 periodic real FP32 29.5 -> 12.1
+// Measured, us per step, streamed -> tiles: 1024^2 periodic real FP32 29.5 -> 11.1
 // (its 3 planes in and 2 out of both components, 43 MB, and 4.5 us per launch of
 // two steps, then instruction issue), 512^2 FP64 62 -> 8.3, 250^2 closed
 // imaginary FP64 101 -> 11.0 (launch, partial sums and three rows' latency).

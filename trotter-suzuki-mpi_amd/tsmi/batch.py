@@ -1,9 +1,10 @@
 """Python view of a batch of independent lattices (libtsmi_hip.so, tsmi_batch_*).
 
 ``HipBatch(workloads, precision)`` puts every workload's lattice, state and E
-table on the device; ``evolve(n)`` advances all of them by n steps with one
-persistent launch per step (HIP-graph captured); ``state(i)`` reads lattice i
-back; ``tune()`` runs the segment-height autotuner.
+table on the device; ``evolve(n)`` advances all of them by n steps with shared
+launches (HIP-graph captured), one or several steps each; ``state(i)`` reads
+lattice i back; ``tune()`` runs the segment-height autotuner of the streaming
+passes (small batches run as register tiles, which have nothing to tune).
 """
 from __future__ import annotations
 
