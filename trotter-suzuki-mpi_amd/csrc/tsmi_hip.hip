@@ -219,28 +219,36 @@ int download_state(tsmi_ctx *c, size_t stride, size_t x, size_t y, size_t w, siz
 }
 
 // Tile-wide kernels between W x H FP64 arrays (row stride W) and pitched planes:
-// a workgroup takes 256 columns of a row at a time, so a cell's row and column
-// cost no division, and both planes of a state go in one launch (50 steps of 64^2
-// with import and export 150 -> 146 us).
-constexpr int kCols = 256;
+// a thread walks the cells, numbered row by row, at the grid's stride, which it
+// takes apart into rows and columns once (two 32-bit divisions), so that a cell
+// costs none and no lane idles whatever the width; both planes of a state go in one
+// launch.  Bound by memory from some 10^6 cells on, by the launch below.  Against a
+// workgroup per 256 columns of a row, us: state import FP32 2 x 10^6 205 -> 32,
+// 16 x 200000 44 -> 14, 1024^2 6.2 -> 5.8; E from V 2 x 10^6 329 -> 69, 257 x 4000
+// 13.8 -> 10.1, 1024^2 10.8 -> 10.2.
+constexpr int kCells = 256;          // threads of a workgroup
 
 template <typename F>
 __device__ __forceinline__ void for_cells(int W, int H, F &&f) {
-    const unsigned chunks = ((unsigned)W + kCols - 1) / kCols;
-    const unsigned items = chunks * (unsigned)H;   // a plane this size is far beyond any memory
-    for (unsigned i = blockIdx.x; i < items; i += gridDim.x) {
-        const unsigned y = i / chunks, x = (i - y * chunks) * kCols + threadIdx.x;
-        if (x < (unsigned)W) f((long)y, (long)x);
+    const unsigned w = (unsigned)W, stride = gridDim.x * kCells, i = blockIdx.x * kCells + threadIdx.x;
+    const unsigned dy = stride / w, dx = stride - dy * w;
+    unsigned y = i / w, x = i - y * w;
+    while (y < (unsigned)H) {        // H <= 2^30 and dy <= 2^19: no wrap
+        f((long)y, (long)x);
+        x += dx;
+        y += dy;
+        if (x >= w) {
+            x -= w;
+            ++y;
+        }
     }
 }
 
-int cell_blocks(int W, int H) {
-    return (int)std::min<long long>(4096, (long long)((W + kCols - 1) / kCols) * H);
-}
+int cell_blocks(int W, int H) { return (int)std::min<long long>(2048, ((long long)W * H + kCells - 1) / kCells); }
 
 // FP64 -> T, rounding once
 template <typename T>
-__global__ void __launch_bounds__(kCols) import_planes(const double *__restrict__ sre, const double *__restrict__ sim,
+__global__ void __launch_bounds__(kCells) import_planes(const double *__restrict__ sre, const double *__restrict__ sim,
                                                        T *__restrict__ dre, T *__restrict__ dim, int W, int H, int pitch) {
     for_cells(W, H, [&](long y, long x) {
         const double re = sre[y * W + x], im = sim[y * W + x];
@@ -251,7 +259,7 @@ __global__ void __launch_bounds__(kCols) import_planes(const double *__restrict_
 
 // T -> FP64, divided by *div when given; either destination may be null
 template <typename T>
-__global__ void __launch_bounds__(kCols) export_planes(const T *__restrict__ sre, const T *__restrict__ sim,
+__global__ void __launch_bounds__(kCells) export_planes(const T *__restrict__ sre, const T *__restrict__ sim,
                                                        double *__restrict__ dre, double *__restrict__ dim, int W, int H,
                                                        int pitch, const double *__restrict__ div) {
     const double d = div ? *div : 1.0;
@@ -300,7 +308,7 @@ __global__ void export_plane(const T *__restrict__ src, double *__restrict__ dst
 // (real time), lambda = -ln(E corr) when E > 0 (imaginary time); a cell without
 // that form sets *bad.
 template <typename T>
-__global__ void __launch_bounds__(kCols) import_exp(const double *__restrict__ sre, const double *__restrict__ sim, double cr, double ci,
+__global__ void __launch_bounds__(kCells) import_exp(const double *__restrict__ sre, const double *__restrict__ sim, double cr, double ci,
                            T *__restrict__ dre, T *__restrict__ dim, T *__restrict__ dph, unsigned *bad, int W,
                            int H, int pitch) {
     bool ok = true;
@@ -327,10 +335,10 @@ __global__ void __launch_bounds__(kCols) import_exp(const double *__restrict__ s
 int launch_import_exp(tsmi_ctx *c, const double *re, const double *im) {
     TSMI_HIP(hipMemsetAsync(c->flag, 0, sizeof(unsigned), c->stream));
     if (c->esz == 4)
-        hipLaunchKernelGGL(import_exp<float>, dim3(cell_blocks(c->W, c->H)), dim3(kCols), 0, c->stream, re, im, c->corr_re, c->corr_im,
+        hipLaunchKernelGGL(import_exp<float>, dim3(cell_blocks(c->W, c->H)), dim3(kCells), 0, c->stream, re, im, c->corr_re, c->corr_im,
                            (float *)c->e_re, (float *)c->e_im, (float *)c->ph, c->flag, c->W, c->H, c->pitch);
     else
-        hipLaunchKernelGGL(import_exp<double>, dim3(cell_blocks(c->W, c->H)), dim3(kCols), 0, c->stream, re, im, c->corr_re, c->corr_im,
+        hipLaunchKernelGGL(import_exp<double>, dim3(cell_blocks(c->W, c->H)), dim3(kCells), 0, c->stream, re, im, c->corr_re, c->corr_im,
                            (double *)c->e_re, (double *)c->e_im, (double *)c->ph, c->flag, c->W, c->H, c->pitch);
     TSMI_HIP(hipGetLastError());
     unsigned bad = 1;
@@ -345,7 +353,7 @@ int launch_import_exp(tsmi_ctx *c, const double *re, const double *im) {
 // it (src/solver.cpp:74-109), times the frame factor, rounded once; the raw V
 // goes to the pitched FP64 plane used by the energies.
 template <typename T>
-__global__ void __launch_bounds__(kCols) exp_from_potential(const double *__restrict__ v, double dt, int imag, double cr, double ci,
+__global__ void __launch_bounds__(kCells) exp_from_potential(const double *__restrict__ v, double dt, int imag, double cr, double ci,
                                    T *__restrict__ dre, T *__restrict__ dim, T *__restrict__ dph,
                                    double *__restrict__ vout, int W, int H, int pitch) {
     // one-plane form: phi = dt V - arg(corr), lambda = dt V - ln(corr)
@@ -372,7 +380,7 @@ int import_typed(tsmi_ctx *c, T *dre, T *dim, const double *re, const double *im
         hipLaunchKernelGGL(import_plane<T>, dim3(2048), dim3(256), 0, c->stream, re, dre, c->W, c->H, c->pitch);
         hipLaunchKernelGGL(import_plane<T>, dim3(2048), dim3(256), 0, c->stream, im, dim, c->W, c->H, c->pitch);
     } else {
-        hipLaunchKernelGGL(import_planes<T>, dim3(cell_blocks(c->W, c->H)), dim3(kCols), 0, c->stream, re, im, dre, dim,
+        hipLaunchKernelGGL(import_planes<T>, dim3(cell_blocks(c->W, c->H)), dim3(kCells), 0, c->stream, re, im, dre, dim,
                            c->W, c->H, c->pitch);
     }
     TSMI_HIP(hipGetLastError());
@@ -394,7 +402,7 @@ int export_typed(tsmi_ctx *c, const T *sre, const T *sim, double *dre, double *d
         if (dim)
             hipLaunchKernelGGL(export_plane<T>, dim3(2048), dim3(256), 0, c->stream, sim, dim, c->W, c->H, c->pitch, div);
     } else {
-        hipLaunchKernelGGL(export_planes<T>, dim3(cell_blocks(c->W, c->H)), dim3(kCols), 0, c->stream, sre, sim, dre, dim,
+        hipLaunchKernelGGL(export_planes<T>, dim3(cell_blocks(c->W, c->H)), dim3(kCells), 0, c->stream, sre, sim, dre, dim,
                            c->W, c->H, c->pitch, div);
     }
     TSMI_HIP(hipGetLastError());
@@ -1155,10 +1163,10 @@ int tsmi_set_potential_exp_device(tsmi_ctx *c, const double *v) {
     const double dt = c->d.delta_t;
     const int imag = c->d.imag_time ? 1 : 0;
     if (c->esz == 4)
-        hipLaunchKernelGGL(exp_from_potential<float>, dim3(cell_blocks(c->W, c->H)), dim3(kCols), 0, c->stream, v, dt, imag, c->corr_re,
+        hipLaunchKernelGGL(exp_from_potential<float>, dim3(cell_blocks(c->W, c->H)), dim3(kCells), 0, c->stream, v, dt, imag, c->corr_re,
                            c->corr_im, (float *)c->e_re, (float *)c->e_im, (float *)c->ph, c->v, c->W, c->H, c->pitch);
     else
-        hipLaunchKernelGGL(exp_from_potential<double>, dim3(cell_blocks(c->W, c->H)), dim3(kCols), 0, c->stream, v, dt, imag, c->corr_re,
+        hipLaunchKernelGGL(exp_from_potential<double>, dim3(cell_blocks(c->W, c->H)), dim3(kCells), 0, c->stream, v, dt, imag, c->corr_re,
                            c->corr_im, (double *)c->e_re, (double *)c->e_im, (double *)c->ph, c->v, c->W, c->H,
                            c->pitch);
     TSMI_HIP(hipGetLastError());
