@@ -42,7 +42,7 @@
 
 namespace tsmi {
 
-constexpr int kTileWavesMax = 8;     // waves per workgroup, at most
+constexpr int kTileWaves = 8;        // most waves per workgroup of a tile (the 16 waves of 4 FP32 rows apart)
 constexpr int kTileCols = 2 * kWave; // columns of a tile
 constexpr int kTileImag = 2;         // MODE of imaginary time
 

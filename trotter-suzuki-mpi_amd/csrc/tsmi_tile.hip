@@ -20,24 +20,25 @@ using namespace tsmi;
 
 namespace {
 
-// Rows per wave of the compiled instances.
-constexpr int kRows32[] = {4, 8, 12}, kRows64[] = {4, 6, 8};
+// Rows per wave of the compiled instances, of 4 or 8 waves each; FP32 with 4 rows
+// also of 16 (80 VGPRs).  No 8 rows in FP32: their tiles, 32 and 64 rows high, are
+// those of 4 rows with twice the waves, which hide each other's latency.
+constexpr int kRows32[] = {4, 12}, kRows64[] = {4, 6, 8};
 
 // The tile shape of a pass of `steps` steps: the one with the least modelled time.
 // A launch costs about 5 us whatever it does; a step costs each SIMD its rows
 // (about 0.17 us a row in FP32, 0.27 in FP64 with several waves per SIMD, up to
 // 60% more for a wave alone) and 0.35 us of exchanges.  Measured around it, us
 // per step: 256^2 FP64 4 rows x 8 waves 6.9, 4.9, 4.4 for 1, 2, 3 steps, 8 x 8
-// 10.7, 7.9, 7.1; 1024^2 FP32 8 x 8 9.4, 6.7, 9.8 (3 steps: more than one
-// workgroup per compute unit), 12 x 8 12.4, 8.9, 7.3, 7.2, 7.0 (5 steps).
+// 10.7, 7.9, 7.1; 1100^2 FP32 4 x 16 9.8, 6.7, 8.7 (3 steps: more than one
+// workgroup per compute unit), 12 x 8 12.3, 8.7, 7.4, 7.2, 9.5 (5 steps).
 TilePlan plan(const std::pair<int, int> *size, size_t count, int esz, int steps) {
     TilePlan best;
     const int a = kApron * steps;
-    const int *rr = esz == 4 ? kRows32 : kRows64;
+    const int *rr = esz == 4 ? kRows32 : kRows64, n_rr = esz == 4 ? 2 : 3;
     const double c_row = esz == 4 ? 0.17 : 0.27, x = 0.35, t0 = 5.0;
-    for (int i = 0; i < 3; ++i)
+    for (int i = 0; i < n_rr; ++i)
         for (int nw : {4, 8, 16}) {
-            // 16 waves: FP32 with 4 rows, the only instance of at most 128 VGPRs
             if (nw == 16 && (esz != 4 || i != 0)) continue;
             TilePlan p;
             p.r = rr[i];
@@ -90,15 +91,16 @@ void launch_mode(int mode, const TilePlan &g, int blocks, const TileParams<T> *p
 
 template <typename T, bool LHY>
 int launch_rows(int mode, const TilePlan &g, int blocks, const TileParams<T> *p, const int2 *items, hipStream_t s) {
-    constexpr const int *rr = sizeof(T) == 4 ? kRows32 : kRows64;
-    constexpr int N = kTileWavesMax;
+    constexpr int N = kTileWaves;
     if constexpr (sizeof(T) == 4) {
-        if (g.nw == 16) launch_mode<T, LHY, rr[0], 16>(mode, g, blocks, p, items, s);
+        if (g.nw == 16) launch_mode<T, LHY, 4, 16>(mode, g, blocks, p, items, s);
+        else if (g.r == 4) launch_mode<T, LHY, 4, N>(mode, g, blocks, p, items, s);
+        else launch_mode<T, LHY, 12, N>(mode, g, blocks, p, items, s);
+    } else {
+        if (g.r == 4) launch_mode<T, LHY, 4, N>(mode, g, blocks, p, items, s);
+        else if (g.r == 6) launch_mode<T, LHY, 6, N>(mode, g, blocks, p, items, s);
+        else launch_mode<T, LHY, 8, N>(mode, g, blocks, p, items, s);
     }
-    if (g.nw == 16) (void)0;   // launched above
-    else if (g.r == rr[0]) launch_mode<T, LHY, rr[0], N>(mode, g, blocks, p, items, s);
-    else if (g.r == rr[1]) launch_mode<T, LHY, rr[1], N>(mode, g, blocks, p, items, s);
-    else launch_mode<T, LHY, rr[2], N>(mode, g, blocks, p, items, s);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return set_error(TSMI_E_HIP, std::string("tile_kernel: ") + hipGetErrorString(e));
     return TSMI_OK;
