@@ -342,6 +342,13 @@ int tsmi_geometry(const tsmi_ctx *ctx, int32_t out[6]);
  * plane.  No reference counterpart (planning and reporting). */
 int tsmi_plan_geometry(const tsmi_desc *desc, int32_t out[12]);
 
+/* Whether an evolve call of n_steps steps runs as register tiles rather than the
+ * passes of tsmi_plan_geometry (small and medium lattices, sweeps and tile_rows 0,
+ * an E table of unit modulus, or positive in imaginary time): out[0..3] = rows per
+ * wave, waves per workgroup, steps and workgroups of its longest launch, or 0s.
+ * Touches no device.  No reference counterpart (planning and reporting). */
+int tsmi_tile_geometry(const tsmi_desc *desc, int32_t n_steps, int32_t out[4]);
+
 /* Message of the calling thread's last failed call ("" if none). */
 const char *tsmi_last_error(void);
 

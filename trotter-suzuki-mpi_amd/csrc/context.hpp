@@ -87,12 +87,22 @@ int ctx_exchange(tsmi_ctx *c, void *re, void *im);
 // several steps per launch; which 0: before, 1: after).
 int ctx_time_mark(tsmi_ctx *c, int kind, int which);
 
-// Tile passes (tsmi_tile.hip), asynchronous on c's stream: whether c's steps run
-// as them; whether c is a doubly periodic lattice whose passes may wrap
-// (several steps per launch); n steps as one or several passes, on the tile
-// closed at its edges or (wrap) on the periodic lattice, the halo refreshed.
-bool tile_runs(const tsmi_ctx *c);
-bool tile_wraps(const tsmi_ctx *c);
+// Tile passes (tsmi_tile.hip), asynchronous on c's stream.
+// How a call of n steps runs: streamed; on the tile closed at its edges, several
+// steps per launch; on the doubly periodic lattice, several steps per launch
+// between a first and a last step of their own; step by step, the halo read from
+// the cells it mirrors (one step in imaginary time always).
+enum TileRoute { kRouteStream, kRouteClosed, kRouteWrap, kRouteSeam };
+TileRoute tile_route(const tsmi_desc &d, int W, int H, int n);   // E in one plane
+TileRoute tile_route(const tsmi_ctx *c, int n);
+// The cells of the tiles that cover W x H cells: columns in whole tile widths, rows in
+// whole heights of the lowest common tile.
+long tile_area(int W, int H);
+// Rows per wave, waves, steps and workgroups of the longest pass of such a call (0s:
+// streamed).
+void tile_geometry(const tsmi_desc &d, int W, int H, int n, int32_t out[4]);
+// n steps as one or several passes, on the tile closed at its edges or (wrap) on the
+// periodic lattice, the halo refreshed.
 int tile_passes(tsmi_ctx *c, int n, bool wrap);
 // n steps, each starting with the halo exchange that has not been run yet (the
 // state's halo cells are read from the cells they mirror).

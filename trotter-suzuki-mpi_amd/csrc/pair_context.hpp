@@ -39,10 +39,11 @@ inline double *norms(tsmi_pair *p) { return p->dv + 4 + 2 * p->norm_slot; }
 int exchange_both(tsmi_pair *p);
 
 // Tile passes (tsmi_pair_tile.hip): whether the lattice takes them (set at
-// creation; the E tables must have the phase form when they run), the most
-// workgroups of an imaginary-time pass, and an evolve of n steps as them (no
+// creation), whether a call of n steps does (the E tables must have the phase form
+// besides), the most workgroups of an imaginary-time pass, and an evolve of n steps as them (no
 // renormalisation pending before; every cell renormalised after).
 bool pair_tiles_fit(const tsmi_pair *p, int tile_rows, int sweeps);
+bool pair_tiles_run(const tsmi_pair *p, int n);
 int pair_tile_blocks(const tsmi_pair *p);
 int pair_tile_evolve(tsmi_pair *p, int n, bool rabi);
 

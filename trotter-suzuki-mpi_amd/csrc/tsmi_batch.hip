@@ -49,7 +49,10 @@ constexpr int kBlock = 256;
 constexpr int kGroups = 4;                     // see the top
 constexpr int kDefaultSegRows = 64;
 constexpr int kVecF = 2;                       // elements per lane of the fused passes
-constexpr long kTileCells32 = 7L << 19, kTileCells64 = 3L << 19;   // most cells of a batch run as tiles
+// Most cells of a batch run as tiles, and most cells of its tiles: each lattice's
+// columns in whole tile widths (120) and rows in eights.
+constexpr long kTileCells32 = 7L << 19, kTileCells64 = 3L << 19;
+constexpr long kTileArea32 = 7L << 20, kTileArea64 = 7L << 19;
 constexpr int kExchChunks = 64;                // most workgroups per lattice of an exchange launch
 
 #define TSMI_HIPB(call)                                                                              \
@@ -799,9 +802,16 @@ int tsmi_batch_create(const tsmi_desc *descs, int32_t n, tsmi_batch **out) {
     // FP32 32 -> 2.7, FP64 33 -> 3.4, 32 x 256^2 FP32 36 -> 12, 12 x 512^2 FP32 35 ->
     // 15; FP64 32 x 256^2, past the line, 38 -> 32).  Above it the streaming passes,
     // which autotuning helps and tiles not, are near their memory time.
-    long cells = 0;
-    for (const Lattice &L : b->lat) cells += (long)L.W * L.H;
-    if (!b->imag && cells <= (b->esz == 4 ? kTileCells32 : kTileCells64))
+    // Lattices much narrower than a tile leave its lanes idle: FP64 1000 x 31^2 odd
+    // periodic, an area of 4.8M cells, 31.4 -> 34.9 (tuned 29.7 -> 34.3), FP32 25.0 ->
+    // 21.7; FP32 1500 x 30^2, 7.2M, 33.1 -> 26.3.
+    long cells = 0, area = 0;
+    for (const Lattice &L : b->lat) {
+        cells += (long)L.W * L.H;
+        area += (L.W + 119L) / 120 * 120 * ((L.H + 7L) / 8 * 8);
+    }
+    if (!b->imag && cells <= (b->esz == 4 ? kTileCells32 : kTileCells64) &&
+        area <= (b->esz == 4 ? kTileArea32 : kTileArea64))
         for (Lattice &L : b->lat) {
             const tsmi_desc &d = L.d;
             if (d.sweeps != 0 || d.tile_rows > 0 || L.H < 2) continue;

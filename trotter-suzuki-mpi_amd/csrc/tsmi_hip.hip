@@ -664,7 +664,7 @@ int exchange_planes(tsmi_ctx *c, void *re, void *im) {
 int exchange_current(tsmi_ctx *c) { return exchange_planes(c, c->psi_base[c->cur][0], c->psi_base[c->cur][1]); }
 
 int step_once(tsmi_ctx *c, int exchange) {
-    if (!tile_runs(c)) return step_rows(c, exchange);
+    if (tile_route(c, 1) == kRouteStream) return step_rows(c, exchange);
     const int st = tile_passes(c, 1, false);
     return st || !exchange ? st : exchange_current(c);
 }
@@ -680,18 +680,21 @@ int step_once(tsmi_ctx *c, int exchange) {
 int evolve_steps(tsmi_ctx *c, int n, bool exchange_last = false) {
     int st = TSMI_OK;
     const int last_ex = exchange_last ? 1 : 0;
-    if (tile_runs(c)) {
-        if (!c->d.periodic_x && !c->d.periodic_y) return tile_passes(c, n, false);
-        if (tile_wraps(c) && n >= 3) {
-            st = tile_passes(c, 1, false);
-            if (!st) st = tile_passes(c, n - 2, true);
-            return st ? st : step_once(c, last_ex);
-        }
+    switch (tile_route(c, n)) {
+    case kRouteClosed:
+        return tile_passes(c, n, false);
+    case kRouteWrap:
+        st = step_once(c, 0);
+        if (!st) st = tile_passes(c, n - 2, true);
+        return st ? st : step_once(c, last_ex);
+    case kRouteSeam:
         // mixed axes; odd periodic extents, where the pair pattern of a halo cell
-        // differs from that of the cell it mirrors
-        if (n > 0) st = tile_passes(c, 1, false);
+        // differs from that of the cell it mirrors; short calls
+        st = tile_passes(c, 1, false);
         if (!st) st = tile_seam_steps(c, n - 1);
-        return st || !last_ex || n <= 0 ? st : exchange_current(c);
+        return st || !last_ex ? st : exchange_current(c);
+    case kRouteStream:
+        break;
     }
     if (c->sweeps != 2 || n < 2 || (c->halo8 && n < 3)) {
         for (int i = 0; i < n && !st; ++i) st = step_once(c, i != n - 1 ? 1 : last_ex);
@@ -716,9 +719,9 @@ int evolve_steps(tsmi_ctx *c, int n, bool exchange_last = false) {
 // The fused passes read E over the whole 8-wide halo: the reference-tile table
 // with every halo cell replaced by its wrapped inner cell.
 int wrap_exp(tsmi_ctx *c) {
-    // tile passes read the reference tile's table (whether they run depends on the
-    // descriptor and the table's form alone)
-    if (!c->halo8 || tile_runs(c)) return TSMI_OK;
+    // tile passes read the reference tile's table (whether a call of three steps
+    // or more takes them depends on the descriptor and the table's form alone)
+    if (!c->halo8 || tile_route(c, 3) != kRouteStream) return TSMI_OK;
     const size_t pb = plane_bytes(c);
     TSMI_HIP(hipMemcpyAsync(c->e8[0], c->e_base[0], pb, hipMemcpyDeviceToDevice, c->stream));
     TSMI_HIP(hipMemcpyAsync(c->e8[1], c->e_base[1], pb, hipMemcpyDeviceToDevice, c->stream));
@@ -1270,7 +1273,7 @@ int tsmi_evolve_checkpointed(tsmi_ctx *c, int32_t n, int32_t every) {
     // closed axes, FP32: two steps per pass wherever no checkpoint falls between
     // them (FP64 measured faster at one step per pass on a 1024^2 lattice: 32.7
     // against 34.9 ms for 2000 steps; FP32 37.7 against 30.3)
-    const bool tiles = tile_runs(c) && !c->d.periodic_x && !c->d.periodic_y;
+    const bool tiles = tile_route(c, 2) == kRouteClosed;
     const bool pairs = c->sweeps == 2 && !c->halo8 && c->esz == 4;
     for (int i = 0; i < n;) {
         if (i % every == 0) {
@@ -1280,7 +1283,7 @@ int tsmi_evolve_checkpointed(tsmi_ctx *c, int32_t n, int32_t every) {
         }
         if (tiles) {   // up to the next checkpoint
             const int m = std::min(n, (i / every + 1) * every) - i;
-            if (const int st = tile_passes(c, m, false)) return st;
+            if (const int st = m == 1 ? step_once(c, 0) : tile_passes(c, m, false)) return st;
             i += m;
             continue;
         }
@@ -1446,6 +1449,15 @@ int tsmi_geometry(const tsmi_ctx *c, int32_t out[6]) {
     if (!c || !out) return fail(TSMI_E_INVALID, "tsmi_geometry: null argument");
     out[0] = c->W; out[1] = c->H; out[2] = c->pitch;
     out[3] = c->n_strips; out[4] = c->n_segs; out[5] = c->seg_rows;
+    return TSMI_OK;
+}
+
+int tsmi_tile_geometry(const tsmi_desc *desc, int32_t n_steps, int32_t out[4]) {
+    if (!desc || !out) return fail(TSMI_E_INVALID, "tsmi_tile_geometry: null argument");
+    if (int st = check_desc(*desc, "tsmi_tile_geometry")) return st;
+    const tsmi_desc &d = *desc;
+    tile_geometry(d, d.dim_x + (d.periodic_x ? 2 * d.halo_x : 0), d.dim_y + (d.periodic_y ? 2 * d.halo_y : 0), n_steps,
+                  out);
     return TSMI_OK;
 }
 

@@ -482,7 +482,7 @@ int tsmi_pair_evolve(tsmi_pair *p, int32_t n_steps, int32_t initial_half) {
     // src/solver.cpp:173-177
     if (initial_half && rabi) st = rabi_pass(p, 0.5, true, false);
     // tile passes or two steps per pass where both E tables have the phase form
-    if (!st && p->tiles && p->c[0]->ph_mode && p->c[1]->ph_mode) {
+    if (!st && pair_tiles_run(p, n_steps) && p->c[0]->ph_mode && p->c[1]->ph_mode) {
         st = settle(p);
         return st ? st : pair_tile_evolve(p, n_steps, rabi);
     }

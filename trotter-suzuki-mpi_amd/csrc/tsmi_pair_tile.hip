@@ -153,6 +153,13 @@ int tile_pass(tsmi_pair *p, int steps, How how, double var, bool rabi, bool firs
     return p->esz == 4 ? pass<float>(p, steps, how, var, rabi, first) : pass<double>(p, steps, how, var, rabi, first);
 }
 
+// A call of n steps that runs on the doubly periodic lattice between its first and
+// its last step.
+bool wraps(const tsmi_pair *p, int n) {
+    const tsmi_desc &d = p->c[0]->d;
+    return d.periodic_x && d.periodic_y && d.dim_x % 2 == 0 && d.dim_y % 2 == 0 && n >= 3;
+}
+
 // The renormalisation after the last step.
 int finish(tsmi_pair *p, double var, bool rabi) {
     const PairNorm q = pending(p, var, rabi);
@@ -191,17 +198,26 @@ int pair_tile_blocks(const tsmi_pair *p) {
 // 512^2 37 / 33 -> 7.8 / 8.0, 1240^2 38 / 35 -> 22 / 29; FP64 100^2 61 / 55 -> 7.7 /
 // 8.6, 1240^2 64 / 59 -> 40 / 43; imaginary FP32 100^2 63 / 58 -> 11 / 12, 1240^2
 // 263 / 257 -> 26 / 33, FP64 1240^2 279 / 275 -> 54 / 54.
+// Narrow and flat lattices leave most of their tiles idle: real FP32 2 x 400000 204 /
+// 563, 8 x 10^5 the other way round 15 / 22, 20 x 15000 29 / 22; imaginary FP64 2 x
+// 400000 811 / 5884, 10 x 40000 289 / 143, FP32 3 x 300000 291 / 177.
 bool pair_tiles_fit(const tsmi_pair *p, int tile_rows, int sweeps) {
-    const long most = p->imag ? 5L << 20 : 3L << 19;
-    return tile_rows == 0 && sweeps == 0 && p->H > 1 && (long)p->W * p->H <= most &&
+    const long most = p->imag ? 5L << 20 : 3L << 19, area = p->imag ? 2 * most : most + most / 4;
+    return tile_rows == 0 && sweeps == 0 && p->H > 1 && (long)p->W * p->H <= most && tile_area(p->W, p->H) <= area &&
            (long)p->pitch * p->c[0]->Hd * p->esz < (1L << 31);
+}
+
+// FP64 in real time where tiles have an edge gives out earlier: closed 1100^2 36.4 /
+// 31.9, 1200^2 37.5 / 39.6; periodic in x 1100^2 41.9 / 32.9, 1200^2 42.4 / 42.4.
+bool pair_tiles_run(const tsmi_pair *p, int n) {
+    return p->tiles && (p->imag || p->esz == 4 || wraps(p, n) || (long)p->W * p->H <= 19L << 16);
 }
 
 int pair_tile_evolve(tsmi_pair *p, int n, bool rabi) {
     if (n <= 0) return TSMI_OK;
     const tsmi_desc &d = p->c[0]->d;
     const bool closed = !d.periodic_x && !d.periodic_y;
-    const bool wrap = d.periodic_x && d.periodic_y && d.dim_x % 2 == 0 && d.dim_y % 2 == 0 && n >= 3;
+    const bool wrap = wraps(p, n);
     const int most = p->imag || !(closed || wrap) ? 1 : n;
     int i = 0, st = TSMI_OK;
     // n steps from step i on; the call's last rotation is by 1/2 (src/solver.cpp:222-225)

@@ -25,18 +25,32 @@ namespace {
 // those of 4 rows with twice the waves, which hide each other's latency.
 constexpr int kRows32[] = {4, 12}, kRows64[] = {4, 6, 8};
 
+// The modelled time of a step, fitted to 800 timings (200^2 to 2400^2, every
+// shape, 1 to 6 steps per pass; 8 % rms in FP64, 12 % in FP32): a launch costs
+// t0 and its planes at bw TB/s (3 in, 2 out; a part h of that when a compute unit
+// holds several workgroups, one computing while another loads), a step costs each
+// SIMD its rows (row us, more for a wave alone) and x of exchanges and passes.
+struct TileCost {
+    double row, alone, x, t0, bw, h;
+};
+constexpr TileCost kCost32 = {0.117, 0.8, 1.9, 2.0, 5.8, 0.8}, kCost64 = {0.207, 0.37, 1.0, 3.3, 6.5, 0.85};
+
+// Waves per SIMD that the registers of an instance leave.
+int tile_waves(int esz, int r) { return esz == 4 ? (r == 4 ? 4 : 2) : (r == 4 ? 3 : 2); }
+
 // The tile shape of a pass of `steps` steps: the one with the least modelled time.
-// A launch costs about 5 us whatever it does; a step costs each SIMD its rows
-// (about 0.17 us a row in FP32, 0.27 in FP64 with several waves per SIMD, up to
-// 60% more for a wave alone) and 0.35 us of exchanges.  Measured around it, us
-// per step: 256^2 FP64 4 rows x 8 waves 6.9, 4.9, 4.4 for 1, 2, 3 steps, 8 x 8
-// 10.7, 7.9, 7.1; 1100^2 FP32 4 x 16 9.8, 6.7, 8.7 (3 steps: more than one
-// workgroup per compute unit), 12 x 8 12.3, 8.7, 7.4, 7.2, 9.5 (5 steps).
-TilePlan plan(const std::pair<int, int> *size, size_t count, int esz, int steps) {
+// Without the planes' time the model took one step per pass at 1800^2 and 2100^2
+// FP32 (21.5 and 28.7 us per step; three and four steps 15.5 and 20.1) and 4 rows
+// x 8 waves for single FP64 steps of 1200^2 (18.7; 8 x 4 15.3).  In imaginary time
+// every wave adds the partial sums of all workgroups: 4 ns each.
+TilePlan plan(const std::pair<int, int> *size, size_t count, int esz, int steps, bool imag) {
     TilePlan best;
     const int a = kApron * steps;
     const int *rr = esz == 4 ? kRows32 : kRows64, n_rr = esz == 4 ? 2 : 3;
-    const double c_row = esz == 4 ? 0.17 : 0.27, x = 0.35, t0 = 5.0;
+    const TileCost &m = esz == 4 ? kCost32 : kCost64;
+    double cells = 0;
+    for (size_t j = 0; j < count; ++j) cells += (double)size[j].first * size[j].second;
+    const double planes = cells * 5 * esz / (m.bw * 1e6);
     for (int i = 0; i < n_rr; ++i)
         for (int nw : {4, 8, 16}) {
             if (nw == 16 && (esz != 4 || i != 0)) continue;
@@ -50,8 +64,10 @@ TilePlan plan(const std::pair<int, int> *size, size_t count, int esz, int steps)
                 tiles += (long)((size[j].first + cols - 1) / cols) * ((size[j].second + rows - 1) / rows);
             const double n = tiles / 256.0;                          // workgroups per compute unit
             const double per_cu = n < 6 ? std::ceil(n) : n + 0.5;    // ... on the busiest one
-            const double waves = std::min(per_cu * nw / 4.0, nw == 16 ? 4.0 : 3.0);   // waves per SIMD
-            p.us = t0 / steps + per_cu * nw * p.r / 4.0 * c_row * (1 + 0.6 / waves) + x;
+            const int held = std::max(1, tile_waves(esz, p.r) * 4 / nw);   // ... that it holds at a time
+            const double waves = std::min(per_cu, (double)held) * nw / 4;  // waves per SIMD
+            p.us = (m.t0 + planes * (std::min(per_cu, (double)held) > 1 ? m.h : 1.0)) / steps +
+                   per_cu * nw * p.r / 4 * m.row * (1 + m.alone / waves) + m.x + (imag ? 0.004 * tiles : 0.0);
             if (p.us < best.us) best = p;
         }
     return best;
@@ -61,7 +77,7 @@ int best_steps(const std::pair<int, int> *size, size_t count, int esz, int most)
     int k = 1;
     double us = 1e30;
     for (int s = 1; s <= std::min(most, 8); ++s) {
-        const TilePlan p = plan(size, count, esz, s);
+        const TilePlan p = plan(size, count, esz, s, false);
         if (p.us < us) {
             us = p.us;
             k = s;
@@ -117,12 +133,10 @@ int launch_any(bool lhy, int mode, const TilePlan &g, int blocks, const TilePara
 enum How { kClosed, kWrap, kSeam };
 
 template <typename T>
-int pass(tsmi_ctx *c, int steps, How how, long double &drift) {
+int pass(tsmi_ctx *c, const TilePlan &g, int steps, How how, long double &drift) {
     TileParams<T> p;
     std::memset(&p, 0, sizeof(p));
     const int nb = 1 - c->cur;
-    const std::pair<int, int> size(c->W, c->H);
-    const TilePlan g = plan(&size, 1, c->esz, steps);
     if (g.r == 0) return set_error(TSMI_E_INVALID, "tile pass: no tile for this many steps");
     const TileFactors f = {c->mH, c->tH, c->mV, c->tV, c->unH, c->unV, c->c_nl_s, c->c_lhy_s, c->corr_abs,
                            c->d.delta_t / (4. * c->d.mass * c->d.delta_y * c->d.delta_y)};
@@ -162,7 +176,7 @@ int pass(tsmi_ctx *c, int steps, How how, long double &drift) {
 namespace tsmi {
 
 TilePlan tile_plan(const std::vector<std::pair<int, int>> &sizes, int esz, int steps) {
-    return plan(sizes.data(), sizes.size(), esz, steps);
+    return plan(sizes.data(), sizes.size(), esz, steps, false);
 }
 
 int tile_best_steps(const std::vector<std::pair<int, int>> &sizes, int esz, int most) {
@@ -219,52 +233,112 @@ int tile_batch_launch(int esz, bool lhy, int mode, const TilePlan &g, const void
                     : launch_any<double>(lhy, mode, g, n_items, (const TileParams<double> *)params, items, stream);
 }
 
-bool tile_wraps(const tsmi_ctx *c) {
-    return c->d.periodic_x && c->d.periodic_y && c->d.dim_x % 2 == 0 && c->d.dim_y % 2 == 0;
+long tile_area(int W, int H) { return (W + 119L) / 120 * 120 * ((H + 23L) / 24 * 24); }
+
+// Cells, and cells of whole tiles (tile_area), up to which a pass of one step, or of
+// several, takes tiles.  us per step, streamed / tiles, closed and doubly periodic
+// alike unless said.
+// Several steps per pass (against two streamed): 64^2 FP64 17.3 / 2.8, FP32 256^2
+// 16.6 / 3.2, 512^2 14.5 / 3.9, 1000^2 14.0 / 5.6, 1800^2 19.0 / 15.5, 2100^2 22.6 /
+// 20.1, 2200^2 22.6 / 22.4; FP64 1000^2 15.4 / 8.0, 1600^2 24.2 / 18.7, 2000^2 29.1 /
+// 27.9, 2100^2 31.0 / 32.9 (the FP64 line is drawn at 1620^2).
+// One step per pass (single steps, short calls, mixed axes, odd periodic extents):
+// FP32 1000^2 17.9 / 9.0, 1800^2 22.9 / 18.9, 2000^2 24.2 / 22.5, 2100^2 25.7 / 24.6
+// before the halo exchange of a periodic step, odd periodic (two steps streamed)
+// 2001^2 23.2 / 22.5; FP64 1000^2 15.8 / 12.0, 1200^2 17.2 / 15.3, 1400^2 22.8 / 20.7,
+// 1500^2 23.3 / 24.7.
+// Imaginary time: FP32 100^2 12.4 / 6.9, 1200^2 14.5 / 13.1, 1300^2 16.9 / 16.7, 1400^2
+// 17.4 / 17.9; FP64 100^2 14.7 / 6.8, 1050^2 18.3 / 15.2, 1200^2 19.4 / 17.7, 1300^2 24.5 /
+// 24.7 (the line is drawn at 1080^2).
+// Narrow and flat lattices leave most of their tiles idle: several FP32 steps 2 x 10^6
+// 202 / 479, 61 x 30000 19 / 12, 30 x 10^5 the other way round 14.8 / 14.5, 9 x 300000
+// 12.7 / 17; single FP32 steps 30 x 10^5 18.4 / 21; FP64 125 x 19000 30 / 40, 30 x 30000
+// 24.3 / 23.8; imaginary time FP32 20 x 20000 15.7 / 12.9, 30 x 30000 20.1 / 20.9, FP64
+// 22.4 / 20.3, 28.1 / 32.1.
+struct TileLimit {
+    long cells, area;
+};
+static bool within(const TileLimit &l, int W, int H) { return (long)W * H <= l.cells && tile_area(W, H) <= l.area; }
+static TileLimit limit_one(int esz, bool imag) {
+    if (imag) return {esz == 4 ? 3L << 19 : 9L << 17, 5L << 19};
+    return esz == 4 ? TileLimit{8L << 19, 9L << 19} : TileLimit{15L << 17, 7L << 19};
+}
+static TileLimit limit_several(int esz) {
+    return esz == 4 ? TileLimit{9L << 19, 10L << 19} : TileLimit{5L << 19, 7L << 19};
 }
 
-// The one-plane form of E, no segment height or steps per pass asked
-// for, offsets within 31 bits, and a lattice small enough that a wave's row
-// latency bounds the streaming passes: us per step, streamed against tiles, 64^2
-// FP64 17.3 / 2.8, 256^2 FP64 23.1 / 4.4, FP32 16.6 / 3.2, 512^2 FP32 14.5 / 3.9,
-// 1024^2 FP32 17.0 / 6.6, FP64 23.6 / 10.5, 1600^2 FP64 36.0 / 19.6, 1700^2 FP64
-// 35.8 / 30.0, 1800^2 37.1 / 32.6, 2000^2 FP32 23.7 / 18.3, 2200^2 FP32 24.7 / 31.3,
-// 2048^2 FP64 33.6 / 43.4.  Imaginary time, one step per pass, gives out earlier: closed FP32 100^2
-// 12.4 / 6.9, 1200^2 15.0 / 13.1, 2048^2 23.1 / 28.8, FP64 100^2 14.7 / 6.8, 1024^2
-// 20.7 / 14.8, 1200^2 21.3 / 22.6.
-bool tile_runs(const tsmi_ctx *c) {
-    const bool imag = c->d.imag_time != 0;
-    const long most = imag ? (c->esz == 4 ? 3L << 19 : 9L << 17) : (c->esz == 4 ? 9L << 19 : 5L << 19);
-    return c->ph_mode && c->d.sweeps == 0 && c->d.tile_rows == 0 && c->H > 1 && (long)c->W * c->H <= most &&
-           (long)c->pitch * c->Hd * c->esz < (1L << 31);
+// No segment height or steps per pass asked for, and a lattice small enough that a wave's row latency bounds the
+// streaming passes.
+TileRoute tile_route(const tsmi_desc &d, int W, int H, int n) {
+    if (n <= 0 || d.sweeps != 0 || d.tile_rows != 0 || H <= 1) return kRouteStream;
+    const int esz = d.precision == 32 ? 4 : 8;
+    const bool imag = d.imag_time != 0, closed = !d.periodic_x && !d.periodic_y;
+    const bool even = d.periodic_x && d.periodic_y && d.dim_x % 2 == 0 && d.dim_y % 2 == 0;
+    const bool one = within(limit_one(esz, imag), W, H);
+    const bool several = imag ? one : within(limit_several(esz), W, H);
+    if (closed && (n == 1 ? one : several)) return kRouteClosed;
+    if (even && n >= 3 && several) return kRouteWrap;
+    return !closed && one ? kRouteSeam : kRouteStream;
+}
+
+TileRoute tile_route(const tsmi_ctx *c, int n) {
+    return c->ph_mode ? tile_route(c->d, c->W, c->H, n) : kRouteStream;
+}
+
+void tile_geometry(const tsmi_desc &d, int W, int H, int n, int32_t out[4]) {
+    const TileRoute route = tile_route(d, W, H, n);
+    for (int i = 0; i < 4; ++i) out[i] = 0;
+    if (route == kRouteStream) return;
+    const std::pair<int, int> size(W, H);
+    const int esz = d.precision == 32 ? 4 : 8;
+    int k = 1;
+    if (!d.imag_time && route != kRouteSeam) {
+        const int m = route == kRouteWrap ? n - 2 : n, q = (m + best_steps(&size, 1, esz, m) - 1) / best_steps(&size, 1, esz, m);
+        k = (m + q - 1) / q;
+    }
+    const TilePlan g = plan(&size, 1, esz, k, d.imag_time != 0);
+    const int cols = kTileCols - 2 * kApron * k, rows = g.nw * g.r - 2 * kApron * k;
+    out[0] = g.r;
+    out[1] = g.nw;
+    out[2] = k;
+    out[3] = ((W + cols - 1) / cols) * ((H + rows - 1) / rows);
+}
+
+static TilePlan plan_of(const tsmi_ctx *c, int steps) {
+    const std::pair<int, int> size(c->W, c->H);
+    return plan(&size, 1, c->esz, steps, c->d.imag_time != 0);
 }
 
 int tile_blocks(const tsmi_ctx *c) {
-    const std::pair<int, int> size(c->W, c->H);
-    const TilePlan g = plan(&size, 1, c->esz, 1);
+    const TilePlan g = plan_of(c, 1);
     const int cols = kTileCols - 2 * kApron, rows = g.nw * g.r - 2 * kApron;
     return ((c->W + cols - 1) / cols) * ((c->H + rows - 1) / rows);
 }
 
-static int tile_pass(tsmi_ctx *c, int steps, How how, long double &drift) {
-    return c->esz == 4 ? pass<float>(c, steps, how, drift) : pass<double>(c, steps, how, drift);
+static int tile_pass(tsmi_ctx *c, const TilePlan &g, int steps, How how, long double &drift) {
+    return c->esz == 4 ? pass<float>(c, g, steps, how, drift) : pass<double>(c, g, steps, how, drift);
 }
 
 int tile_passes(tsmi_ctx *c, int n, bool wrap) {
     if (n <= 0) return TSMI_OK;
     const std::pair<int, int> size(c->W, c->H);
     const int k = c->d.imag_time ? 1 : best_steps(&size, 1, c->esz, n), passes = (n + k - 1) / k;
+    const int steps = n / passes, longer = n % passes;   // the first `longer` passes take a step more
     long double drift = 0.0L;
     int st = TSMI_OK;
-    for (int i = 0; i < passes && !st; ++i)
-        st = tile_pass(c, n / passes + (i < n % passes ? 1 : 0), wrap ? kWrap : kClosed, drift);
+    TilePlan g = plan_of(c, steps + (longer > 0));
+    for (int i = 0; i < passes && !st; ++i) {
+        if (i == longer && longer > 0) g = plan_of(c, steps);
+        st = tile_pass(c, g, steps + (i < longer), wrap ? kWrap : kClosed, drift);
+    }
     return st;
 }
 
 int tile_seam_steps(tsmi_ctx *c, int n) {
+    const TilePlan g = plan_of(c, 1);
     long double drift = 0.0L;
     int st = TSMI_OK;
-    for (int i = 0; i < n && !st; ++i) st = tile_pass(c, 1, kSeam, drift);
+    for (int i = 0; i < n && !st; ++i) st = tile_pass(c, g, 1, kSeam, drift);
     return st;
 }
 

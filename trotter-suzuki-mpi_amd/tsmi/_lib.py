@@ -25,7 +25,7 @@ EXPORTS = (
     "tsmi_adjoint_device", "tsmi_batch_create", "tsmi_batch_destroy", "tsmi_batch_set_state",
     "tsmi_batch_set_exp_potential", "tsmi_batch_evolve", "tsmi_batch_get_state", "tsmi_batch_tune",
     "tsmi_batch_info", "tsmi_batch_synchronize", "tsmi_kernel_timing", "tsmi_kernel_time", "tsmi_squared_norm", "tsmi_energy", "tsmi_energy_device_noalloc", "tsmi_expected_values",
-    "tsmi_get_sample", "tsmi_get_state_device", "tsmi_synchronize", "tsmi_geometry", "tsmi_plan_geometry",
+    "tsmi_get_sample", "tsmi_get_state_device", "tsmi_synchronize", "tsmi_geometry", "tsmi_plan_geometry", "tsmi_tile_geometry",
     "tsmi_last_error",
     "tsmi_pair_create", "tsmi_pair_destroy", "tsmi_pair_set_state", "tsmi_pair_set_exp_potential",
     "tsmi_pair_set_potential", "tsmi_pair_evolve", "tsmi_pair_step", "tsmi_pair_rabi", "tsmi_pair_get_state",
@@ -120,6 +120,7 @@ def load():
     L.tsmi_synchronize.argtypes = [C.c_void_p]
     L.tsmi_geometry.argtypes = [C.c_void_p, C.POINTER(C.c_int32)]
     L.tsmi_plan_geometry.argtypes = [C.POINTER(Desc), C.POINTER(C.c_int32)]
+    L.tsmi_tile_geometry.argtypes = [C.POINTER(Desc), C.c_int32, C.POINTER(C.c_int32)]
     L.tsmi_pair_create.argtypes = [C.POINTER(PairDesc), C.POINTER(C.c_void_p)]
     L.tsmi_pair_destroy.argtypes = [C.c_void_p]
     L.tsmi_pair_destroy.restype = None
