@@ -30,6 +30,7 @@ struct tsmi_ctx {
     // steps read it instead of E when ph_mode (every |E| = 1, or every E > 0)
     void *ph_base = nullptr, *ph = nullptr, *ph8 = nullptr;
     bool ph_mode = false;
+    bool e_wraps = false;                // doubly periodic: E's halo is known to repeat the inner cells
     unsigned *flag = nullptr;             // set by the E import when E has no phase form
     double *v_base = nullptr;
     int Wd = 0, Hd = 0;
@@ -90,10 +91,12 @@ int ctx_time_mark(tsmi_ctx *c, int kind, int which);
 // Tile passes (tsmi_tile.hip), asynchronous on c's stream.
 // How a call of n steps runs: streamed; on the tile closed at its edges, several
 // steps per launch; on the doubly periodic lattice, several steps per launch
-// between a first and a last step of their own; step by step, the halo read from
-// the cells it mirrors (one step in imaginary time always).
+// between a first and a last step of their own, E read from the inner cells; step by
+// step, the state's halo read from the cells it mirrors and E's as it is.  E's halo
+// may differ from the inner cells: real time reads those in the streamed two-step
+// passes too, imaginary time (one step per launch) does only when e_wraps.
 enum TileRoute { kRouteStream, kRouteClosed, kRouteWrap, kRouteSeam };
-TileRoute tile_route(const tsmi_desc &d, int W, int H, int n);   // E in one plane
+TileRoute tile_route(const tsmi_desc &d, int W, int H, int n, bool e_wraps);   // E in one plane
 TileRoute tile_route(const tsmi_ctx *c, int n);
 // The cells of the tiles that cover W x H cells: columns in whole tile widths, rows in
 // whole heights of the lowest common tile.

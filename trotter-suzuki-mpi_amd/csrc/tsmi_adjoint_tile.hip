@@ -89,7 +89,8 @@ int pass(tsmi_ctx *c, int steps, const AdjTileIo &io) {
 
 namespace tsmi {
 
-// Closed axes or even doubly periodic ones, no segment height or steps per pass
+// Closed axes or even doubly periodic ones whose E repeats its inner cells on the halo
+// (the passes read it there; the streamed steps read the halo itself), no segment height or steps per pass
 // asked for, and a lattice where tiles measured faster; us per reverse step,
 // streamed against tiles, linear / nonlinear: closed FP32 100^2 20.7 / 29.2 -> 4.3 /
 // 5.3, 1024^2 23.7 / 31.7 -> 11.2 / 15.8, 1200^2 25.3 / 32.1 -> 15.3 / 23.0; FP64
@@ -99,7 +100,8 @@ namespace tsmi {
 // 15000 42 / 20, FP64 10 x 40000 54 / 73.
 bool adjoint_tiles_run(const tsmi_ctx *c) {
     const bool closed = !c->d.periodic_x && !c->d.periodic_y;
-    const bool even = c->d.periodic_x && c->d.periodic_y && c->d.dim_x % 2 == 0 && c->d.dim_y % 2 == 0;
+    const bool even = c->d.periodic_x && c->d.periodic_y && c->d.dim_x % 2 == 0 && c->d.dim_y % 2 == 0 &&
+                      c->e_wraps;
     const long most = c->esz == 4 ? 3L << 19 : 3L << 18;
     return (closed || even) && c->d.tile_rows == 0 && c->d.sweeps == 0 && c->H > 1 &&
            (long)c->W * c->H <= most && tile_area(c->W, c->H) <= most + most / 4 && (long)c->pitch * c->Hd * 8 < (1L << 31);

@@ -306,12 +306,14 @@ __global__ void export_plane(const T *__restrict__ src, double *__restrict__ dst
 // factors (see tsmi_create).  sim may be null (imaginary time: E is real).
 // The same pass writes the one-plane form: phi = -arg(E corr) when |E| = 1
 // (real time), lambda = -ln(E corr) when E > 0 (imaginary time); a cell without
-// that form sets *bad.
+// that form sets bit 0 of *bad.  On a doubly periodic tile (its halo hx and hy wide;
+// else hx = 0) a halo cell that does not repeat the inner cell it mirrors, up to the
+// roundings of a potential evaluated at wrapped coordinates, sets bit 1.
 template <typename T>
 __global__ void __launch_bounds__(kCells) import_exp(const double *__restrict__ sre, const double *__restrict__ sim, double cr, double ci,
                            T *__restrict__ dre, T *__restrict__ dim, T *__restrict__ dph, unsigned *bad, int W,
-                           int H, int pitch) {
-    bool ok = true;
+                           int H, int pitch, int hx, int hy) {
+    bool ok = true, same = true;
     for_cells(W, H, [&](long y, long x) {
         const double er = sre[y * W + x], ei = sim ? sim[y * W + x] : 0.0;
         const double zr = er * cr - ei * ci, zi = er * ci + ei * cr;
@@ -326,25 +328,36 @@ __global__ void __launch_bounds__(kCells) import_exp(const double *__restrict__ 
             ph = zr > 0.0 ? -log(zr) : 0.0;
         }
         dph[y * pitch + x] = (T)ph;
+        if (hx && (x < hx || x >= W - hx || y < hy || y >= H - hy)) {
+            const long sx = x < hx ? x + W - 2 * hx : (x >= W - hx ? x - (W - 2 * hx) : x);
+            const long sy = y < hy ? y + H - 2 * hy : (y >= H - hy ? y - (H - 2 * hy) : y);
+            const double mr = sre[sy * W + sx], mi = sim ? sim[sy * W + sx] : 0.0;
+            const double tol = 1e-12 * (fabs(mr) + fabs(mi));
+            same = same && fabs(er - mr) <= tol && fabs(ei - mi) <= tol;
+        }
     });
-    if (!ok) atomicOr(bad, 1u);
+    if (!ok || !same) atomicOr(bad, (ok ? 0u : 1u) | (same ? 0u : 2u));
 }
 
 // Imports E (FP64 W x H on the device) and decides whether the steps read its
-// one-plane form; syncs to read the import's flag.
+// one-plane form and whether its halo repeats the inner cells; syncs to read the
+// import's flags.
 int launch_import_exp(tsmi_ctx *c, const double *re, const double *im) {
+    const bool both = c->d.periodic_x && c->d.periodic_y;
+    const int hx = both ? c->d.halo_x : 0, hy = both ? c->d.halo_y : 0;
     TSMI_HIP(hipMemsetAsync(c->flag, 0, sizeof(unsigned), c->stream));
     if (c->esz == 4)
         hipLaunchKernelGGL(import_exp<float>, dim3(cell_blocks(c->W, c->H)), dim3(kCells), 0, c->stream, re, im, c->corr_re, c->corr_im,
-                           (float *)c->e_re, (float *)c->e_im, (float *)c->ph, c->flag, c->W, c->H, c->pitch);
+                           (float *)c->e_re, (float *)c->e_im, (float *)c->ph, c->flag, c->W, c->H, c->pitch, hx, hy);
     else
         hipLaunchKernelGGL(import_exp<double>, dim3(cell_blocks(c->W, c->H)), dim3(kCells), 0, c->stream, re, im, c->corr_re, c->corr_im,
-                           (double *)c->e_re, (double *)c->e_im, (double *)c->ph, c->flag, c->W, c->H, c->pitch);
+                           (double *)c->e_re, (double *)c->e_im, (double *)c->ph, c->flag, c->W, c->H, c->pitch, hx, hy);
     TSMI_HIP(hipGetLastError());
-    unsigned bad = 1;
+    unsigned bad = 3;
     TSMI_HIP(hipMemcpyAsync(&bad, c->flag, sizeof(bad), hipMemcpyDeviceToHost, c->stream));
     TSMI_HIP(hipStreamSynchronize(c->stream));
-    c->ph_mode = bad == 0;
+    c->ph_mode = (bad & 1u) == 0;
+    c->e_wraps = both && (bad & 2u) == 0;
     return TSMI_OK;
 }
 
@@ -1174,6 +1187,7 @@ int tsmi_set_potential_exp_device(tsmi_ctx *c, const double *v) {
                            c->pitch);
     TSMI_HIP(hipGetLastError());
     c->ph_mode = true;   // |E| = 1 (real time), E > 0 (imaginary time) by construction
+    c->e_wraps = false;  // not known without a sync
     if (int we = wrap_exp(c)) return we;
     c->has_e = true;
     c->has_v = true;

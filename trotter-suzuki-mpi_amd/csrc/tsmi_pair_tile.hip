@@ -154,10 +154,12 @@ int tile_pass(tsmi_pair *p, int steps, How how, double var, bool rabi, bool firs
 }
 
 // A call of n steps that runs on the doubly periodic lattice between its first and
-// its last step.
+// its last step, E read from the inner cells, as FP32 real time always does with two
+// steps per pass; elsewhere only when the tables' halos repeat them.
 bool wraps(const tsmi_pair *p, int n) {
     const tsmi_desc &d = p->c[0]->d;
-    return d.periodic_x && d.periodic_y && d.dim_x % 2 == 0 && d.dim_y % 2 == 0 && n >= 3;
+    return d.periodic_x && d.periodic_y && d.dim_x % 2 == 0 && d.dim_y % 2 == 0 && n >= 3 &&
+           ((p->esz == 4 && !p->imag) || (p->c[0]->e_wraps && p->c[1]->e_wraps));
 }
 
 // The renormalisation after the last step.

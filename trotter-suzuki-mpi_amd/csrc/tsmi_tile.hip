@@ -269,7 +269,7 @@ static TileLimit limit_several(int esz) {
 
 // No segment height or steps per pass asked for, and a lattice small enough that a wave's row latency bounds the
 // streaming passes.
-TileRoute tile_route(const tsmi_desc &d, int W, int H, int n) {
+TileRoute tile_route(const tsmi_desc &d, int W, int H, int n, bool e_wraps) {
     if (n <= 0 || d.sweeps != 0 || d.tile_rows != 0 || H <= 1) return kRouteStream;
     const int esz = d.precision == 32 ? 4 : 8;
     const bool imag = d.imag_time != 0, closed = !d.periodic_x && !d.periodic_y;
@@ -277,16 +277,16 @@ TileRoute tile_route(const tsmi_desc &d, int W, int H, int n) {
     const bool one = within(limit_one(esz, imag), W, H);
     const bool several = imag ? one : within(limit_several(esz), W, H);
     if (closed && (n == 1 ? one : several)) return kRouteClosed;
-    if (even && n >= 3 && several) return kRouteWrap;
+    if (even && (!imag || e_wraps) && n >= 3 && several) return kRouteWrap;
     return !closed && one ? kRouteSeam : kRouteStream;
 }
 
 TileRoute tile_route(const tsmi_ctx *c, int n) {
-    return c->ph_mode ? tile_route(c->d, c->W, c->H, n) : kRouteStream;
+    return c->ph_mode ? tile_route(c->d, c->W, c->H, n, c->e_wraps) : kRouteStream;
 }
 
 void tile_geometry(const tsmi_desc &d, int W, int H, int n, int32_t out[4]) {
-    const TileRoute route = tile_route(d, W, H, n);
+    const TileRoute route = tile_route(d, W, H, n, true);
     for (int i = 0; i < 4; ++i) out[i] = 0;
     if (route == kRouteStream) return;
     const std::pair<int, int> size(W, H);
