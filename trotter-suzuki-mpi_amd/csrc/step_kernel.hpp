@@ -367,9 +367,10 @@ __device__ __forceinline__ void sincos_t(float x, float *s, float *c) {
 }
 __device__ __forceinline__ void sincos_t(double x, double *s, double *c) { sincos(x, s, c); }
 // The same for |x| <= 2^50: three-part Cody-Waite reduction by pi/2 with fused
-// multiply-adds (159 bits of pi/2; k is exact enough below 2^50 that |r| stays
-// within an ulp of pi/4), then the Taylor polynomials of sin (to r^17) and cos
-// (to r^16), truncation 8e-20 and 2e-18; the quadrant is k mod 4.  For the
+// multiply-adds (159 bits of pi/2), then the Taylor polynomials of sin (to r^17) and
+// cos (to r^16); the quadrant is k mod 4.  Up to 2^40 |r| stays within 1e-3 of pi/4,
+// truncation 9e-20 and 2e-18; near 2^50 the rounding of x 2/pi can leave |r| = 0.95,
+// truncation 3e-18 and 6e-17, still below half an ulp of the result's scale.  For the
 // tile passes: the device sincos carries a reduction for huge arguments (256^2
 // FP64 in a harmonic trap, where angles exceed 1/64, 53.7 us per two-step
 // streaming launch with it).  The streaming passes keep the device sincos: this
@@ -403,9 +404,13 @@ __device__ __forceinline__ void sincos_near(double x, double *s, double *c) {
     *s = (q & 2) ? -a : a;
     *c = ((q + 1) & 2) ? -b : b;
 }
-// An angle above 2^50, whose own rounding (an ulp of 1/8 or more) leaves no
-// phase: brought within sincos_near's range, bounded for every finite angle; an
-// infinite one becomes NaN.
+// An angle above 2^50, whose own rounding (an ulp of 1/8 or more) leaves no phase:
+// brought within sincos_near's range, bounded for every finite angle (to 1e-12 of
+// the rounded angle's phase at 1e20, 0 above 1e31); an infinite one becomes NaN.
+// Only a density gets here, g dt |psi|^2 > 1e15 in one step: the phases of
+// potentials are imported below 2^50.  The device sincos instead, which reduces
+// exactly, costs registers even out of line (148 -> 163 VGPRs, two components 40 -> 47
+// us per step at 1200^2).
 __device__ __forceinline__ double wrap_far(double x) {
     const double n = rint(x * 0.15915494309189534561);
     double r = fma(-n, 6.28318530717958623200, x);

@@ -382,7 +382,10 @@ __global__ void __launch_bounds__(kCells) exp_from_potential(const double *__res
         }
         dre[y * pitch + x] = (T)(er * cr - ei * ci);
         dim[y * pitch + x] = (T)(er * ci + ei * cr);
-        dph[y * pitch + x] = (T)(dt * vi - shift);
+        // past 2^50, where the difference leaves no phase (and sincos_near its range):
+        // the phase of the product just formed
+        const double ph = dt * vi - shift;
+        dph[y * pitch + x] = (T)(!imag && fabs(ph) > 0x1p50 ? -atan2(er * ci + ei * cr, er * cr - ei * ci) : ph);
         vout[y * pitch + x] = vi;
     });
 }
