@@ -116,6 +116,7 @@ adj_tile_kernel(AdjTileParams<T> p) {
 #pragma unroll
         for (int r = -1; r < R; ++r)
             if (WRAP || (y0 + r >= 0 && y0 + r + 1 < p.H)) ok |= 1u << (r + 1);
+        // per wave: see tile_barrier
         const bool edge = X0 < 0 || X0 + kTileCols > p.W || y0 <= 0 || y0 + R >= p.H;
         if (MODE < 0 || edge) {
             adj_tile_steps<T, NL, MODE, R, true>(p, s, e, gr, xch, w, lane, xl, ok);

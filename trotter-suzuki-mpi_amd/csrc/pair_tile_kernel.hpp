@@ -195,7 +195,7 @@ __device__ __forceinline__ void two_field_steps(const P &p, Row<T, 2> (&s)[2][R]
         x.v[buf][0][w + 1][lane] = top;
         x.v[buf][1][w + 1][lane] = bot;
         rest();
-        __syncthreads();
+        tile_barrier();
         const T4 up = x.v[buf][1][w][lane], dn = x.v[buf][0][w + 2][lane];
         buf ^= 1;
 #pragma unroll
@@ -400,6 +400,7 @@ __global__ void __launch_bounds__(NW * kWave, (kPairWaves<T, R, NW, WRAP && MODE
 #pragma unroll
         for (int r = -1; r < R; ++r)
             if (wrap || (y0 + r >= 0 && y0 + r + 1 < p.H)) ok |= 1u << (r + 1);
+        // per wave: see tile_barrier
         const bool edge = X0 < 0 || X0 + kTileCols > p.W || y0 <= 0 || y0 + R >= p.H;
         if (MODE < 0 || edge) {
             pair_tile_steps<T, IMAG, MODE, R, true>(p, s, xch, w, lane, xl, ok, load_ph);
