@@ -20,7 +20,10 @@
 // the rotation -- so a step stores its raw output and its workgroups' partial
 // sums, and every wave of the next launch adds the partials in order and applies
 // the matrix (in FP64, one rounding) as it loads.  pair_finish_kernel does the
-// same after the last step.
+// same after the last step.  The norms after the rotation, the next step's targets,
+// follow from the same sums, unless the rotation cancels most of a component (a state
+// on its way to the antiphase ground state passes there): then the launch that applied
+// the matrix sums what it loaded, and that sum is the target.
 //
 // The edges of a closed tile take per-lane and per-row pair factors; a periodic
 // lattice has none, and its kernels (WRAP) are compiled without that code, which
@@ -37,7 +40,10 @@
 
 namespace tsmi {
 
-constexpr int kPairSums = 3;         // sum |a|^2, sum |b|^2, sum Re(s conj(a) b)
+// Partial sums of an imaginary-time launch: of its output sum |a|^2, sum |b|^2 and
+// sum Re(s conj(a) b); of its input, the pending matrix applied, sum |a|^2, sum |b|^2
+// (only where the matrix asks for them).
+constexpr int kPairSums = 5, kPairOut = 3;
 
 // Waves per SIMD asked of the compiler for a workgroup of NW waves.  FP32 with 4
 // rows: two workgroups of 8 waves on a CU, so that one loads or stores while the
@@ -50,7 +56,7 @@ struct PairNorm {
     const double *part;              // partial sums [kPairSums][cap] of the step before (nullptr: none)
     const int *n;                    // their count
     int cap;
-    const double *norm_in;           // squared-norm targets of that step (0: no division)
+    const double *norm_in;           // squared-norm targets of that step (0: no division, < 0: the input's sum)
     double *norm_out;                // targets after it
     double cc, cs_r, cs_i;           // its rotation
     int rabi;
@@ -60,26 +66,46 @@ struct PairNorm {
 // a <- aa a + ab b, b <- bb b + ba a; off-diagonals (x, y) = x + i y.
 struct PairMatrix {
     double aa, bb, ab_r, ab_i, ba_r, ba_i;
+    bool sums;                       // a target is the sum over what the matrix gives
 };
+
+// Partial sums j0 .. j0 + N - 1 added up in order, the same bits in every wave.
+template <int N>
+__device__ __forceinline__ void pair_add(const PairNorm &q, int j0, int lane, double (&s)[N]) {
+    const int n = __builtin_amdgcn_readfirstlane(*q.n);
+    double e[N];
+#pragma unroll
+    for (int j = 0; j < N; ++j) s[j] = e[j] = 0.0;
+    for (int i = lane; i < n; i += kWave)
+#pragma unroll
+        for (int j = 0; j < N; ++j) neumaier(s[j], e[j], q.part[(long)(j0 + j) * q.cap + i]);
+#pragma unroll
+    for (int j = 0; j < N; ++j) {
+        s[j] += e[j];
+        for (int o = kWave / 2; o > 0; o >>= 1) s[j] += __shfl_xor(s[j], o, kWave);
+    }
+}
+
+// A norm after a rotation, of the terms it is made of: relative to the total, or -1
+// where they cancel to less than a quarter and its relative error would exceed 1e-15.
+__device__ __forceinline__ double pair_target(double q, double terms, double total, double tot_norm) {
+    return q >= 0.25 * terms && q > 0.0 ? q / total * tot_norm : -1.0;
+}
 
 // The matrix of a pending renormalisation, the same bits in every wave; the
 // wave with `store` also leaves the new targets.
 __device__ __forceinline__ PairMatrix pair_matrix(const PairNorm &q, int lane, bool store) {
-    PairMatrix m = {1.0, 1.0, 0.0, 0.0, 0.0, 0.0};
+    PairMatrix m = {1.0, 1.0, 0.0, 0.0, 0.0, 0.0, false};
     if (!q.part) return m;
-    const int n = __builtin_amdgcn_readfirstlane(*q.n);
-    double s[kPairSums], e[kPairSums];
-#pragma unroll
-    for (int j = 0; j < kPairSums; ++j) s[j] = e[j] = 0.0;
-    for (int i = lane; i < n; i += kWave)
-#pragma unroll
-        for (int j = 0; j < kPairSums; ++j) neumaier(s[j], e[j], q.part[(long)j * q.cap + i]);
-#pragma unroll
-    for (int j = 0; j < kPairSums; ++j) {
-        s[j] += e[j];
-        for (int o = kWave / 2; o > 0; o >>= 1) s[j] += __shfl_xor(s[j], o, kWave);
+    double s[kPairOut];
+    pair_add(q, 0, lane, s);
+    double na = q.norm_in[0], nb = q.norm_in[1];
+    if (na < 0.0 || nb < 0.0) {
+        double t[2];
+        pair_add(q, kPairOut, lane, t);
+        if (na < 0.0) na = t[0] * q.dxdy;
+        if (nb < 0.0) nb = t[1] * q.dxdy;
     }
-    const double na = q.norm_in[0], nb = q.norm_in[1];
     const double ia = na != 0.0 ? 1.0 / sqrt(s[0] * q.dxdy / na) : 1.0;
     const double ib = nb != 0.0 ? 1.0 / sqrt(s[1] * q.dxdy / nb) : 1.0;
     if (!q.rabi) {
@@ -105,9 +131,12 @@ __device__ __forceinline__ PairMatrix pair_matrix(const PairNorm &q, int lane, b
     m.ab_i = q.cs_i * ib * f;
     m.ba_r = q.cs_r * ia * f;
     m.ba_i = -q.cs_i * ia * f;
+    const double ta = pair_target(qa, c2 * va + s2 * vb, qa + qb, q.tot_norm);
+    const double tb = pair_target(qb, c2 * vb + s2 * va, qa + qb, q.tot_norm);
+    m.sums = ta < 0.0 || tb < 0.0;
     if (store) {
-        q.norm_out[0] = qa / (qa + qb) * q.tot_norm;
-        q.norm_out[1] = qb / (qa + qb) * q.tot_norm;
+        q.norm_out[0] = ta;
+        q.norm_out[1] = tb;
     }
     return m;
 }
@@ -381,7 +410,11 @@ __global__ void __launch_bounds__(NW * kWave, (kPairWaves<T, R, NW, WRAP && MODE
                 seam_load<T>(q, make_rsrc(p.in_re[c], bytes), make_rsrc(p.in_im[c], bytes), xl, y0 + r, row_bytes,
                              s[c][r]);
     }
+    const bool own = lane >= A / 2 && lane < A / 2 + p.cols / 2 && xl < p.W;
+    const int y_lo = seg * p.rows, y_hi = min(p.H, y_lo + p.rows);
+    __shared__ double red[IMAG ? kPairSums : 1][NW];
     if constexpr (IMAG) {
+        if (lane == 0) red[kPairOut][w] = red[kPairOut + 1][w] = 0.0;
         if (p.pend.part) {
             const PairMatrix m = pair_matrix(p.pend, lane, blockIdx.x == 0 && threadIdx.x == 0);
 #pragma unroll
@@ -389,6 +422,24 @@ __global__ void __launch_bounds__(NW * kWave, (kPairWaves<T, R, NW, WRAP && MODE
 #pragma unroll
                 for (int k = 0; k < 2; ++k)
                     pair_apply(m, s[0][r].re[k], s[0][r].im[k], s[1][r].re[k], s[1][r].im[k]);
+            if (__builtin_expect(m.sums, 0)) {
+                for (int c = 0; c < 2; ++c) {
+                    double q = 0.0, e = 0.0;
+#pragma unroll
+                    for (int r = 0; r < R; ++r)
+#pragma unroll
+                        for (int k = 0; k < 2; ++k) {
+                            const int y = y0 + r, x = xl + k;
+                            const double re = c ? s[1][r].re[k] : s[0][r].re[k], im = c ? s[1][r].im[k] : s[0][r].im[k];
+                            const bool in = own && y >= y_lo && y < y_hi && y >= p.iy0 && y < p.iy1 && x >= p.ix0 &&
+                                            x < p.ix1;
+                            neumaier(q, e, in ? re * re + im * im : 0.0);
+                        }
+                    double t = q + e;
+                    for (int o = kWave / 2; o > 0; o >>= 1) t += __shfl_xor(t, o, kWave);
+                    if (lane == 0) red[kPairOut + c][w] = t;
+                }
+            }
         }
     }
     __syncthreads();
@@ -409,8 +460,6 @@ __global__ void __launch_bounds__(NW * kWave, (kPairWaves<T, R, NW, WRAP && MODE
         }
     }
 
-    const bool own = lane >= A / 2 && lane < A / 2 + p.cols / 2 && xl < p.W;
-    const int y_lo = seg * p.rows, y_hi = min(p.H, y_lo + p.rows);
 #pragma unroll
     for (int r = 0; r < R; ++r) {
         const int y = y0 + r;
@@ -423,14 +472,14 @@ __global__ void __launch_bounds__(NW * kWave, (kPairWaves<T, R, NW, WRAP && MODE
         }
     }
     if constexpr (IMAG) {
-        double q[kPairSums], e[kPairSums];
+        double q[kPairOut], e[kPairOut];
 #pragma unroll
-        for (int j = 0; j < kPairSums; ++j) q[j] = e[j] = 0.0;
+        for (int j = 0; j < kPairOut; ++j) q[j] = e[j] = 0.0;
 #pragma unroll
         for (int r = 0; r < R; ++r) {
             const int y = y0 + r;
             if (!(y >= y_lo && y < y_hi && y >= p.iy0 && y < p.iy1)) continue;   // uniform
-            double v[kPairSums] = {0.0, 0.0, 0.0};
+            double v[kPairOut] = {0.0, 0.0, 0.0};
 #pragma unroll
             for (int k = 0; k < 2; ++k) {
                 const bool in = own && xl + k >= p.ix0 && xl + k < p.ix1;
@@ -440,11 +489,10 @@ __global__ void __launch_bounds__(NW * kWave, (kPairWaves<T, R, NW, WRAP && MODE
                 v[2] += in ? p.s_r * (ar * br + ai * bi) - p.s_i * (ar * bi - ai * br) : 0.0;
             }
 #pragma unroll
-            for (int j = 0; j < kPairSums; ++j) neumaier(q[j], e[j], v[j]);
+            for (int j = 0; j < kPairOut; ++j) neumaier(q[j], e[j], v[j]);
         }
-        __shared__ double red[kPairSums][NW];
 #pragma unroll
-        for (int j = 0; j < kPairSums; ++j) {
+        for (int j = 0; j < kPairOut; ++j) {
             double t = q[j] + e[j];
             for (int o = kWave / 2; o > 0; o >>= 1) t += __shfl_xor(t, o, kWave);
             if (lane == 0) red[j][w] = t;
@@ -459,21 +507,52 @@ __global__ void __launch_bounds__(NW * kWave, (kPairWaves<T, R, NW, WRAP && MODE
     }
 }
 
-// The pending matrix applied to both tiles in place; the new targets stored.
+// The pending matrix applied to both tiles in place, the new targets stored, and the
+// sums they may stand for (sums 3 and 4 of part_out, as an imaginary-time launch's).
+constexpr int kFinishBlocks = 256;
 template <typename T>
-__global__ void __launch_bounds__(256) pair_finish_kernel(T *ar, T *ai, T *br, T *bi, int W, int H, int pitch,
-                                                          PairNorm q) {
-    const PairMatrix m = pair_matrix(q, threadIdx.x & (kWave - 1), blockIdx.x == 0 && threadIdx.x == 0);
+__global__ void __launch_bounds__(256) pair_finish_kernel(T *ar, T *ai, T *br, T *bi, int W, int H, int pitch, int ix0,
+                                                          int ix1, int iy0, int iy1, PairNorm q, double *part_out,
+                                                          int *n_out) {
+    const int lane = threadIdx.x & (kWave - 1);
+    const PairMatrix m = pair_matrix(q, lane, blockIdx.x == 0 && threadIdx.x == 0);
     const long n = (long)W * H;
+    double t[2] = {0.0, 0.0}, e[2] = {0.0, 0.0};
     for (long i = blockIdx.x * 256L + threadIdx.x; i < n; i += gridDim.x * 256L) {
-        const long y = i / W, k = y * pitch + (i - y * W);
+        const long y = i / W, x = i - y * W, k = y * pitch + x;
         T xr = ar[k], xi = ai[k], yr = br[k], yi = bi[k];
         pair_apply(m, xr, xi, yr, yi);
         ar[k] = xr;
         ai[k] = xi;
         br[k] = yr;
         bi[k] = yi;
+        if (m.sums && x >= ix0 && x < ix1 && y >= iy0 && y < iy1) {
+            neumaier(t[0], e[0], double(xr) * double(xr) + double(xi) * double(xi));
+            neumaier(t[1], e[1], double(yr) * double(yr) + double(yi) * double(yi));
+        }
     }
+    __shared__ double red[2][256 / kWave];
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+        t[c] += e[c];
+        for (int o = kWave / 2; o > 0; o >>= 1) t[c] += __shfl_xor(t[c], o, kWave);
+        if (lane == 0) red[c][threadIdx.x / kWave] = t[c];
+    }
+    __syncthreads();
+    if (threadIdx.x < 2) {
+        double a = 0.0, c = 0.0;
+        for (int i = 0; i < 256 / kWave; ++i) neumaier(a, c, red[threadIdx.x][i]);
+        part_out[(long)(kPairOut + threadIdx.x) * q.cap + blockIdx.x] = a + c;
+    }
+    if (blockIdx.x == 0 && threadIdx.x == 0) *n_out = gridDim.x;
+}
+
+// The targets a finished call leaves: those of its last rotation, or the sums.
+template <typename = void>
+__global__ void __launch_bounds__(kWave) pair_targets_kernel(PairNorm q) {
+    double t[2];
+    pair_add(q, kPairOut, threadIdx.x, t);
+    if (threadIdx.x < 2 && q.norm_out[threadIdx.x] < 0.0) q.norm_out[threadIdx.x] = t[threadIdx.x] * q.dxdy;
 }
 
 }  // namespace tsmi

@@ -163,21 +163,24 @@ bool wraps(const tsmi_pair *p, int n) {
 }
 
 // The renormalisation after the last step.
+template <typename T>
 int finish(tsmi_pair *p, double var, bool rabi) {
-    const PairNorm q = pending(p, var, rabi);
-    const int cur = p->c[0]->cur;
-    const int blocks = (int)std::min<long>(256, ((long)p->W * p->H + 1023) / 1024);
-    hipStream_t s = p->c[0]->stream;
+    PairNorm q = pending(p, var, rabi);
     tsmi_ctx *a = p->c[0], *b = p->c[1];
-    if (p->esz == 4)
-        hipLaunchKernelGGL((pair_finish_kernel<float>), dim3(blocks), dim3(256), 0, s, (float *)a->psi_re[cur],
-                           (float *)a->psi_im[cur], (float *)b->psi_re[cur], (float *)b->psi_im[cur], p->W, p->H,
-                           p->pitch, q);
-    else
-        hipLaunchKernelGGL((pair_finish_kernel<double>), dim3(blocks), dim3(256), 0, s, (double *)a->psi_re[cur],
-                           (double *)a->psi_im[cur], (double *)b->psi_re[cur], (double *)b->psi_im[cur], p->W, p->H,
-                           p->pitch, q);
-    const hipError_t e = hipGetLastError();
+    const int cur = a->cur, blocks = (int)std::min<long>(kFinishBlocks, ((long)p->W * p->H + 1023) / 1024);
+    p->slot = 1 - p->slot;
+    double *part_out = p->tile_part + (size_t)p->slot * kPairSums * (size_t)p->part_cap;
+    int *n_out = p->tile_n + p->slot;
+    hipLaunchKernelGGL((pair_finish_kernel<T>), dim3(blocks), dim3(256), 0, a->stream, (T *)a->psi_re[cur],
+                       (T *)a->psi_im[cur], (T *)b->psi_re[cur], (T *)b->psi_im[cur], p->W, p->H, p->pitch, p->ix0,
+                       p->ix1, p->iy0, p->iy1, q, part_out, n_out);
+    hipError_t e = hipGetLastError();
+    if (e == hipSuccess && rabi) {
+        q.part = part_out;
+        q.n = n_out;
+        hipLaunchKernelGGL(pair_targets_kernel<>, dim3(1), dim3(kWave), 0, a->stream, q);
+        e = hipGetLastError();
+    }
     if (e != hipSuccess) return set_error(TSMI_E_HIP, std::string("pair_finish_kernel: ") + hipGetErrorString(e));
     p->norm_slot = 1 - p->norm_slot;
     return TSMI_OK;
@@ -190,7 +193,7 @@ namespace tsmi {
 int pair_tile_blocks(const tsmi_pair *p) {
     const TwoFieldPlan a = two_field_plan(p->W, p->H, p->esz, 1, false, cost(p->esz, false)),
                        b = two_field_plan(p->W, p->H, p->esz, 1, true, cost(p->esz, one_form(p)));
-    return std::max(a.strips * a.segs, b.strips * b.segs);
+    return std::max({a.strips * a.segs, b.strips * b.segs, kFinishBlocks});
 }
 
 // No segment height or steps per pass asked for, offsets within 31 bits, and a
@@ -244,7 +247,7 @@ int pair_tile_evolve(tsmi_pair *p, int n, bool rabi) {
         // differs from that of the cell it mirrors; a call of two steps
         for (int j = 0; j < n && !st; ++j) passes(1, j == 0 ? kClosed : kSeam);
     }
-    if (!st && p->imag) st = finish(p, 0.5, rabi);
+    if (!st && p->imag) st = p->esz == 4 ? finish<float>(p, 0.5, rabi) : finish<double>(p, 0.5, rabi);
     return st;
 }
 
