@@ -9,13 +9,17 @@
 // single-context one: tsmi_evolve semantics per lattice, including the skipped
 // exchange after the last step of a call.
 //
-// Lattices are in one of two groups.  Group 1 holds the lattices that take two
-// real-time steps per pass (both axes closed or both periodic, sweeps != 1);
+// Lattices are in one of four groups.  Streamed: group 1 holds the lattices that take
+// two real-time steps per pass (both axes closed or both periodic, sweeps != 1);
 // group 0 the rest (imaginary time, mixed boundaries, sweeps == 1), stepped one
 // step per pass.  Group 1 follows the single context's sequence: on the 8-wide
 // halo layout of a doubly periodic lattice, a single step, then fused passes
-// each followed by the 8-wide wrap, then the last single step.  The two groups
-// are independent; when both are present their launches go to two streams.
+// each followed by the 8-wide wrap, then the last single step.  Register tiles, for
+// batches of few cells whose E tables all have the phase form (tile_kernel.hpp): group
+// 2 holds closed and even doubly periodic lattices, several steps per launch; group 3
+// mixed and odd periodic ones, one step per launch, the halo read from its mirrors.
+// The groups are independent; the launches of 0 and 3 go to a stream of their own when
+// the others have some too.
 //
 // tsmi_batch_evolve records the launch sequence of an n-step call in a HIP graph
 // the first time that (n, buffer parities) is seen and replays it after.
@@ -46,7 +50,7 @@ using namespace tsmi;
 namespace {
 
 constexpr int kBlock = 256;
-constexpr int kGroups = 4;                     // see the top
+constexpr int kGroups = 4;                     // 0, 1 streamed, 2, 3 tiles: see the top
 constexpr int kDefaultSegRows = 64;
 constexpr int kVecF = 2;                       // elements per lane of the fused passes
 // Most cells of a batch run as tiles, and most cells of its tiles: each lattice's
@@ -97,13 +101,23 @@ struct GraphRec {
     int end[kGroups] = {0, 0, 0, 0};
 };
 
-// One tile pass over a tile group: its shape, parameters per buffer parity, items.
+// One tile pass over a tile group: its shape, its items, its parameters.  A pass
+// rounds its last step's modulus once (tile_params: drift); as a pass is replayed,
+// that would repeat and drift the norm by up to 1.1e-16 per pass (64^2 FP64, 6000
+// steps: 3.7e-13).  So there are several sets, each taking back what the ones before
+// it left, run through in order; set i reads buffer i mod 2.
+constexpr int kParamSets = 8;
 struct TilePass {
     TilePlan g;
-    void *params[2] = {nullptr, nullptr};
+    void *params[kParamSets] = {};
     int2 *items = nullptr;
     int n_items = 0;
 };
+void free_tile_pass(TilePass &t) {
+    for (void *p : t.params)
+        if (p) (void)hipFree(p);
+    if (t.items) (void)hipFree(t.items);
+}
 enum TileHow { kClosed, kWrap, kSeam };   // as tsmi_tile.hip's passes
 
 }  // namespace
@@ -144,11 +158,7 @@ void drop_graphs(tsmi_batch *b) {
 }
 
 void drop_tile_passes(tsmi_batch *b) {
-    for (auto &t : b->tile_passes) {
-        void *ptrs[] = {t.second.params[0], t.second.params[1], t.second.items};
-        for (void *p : ptrs)
-            if (p) (void)hipFree(p);
-    }
+    for (auto &t : b->tile_passes) free_tile_pass(t.second);
     b->tile_passes.clear();
 }
 
@@ -437,7 +447,7 @@ int build_tile_pass(tsmi_batch *b, int group, TileHow how, int steps, TilePass *
     TilePass t;
     t.g = tile_plan(tile_sizes(b, group), b->esz, steps);
     if (t.g.r == 0) return set_error(TSMI_E_INVALID, "batch tile pass: no tile for this many steps");
-    std::vector<TileParams<T>> h[2];
+    std::vector<TileParams<T>> h[kParamSets];
     std::vector<int2> items;
     char *a = b->arena;
     for (const Lattice &L : b->lat) {
@@ -446,36 +456,36 @@ int build_tile_pass(tsmi_batch *b, int group, TileHow how, int steps, TilePass *
         const TileFactors f = {k.mH, k.tH, k.mV, k.tV, k.unH, k.unV, k.c_nl_s, k.c_lhy_s, k.corr_abs,
                                L.d.delta_t / (4. * L.d.mass * L.d.delta_y * L.d.delta_y)};
         const bool wrap = how == kWrap && L.d.periodic_x;
-        long double drift = 0.0L;   // within the pass
+        long double drift = 0.0L;   // over the sets
         TileParams<T> p;
         std::memset(&p, 0, sizeof(p));
-        tile_params<T>(p, f, t.g, L.W, L.H, L.pitch, wrap ? L.d.dim_x : 0, wrap ? L.d.dim_y : 0, steps, drift);
         p.seam = how == kSeam;
         p.px = L.d.periodic_x != 0; p.py = L.d.periodic_y != 0;
         p.ph = (const T *)(a + L.ph);
-        const int i = (int)h[0].size(), tiles = p.n_strips * ((L.H + p.rows - 1) / p.rows);
-        for (int c = 0; c < 2; ++c) {
+        for (int j = 0; j < kParamSets; ++j) {
+            const int c = j & 1;
+            tile_params<T>(p, f, t.g, L.W, L.H, L.pitch, wrap ? L.d.dim_x : 0, wrap ? L.d.dim_y : 0, steps, drift);
             p.in_re = (const T *)(a + L.psi[c][0]);
             p.in_im = (const T *)(a + L.psi[c][1]);
             p.out_re = (T *)(a + L.psi[1 - c][0]);
             p.out_im = (T *)(a + L.psi[1 - c][1]);
-            h[c].push_back(p);
+            h[j].push_back(p);
         }
+        const int i = (int)h[0].size() - 1, tiles = p.n_strips * ((L.H + p.rows - 1) / p.rows);
         for (int j = 0; j < tiles; ++j) items.push_back(make_int2(i, j));
     }
     t.n_items = (int)items.size();
     const size_t pb = h[0].size() * sizeof(TileParams<T>), ib = items.size() * sizeof(int2);
     hipError_t e = hipMalloc((void **)&t.items, ib);
-    for (int c = 0; c < 2 && e == hipSuccess; ++c) {
+    for (int c = 0; c < kParamSets && e == hipSuccess; ++c) {
         e = hipMalloc(&t.params[c], pb);
         if (e == hipSuccess) e = hipMemcpyAsync(t.params[c], h[c].data(), pb, hipMemcpyHostToDevice, b->stream);
     }
     if (e == hipSuccess) e = hipMemcpyAsync(t.items, items.data(), ib, hipMemcpyHostToDevice, b->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(b->stream);
     if (e != hipSuccess) {
-        void *ptrs[] = {t.params[0], t.params[1], t.items};
-        for (void *p : ptrs)
-            if (p) (void)hipFree(p);
+        (void)hipStreamSynchronize(b->stream);   // copies from h that were queued
+        free_tile_pass(t);
         return set_error(TSMI_E_HIP, std::string("batch tile pass: ") + hipGetErrorString(e));
     }
     *out = t;
@@ -526,10 +536,12 @@ int prepare_tiles(tsmi_batch *b, int n) {
 
 int run_tiles(tsmi_batch *b, hipStream_t s, int group, int n, int *cur) {
     if (b->n_tiled[group] == 0) return TSMI_OK;
+    int set = cur[group];   // its parity is the buffer's throughout
     return tile_sequence(b, group, n, [&](TileHow how, int steps) -> int {
         const TilePass &t = b->tile_passes.at(std::make_tuple(group, (int)how, steps));
-        const int st = tile_batch_launch(b->esz, b->lhy, b->mode, t.g, t.params[cur[group]], t.items, t.n_items, s);
+        const int st = tile_batch_launch(b->esz, b->lhy, b->mode, t.g, t.params[set], t.items, t.n_items, s);
         cur[group] ^= 1;
+        set = (set + 1) % kParamSets;
         return st;
     });
 }
