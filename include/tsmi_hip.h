@@ -48,7 +48,8 @@ typedef struct {
     int32_t sweeps;                /* steps per pass over HBM in tsmi_evolve: 0 chooses
                                       (2 where exact; up to 8 on small lattices), 1, or 2
                                       (real time with both axes closed or both periodic
-                                      only)                                              */
+                                      only; odd periodic extents, where two are not
+                                      exact, still take one)                             */
     double delta_t, mass;
     double coupling;               /* g (Hamiltonian::coupling_a)                        */
     double coupling_lhy;           /* g_LHY (Hamiltonian::LeeHuangYang_coupling_a)       */
@@ -164,7 +165,7 @@ int tsmi_adjoint_device(tsmi_ctx *ctx, const double *g_re, const double *g_im, d
  * own descriptor (size, boundaries, dt, mass, spacing, couplings); precision,
  * time direction and whether g_LHY != 0 are common to the batch.  Each lattice
  * gets exactly tsmi_evolve's steps.  A lattice whose descriptor allows two steps
- * per pass (sweeps 0 or 2, real time, both axes closed or both periodic) is
+ * per pass (sweeps 0 or 2, real time, both axes closed, or both periodic and even) is
  * advanced like a context with that setting; the others one step per pass.  A
  * pass of the batch is one persistent launch over all lattices of its kind
  * (plus one halo-exchange launch when some of them are periodic).
@@ -207,8 +208,8 @@ int tsmi_batch_synchronize(tsmi_batch *batch);
  * src/cpukernel.cpp:332-335); a.norm_target / b.norm_target = the squared norms
  * of the two states when the kernel is built (src/solver.cpp:153-159), the
  * imaginary-time targets.  a.sweeps picks the steps per pass of tsmi_pair_evolve:
- * 0 chooses two wherever they are exact (FP32, real time, both axes closed or both
- * periodic, and both E tables of unit modulus; otherwise one), 1 forces one, 2
+ * 0 chooses two wherever they are exact (FP32, real time, both axes closed, or both
+ * periodic and even, and both E tables of unit modulus; otherwise one), 1 forces one, 2
  * requires a lattice and precision where two can run.
  * b.sweeps is not read. */
 typedef struct {

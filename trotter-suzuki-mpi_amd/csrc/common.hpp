@@ -12,6 +12,19 @@ int set_error(int code, const std::string &msg);
 // Validates a descriptor; `who` prefixes the message.  TSMI_OK or an error code.
 int check_desc(const tsmi_desc &d, const char *who);
 
+// Two steps per pass can be asked for: real time, both axes closed or both periodic.
+inline bool two_steps_allowed(const tsmi_desc &d) {
+    return !d.imag_time && (d.periodic_x != 0) == (d.periodic_y != 0);
+}
+// ... and are two single steps exactly: on a periodic axis of odd extent the pair
+// pattern of a halo cell differs from that of the cell it mirrors, so that the second
+// step, which no exchange precedes, would split the kinetic term otherwise next to
+// the seam (45 x 38 odd periodic, 6 steps: 6e-5 off the reference's step; 1601^2 3e-7).
+// Such a lattice takes one step per pass, also where two are asked for.
+inline bool two_steps_exact(const tsmi_desc &d) {
+    return two_steps_allowed(d) && (!d.periodic_x || (d.dim_x % 2 == 0 && d.dim_y % 2 == 0));
+}
+
 // Largest even segment height whose rows plus the apron rows of a pass
 // (apron_rows in all: 8 for one step per pass, 16 for two) keep a wave's 32-bit
 // byte offsets valid for a row pitch of `pitch` elements (FP64 planes): the

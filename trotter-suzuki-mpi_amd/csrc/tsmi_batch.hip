@@ -10,9 +10,8 @@
 // exchange after the last step of a call.
 //
 // Lattices are in one of four groups.  Streamed: group 1 holds the lattices that take
-// two real-time steps per pass (both axes closed or both periodic, sweeps != 1);
-// group 0 the rest (imaginary time, mixed boundaries, sweeps == 1), stepped one
-// step per pass.  Group 1 follows the single context's sequence: on the 8-wide
+// two real-time steps per pass (both axes closed, or both periodic and of even
+// extents, sweeps != 1); group 0 the rest, stepped one step per pass.  Group 1 follows the single context's sequence: on the 8-wide
 // halo layout of a doubly periodic lattice, a single step, then fused passes
 // each followed by the 8-wide wrap, then the last single step.  Register tiles, for
 // batches of few cells whose E tables all have the phase form (tile_kernel.hpp): group
@@ -748,7 +747,7 @@ int tsmi_batch_create(const tsmi_desc *descs, int32_t n, tsmi_batch **out) {
                              "tsmi_batch_create: all lattices need the same precision, time direction and LHY setting");
         if (d.sweeps < 0 || d.sweeps > 2)
             return set_error(TSMI_E_INVALID, "tsmi_batch_create: sweeps must be 0, 1 or 2");
-        if (d.sweeps == 2 && (d.imag_time || (d.periodic_x != 0) != (d.periodic_y != 0)))
+        if (d.sweeps == 2 && !two_steps_allowed(d))
             return set_error(TSMI_E_UNSUPPORTED, "tsmi_batch_create: two steps per pass need real time and both "
                                                  "axes closed or both periodic");
     }
@@ -771,7 +770,7 @@ int tsmi_batch_create(const tsmi_desc *descs, int32_t n, tsmi_batch **out) {
         L.H = d.dim_y + (d.periodic_y ? 2 * d.halo_y : 0);
         // 0 chooses two steps per pass wherever they are exact (the autotuner may
         // go back to one); 2 insists on them
-        L.fusable = d.sweeps != 1 && !d.imag_time && (d.periodic_x != 0) == (d.periodic_y != 0);
+        L.fusable = d.sweeps != 1 && two_steps_exact(d);
         L.fused = L.fusable;
         L.tunable = L.fusable && d.sweeps == 0;
         L.halo8 = L.fusable && d.periodic_x;

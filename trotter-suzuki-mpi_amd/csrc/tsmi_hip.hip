@@ -1027,13 +1027,11 @@ int tsmi_create(const tsmi_desc *desc, tsmi_ctx **out) {
     const long long W = (long long)d.dim_x + (d.periodic_x ? 2 * d.halo_x : 0);
     const long long H = (long long)d.dim_y + (d.periodic_y ? 2 * d.halo_y : 0);
     if (d.sweeps < 0 || d.sweeps > 2) return fail(TSMI_E_INVALID, "tsmi_create: sweeps must be 0, 1 or 2");
-    // two steps per pass: real time, both axes closed or both periodic
-    const bool fusable = !d.imag_time && ((d.periodic_x && d.periodic_y) || (!d.periodic_x && !d.periodic_y));
-    if (d.sweeps == 2 && !fusable)
+    if (d.sweeps == 2 && !two_steps_allowed(d))
         return fail(TSMI_E_UNSUPPORTED,
                     "tsmi_create: two steps per pass need real time and both axes closed or both periodic");
     // 0 chooses two steps per pass wherever they are exact
-    const int sweeps = (d.sweeps != 1 && fusable) ? 2 : 1;
+    const int sweeps = d.sweeps != 1 && two_steps_exact(d) ? 2 : 1;
     const bool halo8 = sweeps == 2 && d.periodic_x && d.periodic_y;
     const long long Wd = W + (halo8 ? 2 * d.halo_x : 0), Hd = H + (halo8 ? 2 * d.halo_y : 0);
     const long long pitch = (Wd + 63) / 64 * 64;
@@ -1483,11 +1481,10 @@ int tsmi_plan_geometry(const tsmi_desc *desc, int32_t out[12]) {
     const tsmi_desc &d = *desc;
     if (int st = check_desc(d, "tsmi_plan_geometry")) return st;
     if (d.sweeps < 0 || d.sweeps > 2) return fail(TSMI_E_INVALID, "tsmi_plan_geometry: sweeps must be 0, 1 or 2");
-    const bool fusable = !d.imag_time && ((d.periodic_x && d.periodic_y) || (!d.periodic_x && !d.periodic_y));
-    if (d.sweeps == 2 && !fusable)
+    if (d.sweeps == 2 && !two_steps_allowed(d))
         return fail(TSMI_E_UNSUPPORTED,
                     "tsmi_plan_geometry: two steps per pass need real time and both axes closed or both periodic");
-    const int sweeps = (d.sweeps != 1 && fusable) ? 2 : 1;
+    const int sweeps = d.sweeps != 1 && two_steps_exact(d) ? 2 : 1;
     const bool halo8 = sweeps == 2 && d.periodic_x && d.periodic_y;
     const int W = d.dim_x + (d.periodic_x ? 2 * d.halo_x : 0), H = d.dim_y + (d.periodic_y ? 2 * d.halo_y : 0);
     const int Wd = W + (halo8 ? 2 * d.halo_x : 0), Hd = H + (halo8 ? 2 * d.halo_y : 0);

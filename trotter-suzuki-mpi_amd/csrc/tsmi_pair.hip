@@ -344,7 +344,7 @@ int tsmi_pair_create(const tsmi_pair_desc *pd, tsmi_pair **out) {
     if (da.sweeps == 2 && !fusable)
         return set_error(TSMI_E_UNSUPPORTED, "tsmi_pair_create: two steps per pass need FP32, real time and both "
                                              "axes closed or both periodic");
-    const bool fused = fusable && da.sweeps != 1;
+    const bool fused = fusable && two_steps_exact(da) && da.sweeps != 1;
     tsmi_pair *p = new tsmi_pair();
     auto bail = [&](int code) {
         free_pair(p);

@@ -244,8 +244,8 @@ long tile_area(int W, int H) { return (W + 119L) / 120 * 120 * ((H + 23L) / 24 *
 // 27.9, 2100^2 31.0 / 32.9 (the FP64 line is drawn at 1620^2).
 // One step per pass (single steps, short calls, mixed axes, odd periodic extents):
 // FP32 1000^2 17.9 / 9.0, 1800^2 22.9 / 18.9, 2000^2 24.2 / 22.5, 2100^2 25.7 / 24.6
-// before the halo exchange of a periodic step, odd periodic (two steps streamed)
-// 2001^2 23.2 / 22.5; FP64 1000^2 15.8 / 12.0, 1200^2 17.2 / 15.3, 1400^2 22.8 / 20.7,
+// before the halo exchange of a periodic step, mixed or odd periodic axes 2001^2 26.2 /
+// 22.5 with it; FP64 1000^2 15.8 / 12.0, 1200^2 17.2 / 15.3, 1400^2 22.8 / 20.7,
 // 1500^2 23.3 / 24.7.
 // Imaginary time: FP32 100^2 12.4 / 6.9, 1200^2 14.5 / 13.1, 1300^2 16.9 / 16.7, 1400^2
 // 17.4 / 17.9; FP64 100^2 14.7 / 6.8, 1050^2 18.3 / 15.2, 1200^2 19.4 / 17.7, 1300^2 24.5 /
