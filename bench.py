@@ -157,6 +157,30 @@ def time_precision(prec, lat, psi_re, psi_im, e_re, e_im, v, params, steps, warm
     return ms, out_re, out_im, norm, geo, kt
 
 
+def tile_launch(lat, params, prec, steps, tile_rows) -> bool:
+    """Whether such an evolve call runs as register tiles (small lattices)."""
+    import ctypes as C
+    from tsmi import _lib
+    d = _lib.Desc(lat.dim_x, lat.dim_y, int(lat.periodic_x), int(lat.periodic_y), lat.halo_x, lat.halo_y, 0, prec,
+                  tile_rows, 0, params["dt"], params["mass"], params["g"], 0.0, lat.delta_x, lat.delta_y, lat.length_x,
+                  lat.length_y, 0.0)
+    out = (C.c_int32 * 4)()
+    _lib.check(_lib.load().tsmi_tile_geometry(C.byref(d), steps, out), "tsmi_tile_geometry")
+    return out[0] > 0
+
+
+def dominant_kernel(kt, steps: int, tiles: bool):
+    """Name, launches, ms per launch and steps per launch of the kernel that ran most of
+    `steps` steps, from tsmi_kernel_time's counts: the pass of several steps when the
+    run used one (the other launches took one step each), else the single-step pass."""
+    fused = kt["fused_launches"] > 0
+    launches = kt["fused_launches"] if fused else kt["single_launches"]
+    ms = (kt["fused_ms"] if fused else kt["single_ms"]) / max(1, launches)
+    per = (steps - kt["single_launches"]) / launches if fused else 1
+    return ("tile_kernel" if tiles else "step2_kernel" if fused else "step_kernel", launches, ms,
+            int(per) if per == int(per) else per)
+
+
 def host_cpu() -> dict:
     """This host's CPU: model, logical CPUs, the ones this process may use, and
     whether it has AVX-512 (x86-64-v4)."""
@@ -543,17 +567,14 @@ def main():
                                                        args.steps, args.warmup, args.tile_rows)
         per_step = ms / args.steps
         su = sites * args.steps / (ms * 1e-3)
-        # dominant kernel: the fused two-step pass when the run used it
-        fused = kt["fused_launches"] > 0
-        launches = kt["fused_launches"] if fused else kt["single_launches"]
-        kms = (kt["fused_ms"] if fused else kt["single_ms"]) / max(1, launches)
+        tiles = tile_launch(lat, params, prec, args.steps, args.tile_rows)
+        kernel, launches, kms, per_launch = dominant_kernel(kt, args.steps, tiles)
         results[prec] = dict(ms=ms, per_step=per_step, su=su, norm=norm, geo=geo, out=(o_re, o_im),
-                             kernel="step2_kernel" if fused else "step_kernel", kernel_us=kms * 1e3,
-                             launches=launches, sweeps=2 if fused else 1, kt=kt)
+                             kernel=kernel, kernel_us=kms * 1e3, launches=launches, sweeps=per_launch, kt=kt)
         rf = roofline_of(results[prec], prec, sites, args.n)
         results[prec]["roofline"] = rf
         log(f"FP{prec}: {per_step * 1e3:.1f} us/step, {su:.4g} SU/s; {rf['kernel']} {kms * 1e3:.1f} us/launch x "
-            f"{launches} ({rf['steps_per_launch']} steps each): {rf['achieved']:.0f} GB/s of the bytes a launch "
+            f"{launches} ({rf['steps_per_launch']:g} steps each): {rf['achieved']:.0f} GB/s of the bytes a launch "
             f"must move = {rf['frac']:.3f} of HBM peak; norm {norm:.15f}")
 
     accuracy = None

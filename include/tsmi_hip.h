@@ -267,15 +267,17 @@ int tsmi_pair_get_state_complex(tsmi_pair *pair, int32_t which, double *psi);
  * potentials; syncs. */
 int tsmi_pair_energy(tsmi_pair *pair, double out[12]);
 
-/* out[0..5] = W, H, pitch, strips, segments, rows per segment of the pair step. */
+/* out[0..5] = W, H, pitch, strips, segments, rows per segment of the streamed pair
+ * step (tsmi_pair_evolve runs small and medium lattices as register tiles instead). */
 int tsmi_pair_geometry(const tsmi_pair *pair, int32_t out[6]);
 int tsmi_pair_synchronize(tsmi_pair *pair);
 
 /* Kernel timing for measurement (no reference counterpart).  With timing on,
  * every step-kernel launch is bracketed by HIP events on the context stream;
  * tsmi_kernel_time syncs and reports out[0..3] = total ms and number of the
- * fused two-step launches, total ms and number of the single-step launches
- * since timing was (re)enabled. */
+ * launches of several steps (two streamed, two to eight as register tiles, see
+ * tsmi_tile_geometry), total ms and number of the single-step launches since timing
+ * was (re)enabled. */
 int tsmi_kernel_timing(tsmi_ctx *ctx, int32_t enable);
 int tsmi_kernel_time(tsmi_ctx *ctx, double out[4]);
 
@@ -328,8 +330,10 @@ int tsmi_get_state_device(tsmi_ctx *ctx, double *re, double *im);
  * synchronisation, src/gpukernel.cu:502-521). */
 int tsmi_synchronize(tsmi_ctx *ctx);
 
-/* Tile geometry chosen for the context: out[0..5] = W, H, pitch (elements),
- * strips, segments, rows per segment.  No reference counterpart (reporting). */
+/* Geometry of the context: out[0..5] = W, H, pitch (elements), and strips, segments,
+ * rows per segment of its streamed one-step pass (small and medium lattices run as
+ * register tiles instead, see tsmi_tile_geometry).  No reference counterpart
+ * (reporting). */
 int tsmi_geometry(const tsmi_ctx *ctx, int32_t out[6]);
 
 /* The geometry tsmi_create would choose for a descriptor, without creating a

@@ -59,7 +59,7 @@ __global__ void stage_out_kernel(const T *__restrict__ re, const T *__restrict__
     }
 }
 
-// Two pinned chunks of at most kChunk bytes each, allocated at the first use and
+// Two pinned chunks of at most kChunk bytes each (or one row, if that is more), allocated at the first use and
 // released with the owner.  A call returns when its copies are done, so the
 // chunks are free between calls, whatever stream the next one runs on.
 class HostStage {

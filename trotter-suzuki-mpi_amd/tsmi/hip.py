@@ -142,7 +142,8 @@ class HipKernel:
         _lib.check(self._L.tsmi_kernel_timing(self._h, int(bool(enable))), "tsmi_kernel_timing")
 
     def kernel_time(self) -> dict:
-        """Syncs; ms and launch counts of the fused and single-step kernels."""
+        """Syncs; ms and launch counts of the kernels of several steps ("fused": two streamed, up to
+        eight as register tiles) and of the single-step ones."""
         out = np.zeros(4)
         _lib.check(self._L.tsmi_kernel_time(self._h, _lib.dptr(out)), "tsmi_kernel_time")
         return {"fused_ms": out[0], "fused_launches": int(out[1]), "single_ms": out[2], "single_launches": int(out[3])}
